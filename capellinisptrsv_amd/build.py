@@ -75,7 +75,7 @@ def build_oracle(verbose: bool = True) -> None:
     oracle_dir = os.path.join(ROOT, "oracle")
     _run(["make", "-s", "-B", "-C", oracle_dir, "oracle"])
     ref = os.environ.get("CAPELLINI_REFERENCE", "/root/reference")
-    if os.path.isdir(ref) and shutil.which("g++"):
+    if os.path.isfile(os.path.join(ref, "CUDA", "ourWrtFst", "mmio.h")) and shutil.which("g++"):
         _run(["make", "-s", "-B", "-C", oracle_dir, "ref", f"REF={ref}"])
         if verbose:
             print("built oracle/_ref from the reference tree")
