@@ -27,7 +27,7 @@ CAP_ERR_NOT_CONVERGED = -12
 CAP_ERR_WATCHDOG = -13
 
 CAP_F64, CAP_F32 = 0, 1
-ALGO = {"auto": 0, "wrtfst": 1, "twopart": 2, "mix": 3, "csc": 4, "local": 5, "partition": 6, "level": 7}
+ALGO = {"auto": 0, "wrtfst": 1, "twopart": 2, "mix": 3, "csc": 4, "local": 5, "partition": 6, "level": 7, "hop": 8}
 ALGO_NAME = {v: k for k, v in ALGO.items()}
 SYNC = {"auto": 0, "value": 1, "flag": 2}
 ADJOINT = {"auto": 0, "scatter": 1, "gather": 2}
@@ -80,6 +80,7 @@ SIGNATURES = {
     "cap_plan_reset": (c_int, [c_void_p, c_void_p, c_int, c_void_p]),
     "cap_plan_launch": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     "cap_plan_info": (c_int, [c_void_p, PI, PI, PI, PI, PD, PD]),
+    "cap_plan_hops": (c_int, [c_void_p, PI]),
     "cap_plan_poll_count": (c_int, [c_void_p, POINTER(c_ulonglong), c_void_p]),
     "cap_plan_rhs_block": (c_int, [c_void_p, c_int, PI, PI, PI, PI, PI, PI]),
     "cap_plan_tuning": (c_int, [c_void_p, PI, PI, PI, PI, PI, PI]),

@@ -645,6 +645,217 @@ __global__ void __launch_bounds__(BLOCK)
     }
 }
 
+// ------------------------------------------------ look-through solve
+// Solve of matrices whose rows hold at most kHopMax off-diagonals, with half
+// the dependency hops.  A row that would wait for a value of the newest wave
+// of results does not wait for it: it waits for the values THAT row needs
+// and computes it again itself (the same operations on the same operands, so
+// the same bits).  Each cross-CU hop then covers two levels.
+//   hop(i) = 1 + max over i's entries c of min(hop(c), look(c)),
+//   look(c) = max of hop over c's own entries;
+// entry c of row i is looked through where hop(c) exceeds hop(i) - 1.
+//
+// Why: with readiness polled in device memory, a solve of wide levels costs
+// one publish -> observe hop per level, and the hop's length is set by the
+// polls themselves: each lane's poll is a 64-byte fabric request, 64 of them
+// per wavefront, and 65,536 polling rows fill the fabric for about 1.3 us a
+// round (with polls that share lines the same rows poll in a quarter of
+// that).  So this kernel
+//  * halves the hops (155 -> 78 on the wide-level 2M matrix) at 1.2 x the polls;
+//  * hands out rows in hop order and indexes the readiness array by position
+//    in that order, not by row: a wavefront publishes 64 adjacent values, and
+//    where neighbouring rows depend on neighbouring rows (grids) their polls
+//    share lines;
+//  * reads a row's whole description with one coalesced round of loads
+//    (tables laid out at plan creation; the values themselves stay in the
+//    caller's array, which may change between solves), so a workgroup is
+//    ready to poll two memory round trips after its ticket instead of five.
+// Measured (kernel alone, FP64): wide-level 2M 213 -> 148 us; a 100 x 90 x 80
+// grid's 7-point lower factor (268 levels) 2,050 -> 220 us.  In the same
+// tests: hop order without looking through 196 / 311 us; looking through
+// without the reordered readiness array 173 / 275 us; looking through two
+// rows deep (52 hops) 235 us on the wide-level matrix (its longer load
+// chains outweigh the saved hops).
+//
+// Table of slot s (position in hop order; field f at base[f * npad + s]):
+// the row, its first entry, the counts word, then per entry the slot to poll
+// (or, looked through, the row).  Counts word: bits 0-2 the row's entries,
+// bit 3 + j entry j is looked through, bits 8 + 3j the polls of entry j
+// (1, or the looked-through row's entries).  ex holds, per wavefront of
+// slots, for each entry the looked-through row's first entry and its entries'
+// slots, 64 of each.
+constexpr int kHopMax = 4;
+struct HopTab {
+    const int *base, *ex;
+    int npad;
+};
+
+// The tables of E entries per row, from the hop order (order[s] = row of slot
+// s), its inverse and each row's look-through bits.  One thread per slot;
+// slots past n describe row 0 with no entries (their lanes stay idle).
+template <int E>
+__global__ void __launch_bounds__(kBlock)
+    k_hop_tables(const int *__restrict__ rp, const int *__restrict__ ci, const int *__restrict__ order,
+                 const int *__restrict__ slot, const unsigned char *__restrict__ look, int n, int npad,
+                 int *__restrict__ base, int *__restrict__ ex)
+{
+    const int s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= npad) return;
+    const bool in = s < n;
+    const int row = in ? order[s] : 0;
+    const int e0 = rp[row], cnt = in ? rp[row + 1] - 1 - e0 : 0;
+    const unsigned m = in ? look[row] : 0;
+    int cw = cnt;
+    int *x = ex + (size_t)(s >> 6) * (kWave * E * (E + 1)) + (s & (kWave - 1));
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        int c = 0, first = 0, nn = 0, to[E] = {};
+        if (j < cnt) {
+            c = ci[e0 + j];
+            nn = 1;
+            if ((m >> j) & 1) {
+                cw |= 1 << (3 + j);
+                first = rp[c];
+                nn = rp[c + 1] - 1 - first;
+#pragma unroll
+                for (int t = 0; t < E; ++t)
+                    if (t < nn) to[t] = slot[ci[first + t]];
+            } else {
+                c = slot[c];
+            }
+        }
+        cw |= nn << (8 + 3 * j);
+        base[(size_t)(3 + j) * npad + s] = c;
+        x[(j * (E + 1)) * kWave] = first;
+#pragma unroll
+        for (int t = 0; t < E; ++t) x[(j * (E + 1) + 1 + t) * kWave] = to[t];
+    }
+    base[s] = row;
+    base[(size_t)npad + s] = e0;
+    base[(size_t)2 * npad + s] = cw;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_invert(const int *__restrict__ order, int n, int *__restrict__ slot)
+{
+    const int s = blockIdx.x * kBlock + threadIdx.x;
+    if (s < n) slot[order[s]] = s;
+}
+
+// Workgroup barrier that orders LDS only: the plain __syncthreads would also
+// wait for the acknowledgement of the published values.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One lane per row, tickets of BLOCK slots; wavefront 0 takes the next ticket
+// when its own rows are done, while the others may still poll.  n_rev > 0: row r is
+// stored at n_rev - 1 - r of b and x (upper-triangular plans).
+template <typename T, int E, int BLOCK>
+__global__ void __launch_bounds__(BLOCK)
+    k_hop(HopTab tab, const T *__restrict__ val, const T *__restrict__ b, T *__restrict__ x, SyncCtx sc, int n,
+          unsigned *__restrict__ ticket, int n_rev)
+{
+    typedef typename VBits<T>::U U;
+    constexpr U kS = VBits<T>::kSentinel;
+    U *xr = reinterpret_cast<U *>(sc.ready);
+    __shared__ int s_base[2];
+    if (threadIdx.x == 0) s_base[0] = (int)atomicAdd(ticket, (unsigned)BLOCK);
+    for (int turn = 0;; turn ^= 1) {
+        lds_barrier();
+        const int first = s_base[turn];
+        if (first >= n) return;
+        const int s = first + (int)threadIdx.x;
+        const bool in = s < n;
+        // one coalesced round: the row's description (slot 0's past the end)
+        const int sl = in ? s : 0;
+        const int row = tab.base[sl], e0 = tab.base[(size_t)tab.npad + sl];
+        const int cw = in ? tab.base[(size_t)2 * tab.npad + sl] : 0;
+        int c[E], f[E], to[E][E];
+        const int *ex = tab.ex + (size_t)(sl >> 6) * (kWave * E * (E + 1)) + (sl & (kWave - 1));
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            c[j] = tab.base[(size_t)(3 + j) * tab.npad + sl];
+            f[j] = ex[(j * (E + 1)) * kWave];
+#pragma unroll
+            for (int t = 0; t < E; ++t) to[j][t] = ex[(j * (E + 1) + 1 + t) * kWave];
+        }
+        const int cnt = cw & 7;
+        U r[E][E];
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const bool lk = (cw >> (3 + j)) & 1;
+            const int nn = (cw >> (8 + 3 * j)) & 7;
+            if (!lk) to[j][0] = c[j];
+#pragma unroll
+            for (int t = 0; t < E; ++t) r[j][t] = t < nn ? kS : (U)0;
+        }
+        // second round: every value of the row and of the rows it looks
+        // through.  Unused ones read an entry that exists (no branch, so the
+        // loads are issued together) and are left out of the sums below.
+        const int o = n_rev ? n_rev - 1 - row : row;
+        const T bo = b[o], vd = val[e0 + cnt];
+        T v[E], vv[E][E], bb[E], dd[E];
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const bool lk = (cw >> (3 + j)) & 1;
+            const int nn = lk ? (cw >> (8 + 3 * j)) & 7 : 0, g = lk ? c[j] : 0, fj = lk ? f[j] : 0;
+            v[j] = val[e0 + min(j, cnt)];
+            bb[j] = b[n_rev ? n_rev - 1 - g : g];
+            dd[j] = val[fj + nn];
+#pragma unroll
+            for (int t = 0; t < E; ++t) vv[j][t] = val[fj + min(t, nn)];
+        }
+        Idle idle;
+        bool done = !in;
+        do {  // wave-uniform exit: see wrtfst_row
+            if (!done) {
+                bool all = true;
+#pragma unroll
+                for (int j = 0; j < E; ++j)
+#pragma unroll
+                    for (int t = 0; t < E; ++t)
+                        if (r[j][t] == kS) r[j][t] = ld_agent(xr + to[j][t]);
+#pragma unroll
+                for (int j = 0; j < E; ++j)
+#pragma unroll
+                    for (int t = 0; t < E; ++t) all = all && r[j][t] != kS;
+                const bool failed = !all && give_up(sc, idle);
+                if (all || failed) {
+                    T sum = (T)0;
+#pragma unroll
+                    for (int j = 0; j < E; ++j) {
+                        T xj = as_val(r[j][0]);
+                        if ((cw >> (3 + j)) & 1) {
+                            const int nn = (cw >> (8 + 3 * j)) & 7;
+                            T q = (T)0;
+#pragma unroll
+                            for (int t = 0; t < E; ++t)
+                                if (t < nn) q = acc(sc, vv[j][t], as_val(r[j][t]), q);
+                            xj = (bb[j] - q) / dd[j];
+                        }
+                        if (j < cnt) sum = acc(sc, v[j], xj, sum);
+                    }
+                    if (failed) sum = as_val(VBits<T>::kQNaN);  // poison this row; it still publishes
+                    const T xi = (bo - sum) / vd;
+                    U u = as_bits(xi);
+                    if (u == kS) u = VBits<T>::kQNaN;
+                    st_agent(xr + s, u);
+                    x[o] = xi;
+                    asm volatile("" ::: "memory");
+                    done = true;
+                }
+            }
+        } while (__any(!done));
+        // read by the others after the next barrier; the slot they read for
+        // this turn is not written again before the one after it
+        if (threadIdx.x == 0) s_base[turn ^ 1] = (int)atomicAdd(ticket, (unsigned)BLOCK);
+    }
+}
+
 // Value protocol row solver for R right-hand sides per lane: the lane owns
 // right-hand sides q, q + L, ..., q + (R-1)L of row i (those below k), L
 // lanes per row, so each poll instruction of the row's L lanes reads L

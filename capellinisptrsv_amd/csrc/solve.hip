@@ -110,6 +110,13 @@ struct LevelState {
     int max_rhs = 1;         // right-hand sides per solve: 1, or 2 / 4 where their ring fits LDS (E = 4)
 };
 
+// Look-through tables of the write-first solve (layout in kernels.h, k_hop):
+// E entries per row, `hops` publish -> observe hops on the longest chain.
+struct HopState {
+    int *base = nullptr, *ex = nullptr;
+    int E = 0, npad = 0, hops = 0;
+};
+
 // The RHS-block pick of an autotuned plan for one right-hand-side count:
 // thread-per-row workgroups per CU, threads per workgroup and right-hand
 // sides per lane, or the partitioned block solve's right-hand sides per
@@ -203,7 +210,17 @@ struct cap_plan_s {
     struct PartState *part = nullptr;
     // level steps in one workgroup (CAP_ALGO_LEVEL)
     LevelState *lvl = nullptr;
+    // write-first solve of one right-hand side with look-through tables
+    // (autotuned plans, value protocol, staged readiness)
+    HopState *hop = nullptr;
 };
+
+// One right-hand side of a plan whose pick has look-through tables.  The
+// kernel reverses rows itself, so upper-triangular plans need no copies.
+inline bool hop_takes(const cap_plan_s *p, int rhs)
+{
+    return p->hop && rhs == 1 && p->algo == CAP_ALGO_WRTFST && p->sync == CAP_SYNC_VALUE && p->staged;
+}
 
 // Right-hand-side counts a level plan solves: 1, and 2 or 4 where a ring of
 // that many values per slot fits LDS (rows of at most 4 off-diagonals).
@@ -408,11 +425,22 @@ void free_level(cap_plan p)
     p->lvl = nullptr;
 }
 
+void free_hop(cap_plan p)
+{
+    if (!p->hop) return;
+    (void)hipDeviceSynchronize();
+    for (int *b : {p->hop->base, p->hop->ex})
+        if (b) (void)hipFree(b);
+    delete p->hop;
+    p->hop = nullptr;
+}
+
 void plan_free(cap_plan p)
 {
     if (!p) return;
     free_partition(p);
     free_level(p);
+    free_hop(p);
     if (p->ready) {
         (void)hipDeviceSynchronize();  // no kernel of this plan may still poll the block
         ready_release(p->ready);
@@ -808,7 +836,21 @@ int launch_kernel(cap_plan p, int algo, int sync, const T *val, const T *b, T *x
     if (algo != CAP_ALGO_CSC && algo != CAP_ALGO_LOCAL && algo != CAP_ALGO_LEVEL)
         CAP_TRY(sync_ctx<T>(p, sync, (long long)n * rhs, &sc));
     if (fused) sc.unfused = 0;
-    if (algo == CAP_ALGO_WRTFST && p->rpl > 1 && rhs > 1) {  // several right-hand sides per lane
+    if (algo == CAP_ALGO_WRTFST && sync == CAP_SYNC_VALUE && hop_takes(p, rhs)) {
+        const HopState *h = p->hop;
+        const HopTab tab{h->base, h->ex, h->npad};
+        const unsigned nb = grid_for(p, ((long long)n + p->wblock - 1) / p->wblock);
+        auto go = [&](auto kernel) {
+            kernel<<<nb, p->wblock, 0, st>>>(tab, val, b, x, sc, n, p->ticket, p->reversed ? n : 0);
+        };
+        const bool small = p->wblock == kBlockSmall;
+        if (h->E == 2)
+            small ? go(k_hop<T, 2, kBlockSmall>) : go(k_hop<T, 2, kBlock>);
+        else if (h->E == 3)
+            small ? go(k_hop<T, 3, kBlockSmall>) : go(k_hop<T, 3, kBlock>);
+        else
+            small ? go(k_hop<T, 4, kBlockSmall>) : go(k_hop<T, 4, kBlock>);
+    } else if (algo == CAP_ALGO_WRTFST && p->rpl > 1 && rhs > 1) {  // several right-hand sides per lane
         if (rhs > kWave || sync != CAP_SYNC_VALUE || p->lds || p->count_polls) return CAP_ERR_UNSUPPORTED;
         const int l = lpr_log2_for((rhs + p->rpl - 1) / p->rpl);
         const int rows_per_block = p->wblock >> l;
@@ -1047,17 +1089,17 @@ int ensure_csc(cap_plan p, hipStream_t st)
 // column indices.  Two matrices with one row-length profile but different
 // dependencies (a chain and a wide-level matrix) never share a pick.
 struct TuneKey {
-    int n, nnz, vt, staged, unfused, levels;
+    int n, nnz, vt, staged, unfused, count_polls, levels;
     unsigned long long fp;
     bool operator<(const TuneKey &o) const
     {
-        return std::tie(n, nnz, vt, staged, unfused, levels, fp) <
-               std::tie(o.n, o.nnz, o.vt, o.staged, o.unfused, o.levels, o.fp);
+        return std::tie(n, nnz, vt, staged, unfused, count_polls, levels, fp) <
+               std::tie(o.n, o.nnz, o.vt, o.staged, o.unfused, o.count_polls, o.levels, o.fp);
     }
 };
 std::mutex g_tune_mu;
 struct TuneChoice {
-    int algo, sync, border, bpc, lds, staged, block, tile = 0;
+    int algo, sync, border, bpc, lds, staged, block, tile = 0, hop = 0;
 };
 std::map<TuneKey, TuneChoice> g_tune_cache;
 
@@ -1629,6 +1671,78 @@ int build_level(cap_plan p, const std::vector<int> &rp_host)
     return p->vt == CAP_F64 ? build_level_t<double>(p, rp_host) : build_level_t<float>(p, rp_host);
 }
 
+// Look-through tables of the write-first solve (k_hop): each row's hop
+// number and look-through bits on the host, one pass over the entries; the
+// tables on the device.  CAP_ERR_UNSUPPORTED for rows of more than kHopMax
+// off-diagonals: the kernel keeps E values of each of E entries in registers.
+int build_hop(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, hipStream_t st)
+{
+    const int n = p->n;
+    int most = 0;
+    for (int i = 0; i < n; ++i) most = std::max(most, rp[i + 1] - 1 - rp[i]);
+    if (n < 1 || most > kHopMax) return CAP_ERR_UNSUPPORTED;
+    const int E = std::max(2, most);
+    std::vector<int> hop, look, order;  // look: the hop a looked-through row is ready in
+    std::vector<unsigned char> bits;
+    int hops = 0;
+    try {
+        hop.resize((size_t)n);
+        look.resize((size_t)n);
+        order.resize((size_t)n);
+        bits.resize((size_t)n);
+        for (int i = 0; i < n; ++i) {
+            const int lo = rp[i], hi = rp[i + 1] - 1;
+            int ready = 0, newest = 0;
+            for (int j = lo; j < hi; ++j) {
+                newest = std::max(newest, hop[(size_t)ci[j]]);
+                ready = std::max(ready, std::min(hop[(size_t)ci[j]], look[(size_t)ci[j]]));
+            }
+            unsigned m = 0;
+            for (int j = lo; j < hi; ++j) m |= (unsigned)(hop[(size_t)ci[j]] > ready) << (j - lo);
+            hop[(size_t)i] = ready + 1;
+            look[(size_t)i] = newest;
+            bits[(size_t)i] = (unsigned char)m;
+            hops = std::max(hops, ready + 1);
+        }
+        // rows in hop order, by index within a hop
+        std::vector<int> at((size_t)hops + 2, 0);
+        for (int i = 0; i < n; ++i) ++at[(size_t)hop[(size_t)i] + 1];
+        for (int h = 0; h <= hops; ++h) at[(size_t)h + 1] += at[(size_t)h];
+        for (int i = 0; i < n; ++i) order[(size_t)at[(size_t)hop[(size_t)i]]++] = i;
+    } catch (const std::bad_alloc &) {
+        return CAP_ERR_ALLOC;
+    }
+    free_hop(p);
+    HopState *hs = new HopState();
+    p->hop = hs;
+    hs->E = E;
+    hs->hops = hops;
+    hs->npad = (n + kWave - 1) / kWave * kWave;
+    int *d_order = nullptr, *d_slot = nullptr;
+    unsigned char *d_bits = nullptr;
+    int rc = dev_alloc(&hs->base, (size_t)hs->npad * (3 + E));
+    if (rc == CAP_OK) rc = dev_alloc(&hs->ex, (size_t)hs->npad * E * (E + 1));
+    if (rc == CAP_OK) rc = dev_alloc(&d_order, (size_t)n);
+    if (rc == CAP_OK) rc = dev_alloc(&d_slot, (size_t)n);
+    if (rc == CAP_OK) rc = dev_alloc(&d_bits, (size_t)n);
+    if (rc == CAP_OK && (hipMemcpy(d_order, order.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
+                         hipMemcpy(d_bits, bits.data(), (size_t)n, hipMemcpyHostToDevice) != hipSuccess))
+        rc = CAP_ERR_HIP;
+    if (rc == CAP_OK) {
+        k_invert<<<blocks_for(n), kBlock, 0, st>>>(d_order, n, d_slot);
+        auto fill = [&](auto kernel) {
+            kernel<<<blocks_for(hs->npad), kBlock, 0, st>>>(p->rp, p->ci, d_order, d_slot, d_bits, n, hs->npad, hs->base,
+                                                            hs->ex);
+        };
+        E == 2 ? fill(k_hop_tables<2>) : E == 3 ? fill(k_hop_tables<3>) : fill(k_hop_tables<4>);
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) rc = CAP_ERR_HIP;
+    }
+    for (void *b : {(void *)d_order, (void *)d_slot, (void *)d_bits})
+        if (b) (void)hipFree(b);
+    if (rc != CAP_OK) free_hop(p);
+    return rc;
+}
+
 // Candidates are timed on the plan's own matrix (b = 0; the dependency
 // structure, not the values, sets the time) and the fastest is cached per
 // matrix shape: thread-per-row with and without the LDS window, at 1 or 2
@@ -1636,12 +1750,10 @@ int build_level(cap_plan p, const std::vector<int> &rp_host)
 // flag protocol, and mix at three thresholds when the rows are long enough
 // for wavefront mode to matter.  A plan created with readiness in place keeps
 // it in every candidate.
-int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
+int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int> &ci, hipStream_t st)
 {
-    std::vector<int> ci((size_t)p->nnz);
-    CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * ci.size(), hipMemcpyDeviceToHost));
     const int levels = p->n ? cap_matrix_layer(p->n, rp_host.data(), ci.data(), nullptr, nullptr, nullptr) : 1;
-    const TuneKey key{p->n, p->nnz, p->vt, p->staged, p->unfused, levels, fingerprint(rp_host, ci)};
+    const TuneKey key{p->n, p->nnz, p->vt, p->staged, p->unfused, p->count_polls, levels, fingerprint(rp_host, ci)};
     {
         std::lock_guard<std::mutex> g(g_tune_mu);
         auto it = g_tune_cache.find(key);
@@ -1650,6 +1762,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
             if (p->algo == CAP_ALGO_MIX) return build_mix(p, rp_host, it->second.border);
             if (p->algo == CAP_ALGO_LOCAL) return ensure_segments(p, nullptr);
             if (p->algo == CAP_ALGO_LEVEL) return build_level(p, rp_host);
+            if (it->second.hop) return build_hop(p, rp_host, ci, st);
             if (p->algo != CAP_ALGO_PARTITION) return CAP_OK;
             // the pick was cached for this structure; these values may not
             // keep the partition stable, and then the plan is tuned afresh
@@ -1671,6 +1784,11 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
                                      {CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, 1, stg, S},
                                      {CAP_ALGO_WRTFST, CAP_SYNC_FLAG, 0, 1, 0, 0, B}};
     if (stg) cands.push_back({CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
+    // look-through tables, where rows are short: half the hops
+    if (stg && !p->count_polls && build_hop(p, rp_host, ci, st) == CAP_OK)
+        for (int blk : {B, S})
+            cands.insert(cands.begin(), {CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, 0, stg, blk, 0, 1});
+    HopState *const hop_tables = p->hop;
     // the same value-protocol shapes with each ticket's col_idx/val tile staged in LDS
     for (int lds : {0, 1})
         for (int blk : {B, S}) cands.push_back({CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, lds, stg, blk, 1});
@@ -1707,6 +1825,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
     int rc = CAP_OK;
     for (const TuneChoice &c : cands) {
         apply_choice(p, c);
+        p->hop = c.hop ? hop_tables : nullptr;
         if (c.algo == CAP_ALGO_MIX && (rc = build_mix(p, rp_host, c.border)) != CAP_OK) break;
         if (c.algo == CAP_ALGO_LOCAL && (rc = ensure_segments(p, nullptr)) != CAP_OK) break;
         float t = 0;
@@ -1721,8 +1840,10 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
     }
     (void)hipFree(b);
     (void)hipFree(x);
+    p->hop = hop_tables;
     if (rc != CAP_OK) return rc;
     apply_choice(p, pick);
+    if (!pick.hop) free_hop(p);
     if (pick.algo == CAP_ALGO_MIX) CAP_TRY(build_mix(p, rp_host, pick.border));
     if (pick.algo == CAP_ALGO_LOCAL) CAP_TRY(ensure_segments(p, nullptr));
     if (pick.algo != CAP_ALGO_PARTITION) free_partition(p);
@@ -1733,10 +1854,11 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
 }
 
 template <typename T>
-int validate_device_matrix(cap_plan p, std::vector<int> *rp_host)
+int validate_device_matrix(cap_plan p, std::vector<int> *rp_host, std::vector<int> *ci_host)
 {
     const int n = p->n, nnz = p->nnz;
-    std::vector<int> ci((size_t)nnz);
+    std::vector<int> &ci = *ci_host;  // kept for the autotuner's analysis
+    ci.resize((size_t)nnz);
     std::vector<T> v((size_t)nnz);
     CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost));
     CAP_HIP_TRY(hipMemcpy(v.data(), p->val, sizeof(T) * (size_t)nnz, hipMemcpyDeviceToHost));
@@ -1744,6 +1866,15 @@ int validate_device_matrix(cap_plan p, std::vector<int> *rp_host)
     if (sizeof(T) == 8)
         return cap_validate_csr_d(n, nnz, rp_host->data(), ci.data(), (const double *)(const void *)v.data(), &bad);
     return cap_validate_csr_s(n, nnz, rp_host->data(), ci.data(), (const float *)(const void *)v.data(), &bad);
+}
+
+// A host copy of the column indices, unless the layout check already took one.
+int host_columns(cap_plan p, std::vector<int> *ci)
+{
+    if (ci->size() == (size_t)p->nnz) return CAP_OK;
+    ci->resize((size_t)p->nnz);
+    CAP_HIP_TRY(hipMemcpy(ci->data(), p->ci, sizeof(int) * (size_t)p->nnz, hipMemcpyDeviceToHost));
+    return CAP_OK;
 }
 
 // Upper-triangular and implicit-unit-diagonal matrices become the lower,
@@ -1805,6 +1936,9 @@ int plan_create_impl(cap_plan *out, int n, int nnz, const int *rp, const int *ci
         o.rhs_per_lane != 8)
         return CAP_ERR_ARG;
     if (o.row_tiles != 0 && o.row_tiles != 1) return CAP_ERR_ARG;
+    if (o.algo == CAP_ALGO_HOP && ((o.sync != CAP_SYNC_AUTO && o.sync != CAP_SYNC_VALUE) ||
+                                   o.readiness == CAP_READY_IN_PLACE || o.lds_window > 0 || o.count_polls))
+        return CAP_ERR_UNSUPPORTED;
     if (o.row_tiles &&
         ((o.algo != CAP_ALGO_WRTFST && o.algo != CAP_ALGO_MIX) || (o.sync != CAP_SYNC_AUTO && o.sync != CAP_SYNC_VALUE) ||
          o.count_polls || o.rhs_per_lane > 1))
@@ -1860,7 +1994,7 @@ int plan_create_impl(cap_plan *out, int n, int nnz, const int *rp, const int *ci
     p->vbytes = vt == CAP_F64 ? 8 : 4;
     p->device = dev;
     int rc = CAP_OK;
-    std::vector<int> rp_host((size_t)n + 1);
+    std::vector<int> rp_host((size_t)n + 1), ci_host;  // ci_host: filled where it is needed, once
     do {
         if (o.host_inputs) {
             if (o.validate) {
@@ -1889,8 +2023,8 @@ int plan_create_impl(cap_plan *out, int n, int nnz, const int *rp, const int *ci
                 break;
             }
             if (o.validate) {
-                rc = vt == CAP_F64 ? validate_device_matrix<double>(p, &rp_host)
-                                   : validate_device_matrix<float>(p, &rp_host);
+                rc = vt == CAP_F64 ? validate_device_matrix<double>(p, &rp_host, &ci_host)
+                                   : validate_device_matrix<float>(p, &rp_host, &ci_host);
                 if (rc != CAP_OK) break;
             }
         }
@@ -1915,25 +2049,27 @@ int plan_create_impl(cap_plan *out, int n, int nnz, const int *rp, const int *ci
         if (p->algo == CAP_ALGO_MIX) {
             int border = o.border;
             if (border <= 0) {  // from the matrix's rows per level
-                std::vector<int> ci_host((size_t)p->nnz);
-                if (p->nnz > 0 && hipMemcpy(ci_host.data(), p->ci, sizeof(int) * (size_t)p->nnz,
-                                            hipMemcpyDeviceToHost) != hipSuccess)
-                    rc = CAP_ERR_HIP;
+                rc = host_columns(p, &ci_host);
                 const int levels =
-                    p->n ? cap_matrix_layer(p->n, rp_host.data(), ci_host.data(), nullptr, nullptr, nullptr) : 1;
+                    rc == CAP_OK && p->n
+                        ? cap_matrix_layer(p->n, rp_host.data(), ci_host.data(), nullptr, nullptr, nullptr)
+                        : 1;
                 border = mix_border_for(p->n, levels);
             }
             if (rc == CAP_OK) rc = build_mix(p, rp_host, border);
         } else if (p->algo == CAP_ALGO_CSC) {
             rc = ensure_csc(p, st);
         } else if (p->algo == CAP_ALGO_AUTO) {
-            rc = autotune(p, rp_host, st);
+            if ((rc = host_columns(p, &ci_host)) == CAP_OK) rc = autotune(p, rp_host, ci_host, st);
         } else if (p->algo == CAP_ALGO_LOCAL) {
             rc = ensure_segments(p, nullptr);
         } else if (p->algo == CAP_ALGO_PARTITION) {
             rc = build_partition(p, rp_host, st);
         } else if (p->algo == CAP_ALGO_LEVEL) {
             rc = build_level(p, rp_host);
+        } else if (p->algo == CAP_ALGO_HOP) {
+            p->algo = CAP_ALGO_WRTFST;
+            if ((rc = host_columns(p, &ci_host)) == CAP_OK) rc = build_hop(p, rp_host, ci_host, st);
         } else if (p->algo != CAP_ALGO_WRTFST && p->algo != CAP_ALGO_TWOPART) {
             rc = CAP_ERR_ARG;
         }
@@ -2059,7 +2195,7 @@ int cap_plan_solve(cap_plan p, const void *b, void *x, int rhs, void *stream)
     if (p->tune_rhs && rhs > 1 && rhs <= kWave && !p->reversed && !p->rhs_pick.count(rhs))
         CAP_TRY(tune_rhs_block(p, b, x, rhs, S(stream)));
     const int algo = algo_for(p, rhs), sync = sync_for(p, rhs);
-    if (!p->reversed) return plan_solve_with(p, algo, sync, b, x, rhs, S(stream));
+    if (!p->reversed || hop_takes(p, rhs)) return plan_solve_with(p, algo, sync, b, x, rhs, S(stream));
     CAP_TRY(ensure_reversal(p, rhs));
     CAP_TRY(reverse_rows(p, b, p->rev_b, rhs, S(stream)));
     CAP_TRY(plan_solve_with(p, algo, sync, p->rev_b, p->rev_x, rhs, S(stream)));
@@ -2069,7 +2205,7 @@ int cap_plan_solve(cap_plan p, const void *b, void *x, int rhs, void *stream)
 int cap_plan_reset(cap_plan p, void *x, int rhs, void *stream)
 {
     if (!p || !x || rhs < 1) return CAP_ERR_ARG;
-    if (p->reversed) {
+    if (p->reversed && !hop_takes(p, rhs)) {
         CAP_TRY(ensure_reversal(p, rhs));
         x = p->rev_x;
     }
@@ -2081,7 +2217,7 @@ int cap_plan_reset(cap_plan p, void *x, int rhs, void *stream)
 int cap_plan_launch(cap_plan p, const void *b, void *x, int rhs, void *stream)
 {
     if (!p || !b || !x || rhs < 1) return CAP_ERR_ARG;
-    if (!p->reversed) return launch_plain(p, b, x, rhs, S(stream));
+    if (!p->reversed || hop_takes(p, rhs)) return launch_plain(p, b, x, rhs, S(stream));
     if (p->rev_bytes < (size_t)p->n * rhs * p->vbytes) return CAP_ERR_ARG;  // launch without its reset
     CAP_TRY(reverse_rows(p, b, p->rev_b, rhs, S(stream)));
     CAP_TRY(launch_plain(p, p->rev_b, p->rev_x, rhs, S(stream)));
@@ -2110,6 +2246,14 @@ int cap_plan_status(cap_plan p, void *stream)
     CAP_HIP_TRY(hipMemcpy(&e, p->err, sizeof(int), hipMemcpyDeviceToHost));
     if (e) CAP_HIP_TRY(hipMemset(p->err, 0, sizeof(int)));
     return e ? CAP_ERR_WATCHDOG : CAP_OK;
+}
+
+int cap_plan_hops(cap_plan p, int *hops)
+{
+    if (!p || !hops) return CAP_ERR_ARG;
+    if (!hop_takes(p, 1)) return CAP_ERR_UNSUPPORTED;
+    *hops = p->hop->hops;
+    return CAP_OK;
 }
 
 int cap_plan_poll_count(cap_plan p, unsigned long long *polls, void *stream)

@@ -38,7 +38,7 @@ class Plan:
 
     row_ptr/col_idx: int32 CUDA tensors; values: float64/float32 CUDA tensor.
     The plan keeps references to the three tensors (their memory is used in
-    place).  algo: auto|wrtfst|twopart|mix|csc|local|partition|level; sync:
+    place).  algo: auto|wrtfst|twopart|mix|csc|local|partition|level|hop; sync:
     auto|value|flag.
     row_threads: 128 or 256 threads per workgroup of the thread-per-row
     kernels (0: tuned with algo auto, else 256).
@@ -106,6 +106,16 @@ class Plan:
         v = c_ulonglong()
         N.check(N.lib().cap_plan_poll_count(self._h, byref(v), _stream(stream)), "cap_plan_poll_count")
         return v.value
+
+    def hops(self) -> int:
+        """Waits on the longest dependency chain of a plan that solves with
+        look-through tables (algo hop, or auto's pick of them); 0 for others."""
+        h = c_int()
+        rc = N.lib().cap_plan_hops(self._h, byref(h))
+        if rc == N.CAP_ERR_UNSUPPORTED:
+            return 0
+        N.check(rc, "cap_plan_hops")
+        return h.value
 
     def rhs_block(self, k: int):
         """The RHS block the autotuner picked for k right-hand sides (after a

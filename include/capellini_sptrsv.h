@@ -86,6 +86,22 @@ extern "C" {
                               with the few-rows-per-level candidates; its
                               refined solves use the write-first kernels. */
 
+#define CAP_ALGO_HOP 8       /* the thread-per-row write-first solve with
+                              look-through tables: a row whose dependency is
+                              too new computes that row again itself from the
+                              values it needs, so the chain takes about half
+                              the waits (cap_plan_hops).  Needs rows of at most
+                              4 off-diagonals, the value protocol and staged
+                              readiness, no LDS window, row tiles or poll
+                              counting (CAP_ERR_UNSUPPORTED otherwise).  One
+                              right-hand side; several go through
+                              CAP_ALGO_WRTFST, which is what cap_plan_info
+                              reports.  Bit-exact (each row is computed by the
+                              thread-per-row operations, however often).  The
+                              tables hold the pattern only: the caller's
+                              values are read on every solve.  Timed by algo
+                              AUTO. */
+
 /* adjoint method (cap_opts.adjoint) */
 #define CAP_ADJOINT_AUTO 0
 #define CAP_ADJOINT_SCATTER 1 /* column-driven on the CSR of L: in-degree counters
@@ -237,6 +253,11 @@ int cap_plan_rhs_block(cap_plan plan, int k, int *blocks_per_cu,
  * those algorithms refuses k > 1 with CAP_ERR_UNSUPPORTED.) */
 int cap_plan_info(cap_plan plan, int *algo, int *sync, int *border,
                   int *mix_len, double *warp_occupy, double *element_occupy);
+/* No counterpart in the reference: publish -> observe waits on the longest
+ * dependency chain of a plan that solves with look-through tables
+ * (CAP_ALGO_HOP, or algo AUTO's pick of them): about half its levels.
+ * CAP_ERR_UNSUPPORTED for plans without them. */
+int cap_plan_hops(cap_plan plan, int *hops);
 /* Grid, window, readiness and row-tile choices the plan uses (after
  * autotuning); *readiness is CAP_READY_STAGED or CAP_READY_IN_PLACE;
  * *row_threads of a CAP_ALGO_LEVEL plan is its one workgroup's size. */

@@ -1,0 +1,143 @@
+"""GPU parity of the look-through solve (CAP_ALGO_HOP, k_hop).
+
+Every row, also one computed a second time by a row that looks through it,
+is the stored-order chain of the thread-per-row kernels, so x must equal the
+oracle's bits and the plain write-first plan's, in both arithmetics and both
+precisions.  The number of waits is restated here from the rows.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from capellinisptrsv_amd import api, _native
+from conftest import drop_diagonal, random_lower, upper_from_lower
+
+pytestmark = pytest.mark.gpu
+
+
+def hops_of(rp, ci):
+    """hop(i) = 1 + max over entries c of min(hop(c), max of hop over c's entries)."""
+    n = len(rp) - 1
+    hop, look = [0] * n, [0] * n
+    for i in range(n):
+        cs = ci[rp[i]:rp[i + 1] - 1]
+        hop[i] = 1 + max((min(hop[c], look[c]) for c in cs), default=0)
+        look[i] = max((hop[c] for c in cs), default=0)
+    return max(hop)
+
+
+def _mats():
+    # edges of the wavefront and of both workgroup sizes' tickets; 2, 3 and 4
+    # entries per row; duplicates, unsorted rows
+    for n in (1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 1000):
+        yield f"n{n}", random_lower(n, max_off=2 + n % 3, band=40, seed=n, dup=False)
+    yield "dup", random_lower(3000, max_off=3, band=500, seed=2, dup=True)
+    yield "shuffled", random_lower(3000, max_off=4, band=90, seed=3, shuffle=True)
+    yield "diagonal", random_lower(300, max_off=0, seed=4)
+    yield "chain", api.generate("band", n=700, offdiag=1, band=1, seed=5)
+    yield "wide", api.make_config(1, seed=6, scale=0.05)
+    yield "level_o4", api.generate("level", n=30000, levels=30, width=1000, depth=3, offdiag=4, seed=7)
+
+
+MATS = [(name, m) for name, m in _mats() if np.diff(m[0]).max() <= 5]
+
+
+def _plan(cuda, rp, ci, v, **kw):
+    import torch
+    from capellinisptrsv_amd import Plan
+    return Plan(*(torch.from_numpy(np.ascontiguousarray(a)).to(cuda) for a in (rp, ci, v)), **kw)
+
+
+def _run(plan, cuda, b):
+    import torch
+    x = plan.solve(torch.from_numpy(np.ascontiguousarray(b)).to(cuda))
+    torch.cuda.synchronize()
+    assert plan.status() == 0
+    return x.cpu().numpy()
+
+
+@pytest.mark.parametrize("threads", [128, 256])
+@pytest.mark.parametrize("name,mat", MATS, ids=[m[0] for m in MATS])
+def test_hop_bit_exact(cuda, name, mat, threads):
+    rp, ci, v = mat
+    n = len(rp) - 1
+    for dtype, bits in ((np.float64, np.uint64), (np.float32, np.uint32)):
+        vt, b = v.astype(dtype), api.uniform(21, n).astype(dtype)
+        for arith, fused in (("fused", True), ("reference", False)):
+            plan = _plan(cuda, rp, ci, vt, algo="hop", row_threads=threads, arith=arith)
+            assert plan.hops() == hops_of(rp, ci)
+            x = _run(plan, cuda, b)
+            assert np.array_equal(x.view(bits), oracle.csr_forward(rp, ci, vt, b, fused=fused).view(bits)), (name, dtype)
+            assert np.array_equal(_run(plan, cuda, b).view(bits), x.view(bits))  # again on the same plan
+            plan.close()
+
+
+@pytest.mark.parametrize("kind", ["upper", "unit", "upper_unit"])
+def test_hop_triangular_kinds(cuda, kind):
+    """Rows are reversed inside the kernel (no copies of b and x): the
+    oracle's bits, also through reset / launch."""
+    import torch
+    rp, ci, v = random_lower(2500, max_off=4, band=300, seed=8, dup=False)
+    upper, unit = kind != "unit", kind != "upper"
+    if upper:
+        rp, ci, v = upper_from_lower(rp, ci, v)
+    if unit:
+        rp, ci, v = drop_diagonal(rp, ci, v, upper=upper)
+    n = len(rp) - 1
+    plan = _plan(cuda, rp, ci, v, algo="hop", upper=upper, unit_diagonal=unit)
+    b = api.uniform(22, n)
+    ref = oracle.csr_solve(rp, ci, v, b, upper=upper, unit=unit, fused=True)
+    assert np.array_equal(_run(plan, cuda, b).view(np.uint64), ref.view(np.uint64))
+    d, x = torch.from_numpy(b).to(cuda), torch.zeros(n, dtype=torch.float64, device=cuda)
+    plan.reset(x)
+    plan.launch(d, x)
+    assert plan.status() == 0
+    assert np.array_equal(x.cpu().numpy().view(np.uint64), ref.view(np.uint64))
+    # several right-hand sides go through the write-first kernel
+    bk = api.uniform(23, n * 3).reshape(n, 3)
+    xk = _run(plan, cuda, bk)
+    for q in range(3):
+        refq = oracle.csr_solve(rp, ci, v, np.ascontiguousarray(bk[:, q]), upper=upper, unit=unit, fused=True)
+        assert np.array_equal(xk[:, q], refq)
+    plan.close()
+
+
+def test_hop_reads_the_callers_values_and_special_values(cuda):
+    """The tables hold the pattern only: values changed in place between two
+    solves count.  Infinities, NaN and the sentinel's own bits in b spread
+    like in the write-first kernel."""
+    import torch
+    from capellinisptrsv_amd import Plan
+    rp, ci, v = random_lower(2000, max_off=3, band=200, seed=9)
+    d = [torch.from_numpy(a).to(cuda) for a in (rp, ci, v)]
+    plan = Plan(*d, algo="hop")
+    b = api.uniform(24, 2000)
+    assert np.array_equal(_run(plan, cuda, b), oracle.csr_forward(rp, ci, v, b, fused=True))
+    d[2].mul_(1.5)
+    assert np.array_equal(_run(plan, cuda, b), oracle.csr_forward(rp, ci, v * 1.5, b, fused=True))
+    b[3], b[700], b[1400] = np.inf, np.nan, np.array([0xFFF0000000000001], np.uint64).view(np.float64)[0]
+    plain = Plan(*d, algo="wrtfst")
+    x, ref = _run(plan, cuda, b), _run(plain, cuda, b)
+    assert np.array_equal(x, ref, equal_nan=True) and np.isnan(x).any() and np.isinf(x).any()
+    plan.close()
+    plain.close()
+
+
+def test_hop_refusals_and_replay(cuda):
+    import torch
+    rp, ci, v = random_lower(400, max_off=5, band=100, seed=10)
+    assert np.diff(rp).max() == 6
+    for kw in (dict(), dict(sync="flag"), dict(readiness="in_place"), dict(lds_window=True), dict(row_tiles=True)):
+        with pytest.raises(_native.CapError):
+            m = (rp, ci, v) if not kw else random_lower(400, max_off=3, band=100, seed=10)
+            _plan(cuda, *m, algo="hop", **kw)
+    rp, ci, v = api.make_config(1, seed=11, scale=0.02)
+    n = len(rp) - 1
+    plan = _plan(cuda, rp, ci, v, algo="hop")
+    b = torch.from_numpy(api.uniform(25, n)).to(cuda)
+    eager = plan.solve(b).clone()
+    out = torch.empty_like(b)
+    from test_gpu_capture import _replays
+    _replays(lambda: plan.solve(b, out=out, stream=torch.cuda.current_stream()), out, eager)
+    assert plan.status() == 0
+    plan.close()
