@@ -1811,13 +1811,15 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             cands.insert(cands.begin(), {CAP_ALGO_LEVEL, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
     }
     // thresholds 4 and 32 (see mix_border_for) always; 16 where the mean row
-    // length is at least 4 (some chunks may then reach it)
+    // length is at least 4 (some chunks may then reach it).  One workgroup per
+    // CU: two of its 1024-thread workgroups fill every wave slot, and in FP32,
+    // where they do fit, the untiled kernel on a 777,001-row wide-level matrix
+    // stalled until its waits gave up (10 s of plan creation); with row tiles
+    // two gave 268 us against one's 270.
     for (int bd : {kMixBorderWide, 16, kMixBorderNarrow})
         if (bd != 16 || avg * 4 >= bd) {
             cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 1, 0, stg, B});
-            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 2, 0, stg, B});
             cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 1, 0, stg, B, 1});
-            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 2, 0, stg, B, 1});
         }
     float best = 1e30f;
     TuneChoice pick = cands[0];
