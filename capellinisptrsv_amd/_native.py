@@ -86,6 +86,7 @@ SIGNATURES = {
     "cap_plan_tuning": (c_int, [c_void_p, PI, PI, PI, PI, PI, PI]),
     "cap_batch_info": (c_int, [c_void_p, PI, PI]),
     "cap_batch_tuning": (c_int, [c_void_p, PI, PI, PI, PI]),
+    "cap_batch_steps": (c_int, [c_void_p, PI]),
     "cap_batch_partitioned": (c_int, [c_void_p, PI, c_int]),
     "cap_plan_destroy": (c_int, [c_void_p]),
     "cap_plan_adjoint": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),

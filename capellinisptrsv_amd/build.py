@@ -54,8 +54,10 @@ def build_library(verbose: bool = True) -> str:
                         os.path.join(BUILD, "host_prep.o")],
         "solve.o": [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "solve.hip"), "-o",
                     os.path.join(BUILD, "solve.o")],
+        "steps.o": [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "steps.hip"), "-o",
+                    os.path.join(BUILD, "steps.o")],
     }
-    with ThreadPoolExecutor(max_workers=2) as ex:
+    with ThreadPoolExecutor(max_workers=3) as ex:
         list(ex.map(_run, objs.values()))
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-o", tmp,

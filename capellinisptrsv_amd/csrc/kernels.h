@@ -32,10 +32,10 @@
 
 #include <type_traits>
 
+#include "device_base.h"
+
 namespace cap {
 
-constexpr int kWave = 64;
-constexpr int kBlock = 256;       // 4 wavefronts per workgroup
 constexpr int kBlockSmall = 128;  // the thread-per-row kernels' other workgroup size
 // Thread-per-row workgroups of several right-hand sides (value protocol, no
 // LDS window): a ticket covers BLOCK / lanes-per-row rows, and each ticket
@@ -44,21 +44,6 @@ constexpr int kBlockSmall = 128;  // the thread-per-row kernels' other workgroup
 constexpr int kBlockLarge = 1024;
 constexpr int kWin = 4;      // dependencies polled concurrently per lane (flag protocol)
 
-
-template <typename T>
-struct VBits;
-template <>
-struct VBits<double> {
-    typedef unsigned long long U;
-    static constexpr U kSentinel = 0xFFF0000000000001ULL;  // negative signalling NaN
-    static constexpr U kQNaN = 0x7FF8000000000000ULL;
-};
-template <>
-struct VBits<float> {
-    typedef unsigned int U;
-    static constexpr U kSentinel = 0xFF800001u;
-    static constexpr U kQNaN = 0x7FC00000u;
-};
 
 template <typename U>
 __device__ __forceinline__ U ld_agent(const U *p)
@@ -70,12 +55,6 @@ __device__ __forceinline__ void st_agent(U *p, U v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ double as_val(unsigned long long u) { return __longlong_as_double((long long)u); }
-__device__ __forceinline__ float as_val(unsigned int u) { return __uint_as_float(u); }
-__device__ __forceinline__ unsigned long long as_bits(double v) { return (unsigned long long)__double_as_longlong(v); }
-__device__ __forceinline__ unsigned int as_bits(float v) { return __float_as_uint(v); }
-__device__ __forceinline__ double fmac(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fmac(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 // hardware FP / int atomic add at agent scope (global_atomic_add_f64 / _f32)
 template <typename V>
 __device__ __forceinline__ void atomic_add_agent(V *p, V v)
@@ -740,15 +719,6 @@ __global__ void __launch_bounds__(kBlock)
 {
     const int s = blockIdx.x * kBlock + threadIdx.x;
     if (s < n) slot[order[s]] = s;
-}
-
-// Workgroup barrier that orders LDS only: the plain __syncthreads would also
-// wait for the acknowledgement of the published values.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // One lane per row, tickets of BLOCK slots; wavefront 0 takes the next ticket
@@ -1583,173 +1553,6 @@ __global__ void __launch_bounds__(kLocalBlock)
                 local_rows_global<T>(rp, ci, val, b, xu, sc, k, sg, s_cur);
             if (lane == 0) __hip_atomic_store(s_cur + w, sg.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         });
-}
-
-// ------------------------------------------------ level steps in one workgroup
-// CAP_ALGO_LEVEL.  One workgroup walks the matrix level by level: the rows
-// of a level (in steps of at most B rows, B = the workgroup's 64 to
-// kLevelBlock threads, chosen by the plan) are solved in parallel,
-// one row per thread, and a workgroup barrier ends each step.  No thread
-// waits on another row's value, so there is no polling and no readiness
-// state; a step costs LDS reads, the row's chain and one barrier inside one
-// compute unit, against the memory round trip of a publish -> observe hop
-// between compute units.
-//
-// K right-hand sides (1, 2 or 4) are solved per row by the same thread,
-// interleaved in b and x (row * K + h); the ring holds K values per slot.
-//
-// Values travel through an LDS ring, row i in slot i & mask.  The plan
-// checks, for every off-diagonal entry c of a row in level L, that c > M_L -
-// R (M_L: the largest row index in levels <= L; R = mask + 1): no row that
-// maps to c's slot has been written by then.  Two slots follow the ring: R
-// holds 0 (never written) and R + 1 takes the padding rows' results.
-//
-// The row data is laid out by the plan in step order (slot s * B +
-// thread): {row, off-diagonal count}, the first E entries in stored order as
-// ring slots (c & mask) and values, and the diagonal.  Unused entries are
-// (slot R, value 0) and padding rows are {-1, 0} with diagonal 1, so every
-// thread runs the same straight-line step: fma(0, 0, s) = s exactly (a sum
-// that starts at +0 is never -0), and padding results go to slot R + 1 and
-// to the sink.  Rows longer than E read the rest from the CSR (LONG).  The
-// data is loaded D steps ahead into registers, the {row, count} pair 2D
-// steps ahead (b is gathered through the row index); the barriers order LDS
-// alone, so they do not wait for those loads.  The plan pads the steps to a
-// multiple of 2D with padding slots.  Each sum is the thread-per-row
-// kernels' stored-order chain and division: the same x bit for bit.
-constexpr int kLevelBlock = 256;
-constexpr int kLevelDepth4 = 10;  // steps of row data in flight with E = 4 entries carried
-constexpr int kLevelDepth8 = 6;   // with E = 8 (the load counter holds 63 loads in flight)
-constexpr int kLevelDepthK2 = 8;  // E = 4, 2 right-hand sides per row (registers)
-constexpr int kLevelDepthK4 = 6;  // E = 4, 4 right-hand sides per row
-
-template <typename T, int E, int K>
-struct LevelStage {
-    int row, cnt;
-    int c[E];
-    T v[E];
-    T d, bo[K];
-};
-
-// 16-byte loads of E consecutive elements (E * sizeof(T) is a multiple of
-// 16 for the instantiated E; the plan's arrays are 16-byte aligned)
-template <typename V, int E>
-__device__ __forceinline__ void load16(const V *__restrict__ src, V (&dst)[E])
-{
-    static_assert((E * sizeof(V)) % 16 == 0, "E values must fill 16-byte loads");
-    const uint4 *s4 = reinterpret_cast<const uint4 *>(src);
-#pragma unroll
-    for (int h = 0; h < (int)(E * sizeof(V) / 16); ++h) {
-        const uint4 w = s4[h];
-        __builtin_memcpy(reinterpret_cast<char *>(dst) + 16 * h, &w, 16);
-    }
-}
-
-template <typename T, int E, int K>
-__device__ __forceinline__ void level_load(LevelStage<T, E, K> &st, int2 rec, unsigned q, const int *__restrict__ lci,
-                                           const T *__restrict__ lv, const T *__restrict__ ld, const T *__restrict__ b)
-{
-    st.row = rec.x;
-    st.cnt = rec.y;
-    load16<int, E>(lci + (size_t)q * E, st.c);
-    load16<T, E>(lv + (size_t)q * E, st.v);
-    st.d = ld[q];
-    // padding slots read row 0's b, unused
-    if constexpr (K == 1) {
-        st.bo[0] = b[rec.x < 0 ? 0 : rec.x];
-    } else {
-        const size_t o = (size_t)(rec.x < 0 ? 0 : rec.x) * K;
-#pragma unroll
-        for (int h = 0; h < K; ++h) st.bo[h] = b[o + h];
-    }
-}
-
-__device__ __forceinline__ void level_barrier()
-{
-    // only LDS carries values between steps: the fences order LDS alone, so
-    // the barrier does not wait for the row-data loads in flight
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <typename T, int E, int D, bool UNFUSED, bool LONG, int K>
-__global__ void __launch_bounds__(kLevelBlock)
-    k_level(const int2 *__restrict__ rec, const int *__restrict__ lci, const T *__restrict__ lv,
-            const T *__restrict__ ld, const int *__restrict__ rp, const int *__restrict__ ci,
-            const T *__restrict__ val, const T *__restrict__ b, T *__restrict__ x, T *__restrict__ sink, int steps,
-            int mask)
-{
-    const int B = blockDim.x;
-    typedef typename VBits<T>::U U;
-    extern __shared__ unsigned long long smem_level[];
-    T *ring = reinterpret_cast<T *>(smem_level);
-    const int t = threadIdx.x;
-    LevelStage<T, E, K> st[D];
-    int2 ahead[D], first[D];
-    // the row pairs first, so no stage's b load waits behind another stage
-#pragma unroll
-    for (int r = 0; r < D; ++r) first[r] = rec[r * B + t];
-#pragma unroll
-    for (int r = 0; r < D; ++r) ahead[r] = rec[(D + r) * B + t];
-#pragma unroll
-    for (int r = 0; r < D; ++r) level_load<T, E, K>(st[r], first[r], r * B + t, lci, lv, ld, b);
-    if (t < K) ring[(mask + 1) * K + t] = (T)0;
-    level_barrier();
-    // Two rounds of the D stages per iteration (steps is a multiple of 2D,
-    // padded by the plan, so the body has no exit): the compiler's
-    // load-counter waits are exact in the second round (the first round's,
-    // merged at the loop head, assume about half the loads in flight).
-    for (int s0 = 0; s0 < steps; s0 += 2 * D) {
-#pragma unroll
-        for (int h = 0; h < 2 * D; ++h) {
-            const int r = h % D;
-            const int s = s0 + h;
-            const LevelStage<T, E, K> &w = st[r];
-            T xv[E][K];
-#pragma unroll
-            for (int u = 0; u < E; ++u)
-#pragma unroll
-                for (int h = 0; h < K; ++h) xv[u][h] = ring[w.c[u] * K + h];
-            T sum[K];
-#pragma unroll
-            for (int h = 0; h < K; ++h) {
-                sum[h] = (T)0;
-#pragma unroll
-                for (int u = 0; u < E; ++u)
-                    sum[h] = UNFUSED ? sum[h] + w.v[u] * xv[u][h] : fmac(w.v[u], xv[u][h], sum[h]);
-            }
-            if (LONG && w.cnt > E) {  // the rest of a long row, from the CSR
-                const int j1 = rp[w.row] + w.cnt;
-                for (int j = j1 - w.cnt + E; j < j1; ++j) {
-                    const T a = val[j];
-                    const int c = (ci[j] & mask) * K;
-#pragma unroll
-                    for (int h = 0; h < K; ++h) sum[h] = UNFUSED ? sum[h] + a * ring[c + h] : fmac(a, ring[c + h], sum[h]);
-                }
-            }
-            const bool real = w.row >= 0;
-            const int slot = (real ? w.row & mask : mask + 2) * K;
-#pragma unroll
-            for (int h = 0; h < K; ++h) {
-                U o = as_bits((w.bo[h] - sum[h]) / w.d);
-                if (o == VBits<T>::kSentinel) o = VBits<T>::kQNaN;  // as the publishing kernels do
-                ring[slot + h] = as_val(o);
-                if constexpr (K == 1)
-                    *(real ? x + w.row : sink) = as_val(o);
-                else
-                    *(real ? x + (size_t)w.row * K + h : sink + h) = as_val(o);
-            }
-            // refill this stage for step s + D (padded: the arrays hold 2D
-            // steps past the last), and its row pair for step s + 2D.  Kept
-            // after the step's own work: interleaved with it, the compiler
-            // parks in-flight load results in accumulation registers, and
-            // each such move waits for its load.
-            __builtin_amdgcn_sched_barrier(0);
-            level_load<T, E, K>(st[r], ahead[r], (s + D) * B + t, lci, lv, ld, b);
-            ahead[r] = rec[(s + 2 * D) * B + t];
-            level_barrier();
-        }
-    }
 }
 
 // ------------------------------------------------ SyncFree CSC (K4 / K5)

@@ -19,6 +19,7 @@
 #include "../../include/capellini_sptrsv.h"
 #include "cap_internal.h"
 #include "kernels.h"
+#include "steps.h"
 
 using namespace cap;
 
@@ -96,20 +97,6 @@ struct PartState {
     double *res = nullptr, *cor = nullptr;  // refinement: FP64 residual and correction (n * kcap)
 };
 
-// Step-ordered row data of CAP_ALGO_LEVEL (layout in kernels.h, k_level):
-// steps + 2 * depth steps of `block` slots (the workgroup size); E entries
-// carried per slot;
-// the LDS ring has mask + 1 slots.
-constexpr int kCtrlSink = 2048;  // k_level's padding-lane stores (up to 4 values, never read)
-struct LevelState {
-    int2 *rec = nullptr;
-    int *ci = nullptr;
-    void *v = nullptr, *d = nullptr;
-    int steps = 0, E = 4, mask = 0, block = kLevelBlock;
-    bool long_rows = false;  // some row has more than E off-diagonal entries
-    int max_rhs = 1;         // right-hand sides per solve: 1, or 2 / 4 where their ring fits LDS (E = 4)
-};
-
 // Look-through tables of the write-first solve (layout in kernels.h, k_hop):
 // E entries per row, `hops` publish -> observe hops on the longest chain.
 struct HopState {
@@ -143,8 +130,7 @@ struct cap_plan_s {
     long long flags_len = 0;
     int epoch = 0;
     // control block (one 4 KiB allocation): tickets at +0, watchdog word at
-    // +256, refinement norms at +512, poll counters at +1024, the level
-    // steps' store sink at +kCtrlSink
+    // +256, refinement norms at +512, poll counters at +1024
     unsigned char *ctrl = nullptr;
     unsigned *ticket = nullptr;
     int *err = nullptr;
@@ -208,8 +194,15 @@ struct cap_plan_s {
     int graph_rhs = 0;
     // partitioned banded solve (CAP_ALGO_PARTITION)
     struct PartState *part = nullptr;
-    // level steps in one workgroup (CAP_ALGO_LEVEL)
-    LevelState *lvl = nullptr;
+    // steps in one workgroup (CAP_ALGO_LEVEL).  lvl_rhs: right-hand sides per
+    // solve an explicit plan takes (1, 2 or 4; 0: any).  lvl_live: the tables
+    // take the caller's values again on every solve
+    StepTables *lvl = nullptr;
+    int lvl_rhs = 0;
+    bool lvl_live = false;
+    // batch: the matrices outside the partitioned ones solved by steps, one
+    // workgroup per matrix and right-hand-side chunk (nullptr: by algo)
+    StepTables *batch_steps = nullptr;
     // write-first solve of one right-hand side with look-through tables
     // (autotuned plans, value protocol, staged readiness)
     HopState *hop = nullptr;
@@ -222,11 +215,12 @@ inline bool hop_takes(const cap_plan_s *p, int rhs)
     return p->hop && rhs == 1 && p->algo == CAP_ALGO_WRTFST && p->sync == CAP_SYNC_VALUE && p->staged;
 }
 
-// Right-hand-side counts a level plan solves: 1, and 2 or 4 where a ring of
-// that many values per slot fits LDS (rows of at most 4 off-diagonals).
+// Right-hand-side counts a plan's steps solve: an explicit level plan's 1,
+// and 2 or 4 where its rule allows; any of an autotuned one's.
 inline bool level_takes(const cap_plan_s *p, int rhs)
 {
-    return p->lvl && (rhs == 1 || ((rhs == 2 || rhs == 4) && rhs <= p->lvl->max_rhs));
+    if (!steps_take(p->lvl, rhs)) return false;
+    return p->lvl_rhs == 0 || rhs == 1 || ((rhs == 2 || rhs == 4) && rhs <= p->lvl_rhs);
 }
 
 // Side streams of a hybrid batch: its partitioned matrices' solves run
@@ -416,12 +410,9 @@ void free_partition(cap_plan p)
 
 void free_level(cap_plan p)
 {
-    LevelState *ls = p->lvl;
-    if (!ls) return;
+    if (!p->lvl) return;
     (void)hipDeviceSynchronize();
-    for (void *b : {(void *)ls->rec, (void *)ls->ci, ls->v, ls->d})
-        if (b) (void)hipFree(b);
-    delete ls;
+    steps_free(p->lvl);
     p->lvl = nullptr;
 }
 
@@ -441,6 +432,7 @@ void plan_free(cap_plan p)
     free_partition(p);
     free_level(p);
     free_hop(p);
+    steps_free(p->batch_steps);
     if (p->ready) {
         (void)hipDeviceSynchronize();  // no kernel of this plan may still poll the block
         ready_release(p->ready);
@@ -537,13 +529,20 @@ int launch_prepare(cap_plan p, int algo, int sync, void *x, long long count, hip
 // matrix, or (batches) for every matrix, ordered by decreasing nonzero count
 // so that the largest matrices start first.  The bandwidth (largest row -
 // column distance) decides whether a segment's dependencies fit the LDS ring.
-int ensure_segments(cap_plan p, const std::vector<int> *row_off)
+// rp_host, ci_host: host copies of the rows where the caller has them.
+int ensure_segments(cap_plan p, const std::vector<int> *row_off, const std::vector<int> *rp_host = nullptr,
+                    const std::vector<int> *ci_host = nullptr)
 {
     if (p->seg && !row_off) return CAP_OK;
     const int n = p->n;
-    std::vector<int> rp((size_t)n + 1), ci((size_t)p->nnz), bw((size_t)std::max(n, 1), 0);
-    CAP_HIP_TRY(hipMemcpy(rp.data(), p->rp, sizeof(int) * rp.size(), hipMemcpyDeviceToHost));
-    CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * ci.size(), hipMemcpyDeviceToHost));
+    std::vector<int> rp_own, ci_own, bw((size_t)std::max(n, 1), 0);
+    if (!rp_host) {
+        rp_own.resize((size_t)n + 1);
+        ci_own.resize((size_t)p->nnz);
+        CAP_HIP_TRY(hipMemcpy(rp_own.data(), p->rp, sizeof(int) * rp_own.size(), hipMemcpyDeviceToHost));
+        CAP_HIP_TRY(hipMemcpy(ci_own.data(), p->ci, sizeof(int) * ci_own.size(), hipMemcpyDeviceToHost));
+    }
+    const std::vector<int> &rp = rp_host ? *rp_host : rp_own, &ci = rp_host ? *ci_host : ci_own;
     for (int i = 0; i < n; ++i)
         for (int j = rp[i]; j < rp[i + 1]; ++j) bw[i] = std::max(bw[i], i - ci[j]);
     std::vector<int4> h;
@@ -935,28 +934,10 @@ int launch_kernel(cap_plan p, int algo, int sync, const T *val, const T *b, T *x
         k_local<T><<<nb, kLocalBlock, bytes, st>>>(p->rp, p->ci, val, b, x, sc, rhs, p->seg, p->n_seg, p->ticket,
                                                     rl);
     } else if (algo == CAP_ALGO_LEVEL) {
-        // one right-hand side, the plan's own values (the tables hold them)
-        const LevelState *ls = p->lvl;
+        // the plan's own values (the tables hold them)
         if (!level_takes(p, rhs) || (const void *)val != p->val) return CAP_ERR_UNSUPPORTED;
-        // the ring, its zero slot and its sink slot, rhs values each
-        const size_t bytes = (size_t)(ls->mask + 3) * rhs * sizeof(T);
-        const T *lv = (const T *)ls->v, *ld = (const T *)ls->d;
-        T *sink = reinterpret_cast<T *>(p->ctrl + kCtrlSink);
-        auto go = [&](auto kernel) {
-            kernel<<<1, ls->block, bytes, st>>>(ls->rec, ls->ci, lv, ld, p->rp, p->ci, val, b, x, sink, ls->steps,
-                                                  ls->mask);
-        };
-        const bool uf = sc.unfused != 0;
-        if (rhs == 2)
-            uf ? go(k_level<T, 4, kLevelDepthK2, true, false, 2>) : go(k_level<T, 4, kLevelDepthK2, false, false, 2>);
-        else if (rhs == 4)
-            uf ? go(k_level<T, 4, kLevelDepthK4, true, false, 4>) : go(k_level<T, 4, kLevelDepthK4, false, false, 4>);
-        else if (ls->E == 4)
-            uf ? go(k_level<T, 4, kLevelDepth4, true, false, 1>) : go(k_level<T, 4, kLevelDepth4, false, false, 1>);
-        else if (!ls->long_rows)
-            uf ? go(k_level<T, 8, kLevelDepth8, true, false, 1>) : go(k_level<T, 8, kLevelDepth8, false, false, 1>);
-        else
-            uf ? go(k_level<T, 8, kLevelDepth8, true, true, 1>) : go(k_level<T, 8, kLevelDepth8, false, true, 1>);
+        if (p->lvl_live) CAP_TRY(steps_refresh(p->lvl, p->rp, p->ci, p->val, st));
+        return steps_launch(p->lvl, b, x, rhs, sc.unfused != 0, st);
     } else if (algo == CAP_ALGO_CSC) {
         if (rhs != 1) return CAP_ERR_UNSUPPORTED;
         // lanes per column from the mean column length (diagonal included)
@@ -1540,31 +1521,26 @@ int build_partition_tables(cap_plan p, const std::vector<int> &rp_host, hipStrea
     return rc;
 }
 
-// Tables of CAP_ALGO_LEVEL (k_level), from host copies of the rows.  The
-// workgroup size B is the smallest of 64, 128, 192 and 256 threads that
-// needs at most 1/8 more steps than 256 would (fewer wavefronts per
-// barrier, fewer padding slots).  The rows of each level fill whole steps of B slots in
-// row order; the
-// ring is the smallest power of two (>= 64) that keeps every off-diagonal
-// entry's value in place until its last reader (c > M_L - R, see k_level);
-// entries are stored as ring slots, unused ones as (slot R, value 0).
-// CAP_ERR_UNSUPPORTED when that ring exceeds kLevelRingBytes, or the padded
-// steps exceed kLevelPadMax slots per row (many narrow levels: a thread per
-// slot would mostly idle).
+// What an explicit CAP_ALGO_LEVEL plan takes, from its levels.  Every
+// off-diagonal entry c of a row in level L must satisfy c > M_L - R (M_L:
+// the largest row index in levels <= L) with a ring R, a power of two >= 64,
+// of at most kLevelRingBytes of values; and the levels padded to whole steps
+// of B rows -- B the smallest of 64, 128, 192 and 256 that needs at most 1/8
+// more steps than 256 -- must hold at most kLevelPadMax slots per row.  The
+// solve schedules rows more freely (steps.hip) and needs less; an autotuned
+// plan uses the steps wherever that schedule fits.  *max_rhs: 1, or 2 or 4
+// where rows hold at most 4 off-diagonals and R values of each fit LDS.
 constexpr size_t kLevelRingBytes = 65536;
-constexpr double kLevelMaxWidth = 4096;  // the autotuner tries the level steps up to these rows per level
+constexpr double kLevelMaxWidth = 4096;  // the autotuner tries the steps up to these rows per level
 constexpr int kLevelPadMax = 4;
+// An autotuned plan's steps may be mostly idle threads: with 4 rows per
+// level a step still costs a third of what the one-workgroup kernel spends
+// on them one by one.
+constexpr int kStepPadMax = 16;
 
-template <typename T>
-int build_level_t(cap_plan p, const std::vector<int> &rp)
+int level_accepts(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, int *max_rhs)
 {
-    const int n = p->n, nnz = p->nnz;
-    std::vector<int> ci((size_t)nnz);
-    std::vector<T> v((size_t)nnz);
-    if (nnz) {
-        CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * ci.size(), hipMemcpyDeviceToHost));
-        CAP_HIP_TRY(hipMemcpy(v.data(), p->val, sizeof(T) * v.size(), hipMemcpyDeviceToHost));
-    }
+    const int n = p->n, vb = p->vbytes;
     std::vector<int> lv((size_t)std::max(n, 1));
     const int L = n ? cap_matrix_layer(n, rp.data(), ci.data(), nullptr, nullptr, lv.data()) : 0;  // 1-based
     std::vector<long long> width((size_t)L + 1, 0);
@@ -1581,94 +1557,39 @@ int build_level_t(cap_plan p, const std::vector<int> &rp)
         for (int j = rp[i]; j < rp[i + 1] - 1; ++j) need = std::max(need, (long long)top[(size_t)lv[i]] - ci[j] + 1);
     long long R = 64;
     while (R < need) R *= 2;
-    if ((size_t)R * sizeof(T) > kLevelRingBytes) return CAP_ERR_UNSUPPORTED;
-    const int E = maxoff <= 4 ? 4 : 8;
-    const int D = E == 4 ? kLevelDepth4 : kLevelDepth8;
+    if ((size_t)(R * vb) > kLevelRingBytes) return CAP_ERR_UNSUPPORTED;
     auto steps_for = [&](int B) {
         long long c = 0;
         for (int l = 1; l <= L; ++l) c += (width[(size_t)l] + B - 1) / B;
         return c;
     };
-    int B = kLevelBlock;
-    const long long full = steps_for(kLevelBlock);
-    for (int cand = kLevelBlock - kWave; cand >= kWave; cand -= kWave)
+    int B = 256;
+    const long long full = steps_for(B);
+    for (int cand = B - kWave; cand >= kWave; cand -= kWave)
         if (steps_for(cand) <= full + full / 8) B = cand;
-    std::vector<long long> next((size_t)L + 1, 0);  // next free slot of each level
-    long long steps = 0;
-    for (int l = 1; l <= L; ++l) {
-        next[(size_t)l] = steps * B;
-        steps += (width[(size_t)l] + B - 1) / B;
-    }
-    if (steps * B > std::max((long long)kLevelPadMax * n, 1LL << 16)) return CAP_ERR_UNSUPPORTED;
-    steps = (steps + 2 * D - 1) / (2 * D) * (2 * D);  // the kernel runs whole rounds of 2D steps
-    const size_t S = (size_t)(steps + 2 * D) * B;
-    if (S * E > (size_t)INT32_MAX) return CAP_ERR_UNSUPPORTED;  // the kernel's 32-bit slot indices
-    std::vector<int2> rec(S, make_int2(-1, 0));
-    std::vector<int> lci(S * E, (int)R);
-    std::vector<T> lval(S * E, (T)0), ldiag(S, (T)1);
-    for (int i = 0; i < n; ++i) {
-        const size_t q = (size_t)next[(size_t)lv[i]]++;
-        const int off = rp[i + 1] - 1 - rp[i];
-        rec[q] = make_int2(i, off);
-        for (int u = 0; u < std::min(off, E); ++u) {
-            lci[q * E + u] = ci[(size_t)rp[i] + u] & (int)(R - 1);
-            lval[q * E + u] = v[(size_t)rp[i] + u];
-        }
-        ldiag[q] = v[(size_t)rp[i + 1] - 1];
-    }
-    free_level(p);
-    LevelState *ls = new LevelState();
-    p->lvl = ls;
-    ls->steps = (int)steps;
-    ls->E = E;
-    ls->mask = (int)R - 1;
-    ls->long_rows = maxoff > E;
-    ls->block = B;
-    // the ring and its two extra slots (K values each) may pass the default
-    // 64 KiB of dynamic LDS; 2 and 4 right-hand sides where they fit
-    ls->max_rhs = E == 4 && (size_t)(R + 2) * 4 * sizeof(T) <= (size_t)p->lds_max   ? 4
-                  : E == 4 && (size_t)(R + 2) * 2 * sizeof(T) <= (size_t)p->lds_max ? 2
-                                                                                     : 1;
-    auto allow = [&](auto kernel, int K) {
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)((R + 2) * K * sizeof(T))) == hipSuccess;
-    };
-    bool ok;
-    if (E == 4) {
-        ok = allow(&k_level<T, 4, kLevelDepth4, true, false, 1>, 1) && allow(&k_level<T, 4, kLevelDepth4, false, false, 1>, 1);
-        if (ok && ls->max_rhs >= 2)
-            ok = allow(&k_level<T, 4, kLevelDepthK2, true, false, 2>, 2) &&
-                 allow(&k_level<T, 4, kLevelDepthK2, false, false, 2>, 2);
-        if (ok && ls->max_rhs >= 4)
-            ok = allow(&k_level<T, 4, kLevelDepthK4, true, false, 4>, 4) &&
-                 allow(&k_level<T, 4, kLevelDepthK4, false, false, 4>, 4);
-    } else if (!ls->long_rows) {
-        ok = allow(&k_level<T, 8, kLevelDepth8, true, false, 1>, 1) && allow(&k_level<T, 8, kLevelDepth8, false, false, 1>, 1);
-    } else {
-        ok = allow(&k_level<T, 8, kLevelDepth8, true, true, 1>, 1) && allow(&k_level<T, 8, kLevelDepth8, false, true, 1>, 1);
-    }
-    if (!ok) {
-        free_level(p);
-        return CAP_ERR_HIP;
-    }
-    if (hipMalloc(&ls->rec, sizeof(int2) * S) != hipSuccess || hipMalloc(&ls->ci, sizeof(int) * lci.size()) != hipSuccess ||
-        hipMalloc(&ls->v, sizeof(T) * lval.size()) != hipSuccess || hipMalloc(&ls->d, sizeof(T) * S) != hipSuccess) {
-        free_level(p);
-        return CAP_ERR_ALLOC;
-    }
-    if (hipMemcpy(ls->rec, rec.data(), sizeof(int2) * S, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(ls->ci, lci.data(), sizeof(int) * lci.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(ls->v, lval.data(), sizeof(T) * lval.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(ls->d, ldiag.data(), sizeof(T) * S, hipMemcpyHostToDevice) != hipSuccess) {
-        free_level(p);
-        return CAP_ERR_HIP;
-    }
+    if (steps_for(B) * B > std::max((long long)kLevelPadMax * n, 1LL << 16)) return CAP_ERR_UNSUPPORTED;
+    *max_rhs = maxoff > 4                              ? 1
+               : (R + 2) * 4 * vb <= (long long)p->lds_max ? 4
+               : (R + 2) * 2 * vb <= (long long)p->lds_max ? 2
+                                                           : 1;
     return CAP_OK;
 }
 
-int build_level(cap_plan p, const std::vector<int> &rp_host)
+// The plan's step tables.  An explicit plan is held to level_accepts.  An
+// autotuned plan whose matrix that rule refuses, over the caller's own
+// values, copies them into the tables again on every solve (about 10 us):
+// the kernels it would run otherwise read them there.
+int build_level(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, bool explicit_algo, hipStream_t st)
 {
-    return p->vt == CAP_F64 ? build_level_t<double>(p, rp_host) : build_level_t<float>(p, rp_host);
+    int rule_rhs = 0;
+    const int rule = level_accepts(p, rp, ci, &rule_rhs);
+    if (explicit_algo && rule != CAP_OK) return rule;
+    free_level(p);
+    CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rule_rhs : 4, p->lds_max,
+                        kStepPadMax, p->rp, p->ci, p->val, st));
+    p->lvl_rhs = explicit_algo ? rule_rhs : 0;
+    p->lvl_live = rule != CAP_OK && !p->owns_matrix;
+    return CAP_OK;
 }
 
 // Look-through tables of the write-first solve (k_hop): each row's hop
@@ -1761,7 +1682,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             apply_choice(p, it->second);
             if (p->algo == CAP_ALGO_MIX) return build_mix(p, rp_host, it->second.border);
             if (p->algo == CAP_ALGO_LOCAL) return ensure_segments(p, nullptr);
-            if (p->algo == CAP_ALGO_LEVEL) return build_level(p, rp_host);
+            if (p->algo == CAP_ALGO_LEVEL) return build_level(p, rp_host, ci, false, st);
             if (it->second.hop) return build_hop(p, rp_host, ci, st);
             if (p->algo != CAP_ALGO_PARTITION) return CAP_OK;
             // the pick was cached for this structure; these values may not
@@ -1804,10 +1725,10 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             if (!p->unfused && build_partition(p, rp_host, st) == CAP_OK)
                 cands.insert(cands.begin(), {CAP_ALGO_PARTITION, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
         }
-        // level steps in one workgroup, where the ring and the padding allow:
-        // up to a few thousand rows per level a step per 256 rows can still
-        // beat a cross-CU hop per level
-        if ((double)p->n / std::max(1, levels) <= kLevelMaxWidth && build_level(p, rp_host) == CAP_OK)
+        // steps in one workgroup, where the ring and the padding allow: up to
+        // a few thousand rows per level a step per 256 rows can still beat a
+        // cross-CU hop per level
+        if ((double)p->n / std::max(1, levels) <= kLevelMaxWidth && build_level(p, rp_host, ci, false, st) == CAP_OK)
             cands.insert(cands.begin(), {CAP_ALGO_LEVEL, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
     }
     // thresholds 4 and 32 (see mix_border_for) always; 16 where the mean row
@@ -2068,7 +1989,7 @@ int plan_create_impl(cap_plan *out, int n, int nnz, const int *rp, const int *ci
         } else if (p->algo == CAP_ALGO_PARTITION) {
             rc = build_partition(p, rp_host, st);
         } else if (p->algo == CAP_ALGO_LEVEL) {
-            rc = build_level(p, rp_host);
+            if ((rc = host_columns(p, &ci_host)) == CAP_OK) rc = build_level(p, rp_host, ci_host, true, st);
         } else if (p->algo == CAP_ALGO_HOP) {
             p->algo = CAP_ALGO_WRTFST;
             if ((rc = host_columns(p, &ci_host)) == CAP_OK) rc = build_hop(p, rp_host, ci_host, st);
@@ -2644,14 +2565,15 @@ extern "C" int cap_plan_solve_refined(cap_plan p, const double *b, double *x, in
 namespace {
 
 // Row levels of a batch's block-diagonal matrix (host copy).
-int batch_levels(cap_plan p, std::vector<int> *lv)
+int batch_levels(cap_plan p, std::vector<int> *rp, std::vector<int> *ci, std::vector<int> *lv)
 {
     const int n = p->n, nnz = p->nnz;
-    std::vector<int> rp((size_t)n + 1), ci((size_t)nnz);
+    rp->resize((size_t)n + 1);
+    ci->resize((size_t)nnz);
     lv->assign((size_t)std::max(n, 1), 0);
-    CAP_HIP_TRY(hipMemcpy(rp.data(), p->rp, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost));
-    CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost));
-    cap_matrix_layer(n, rp.data(), ci.data(), nullptr, nullptr, lv->data());
+    CAP_HIP_TRY(hipMemcpy(rp->data(), p->rp, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost));
+    CAP_HIP_TRY(hipMemcpy(ci->data(), p->ci, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost));
+    cap_matrix_layer(n, rp->data(), ci->data(), nullptr, nullptr, lv->data());
     return CAP_OK;
 }
 
@@ -2821,16 +2743,24 @@ int plan_launch_with(cap_plan p, int algo, int sync, const void *b, void *x, int
 int batch_solve_parts(cap_plan p, const std::vector<cap_plan> &parts, const std::vector<int> &lo, int k,
                       const void *b, void *x, hipStream_t st, const Fork *fk)
 {
-    if (parts.empty()) return plan_solve_with(p, p->algo, p->sync, b, x, k, st);
+    // the rest by steps: no reset, only the rest's rows of x are touched
+    const StepTables *steps = p->batch_steps;
+    if (parts.empty())
+        return steps ? steps_launch(steps, b, x, k, p->unfused != 0, st)
+                     : plan_solve_with(p, p->algo, p->sync, b, x, k, st);
     const size_t row_bytes = (size_t)k * p->vbytes;
-    const bool x_reset = !p->staged && p->algo != CAP_ALGO_LOCAL;
+    const bool x_reset = !steps && !p->staged && p->algo != CAP_ALGO_LOCAL;
     if (x_reset) CAP_TRY(plan_reset_with(p, p->algo, p->sync, x, k, st));
     int rc = fork_parts(parts.size(), fk, st, [&](size_t h, hipStream_t s) {
         return plan_solve_with(parts[h], parts[h]->algo, parts[h]->sync, (const char *)b + lo[h] * row_bytes,
                                (char *)x + lo[h] * row_bytes, k, s);
     });
-    if (rc == CAP_OK && !x_reset) rc = plan_reset_with(p, p->algo, p->sync, x, k, st);
-    if (rc == CAP_OK) rc = plan_launch_with(p, p->algo, p->sync, b, x, k, st);
+    if (rc == CAP_OK && steps) {
+        rc = steps_launch(steps, b, x, k, p->unfused != 0, st);
+    } else {
+        if (rc == CAP_OK && !x_reset) rc = plan_reset_with(p, p->algo, p->sync, x, k, st);
+        if (rc == CAP_OK) rc = plan_launch_with(p, p->algo, p->sync, b, x, k, st);
+    }
     const int rj = join_parts(fk, st);  // joined whatever happened
     return rc != CAP_OK ? rc : rj;
 }
@@ -2856,6 +2786,47 @@ float time_batch(cap_plan p, const std::vector<cap_plan> &parts, const std::vect
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     return best;
+}
+
+// Steps for a batch's matrices (those outside `lo`, the partitioned ones):
+// kept where the tables fit and the whole batch solve is 2 % faster with
+// them.  The thread-per-row schedule pays a cross-CU hop per level of the
+// deepest matrix (1.16 us on 40 matrices of up to 775 levels with 16
+// right-hand sides, 898 us); a step inside one CU costs 0.33 us there.
+int choose_batch_steps(cap_plan p, int k, const std::vector<int> &ro, const std::vector<int> &rp,
+                       const std::vector<int> &ci, const std::vector<cap_plan> &parts, const std::vector<int> &lo,
+                       const Fork *fk, hipStream_t st)
+{
+    std::vector<int2> mats;
+    for (size_t m = 0; m + 1 < ro.size(); ++m)
+        if (ro[m + 1] > ro[m] && std::find(lo.begin(), lo.end(), ro[m]) == lo.end())
+            mats.push_back(make_int2(ro[m], ro[m + 1]));
+    if (mats.empty()) return CAP_OK;
+    StepTables *t = nullptr;
+    int rc = steps_build(&t, rp, ci, mats, p->vt, 4, p->lds_max, kStepPadMax, p->rp, p->ci, p->val, st);
+    if (rc == CAP_ERR_UNSUPPORTED || rc == CAP_ERR_ALLOC) return CAP_OK;  // the plain batch stays
+    if (rc != CAP_OK) return rc;
+    if (!steps_take(t, k)) {
+        steps_free(t);
+        return CAP_OK;
+    }
+    const size_t bytes = (size_t)p->n * k * p->vbytes + 8;
+    void *b = nullptr, *x = nullptr;
+    if (hipMalloc(&b, bytes) != hipSuccess || hipMalloc(&x, bytes) != hipSuccess ||
+        hipMemsetAsync(b, 0, bytes, st) != hipSuccess)
+        rc = CAP_ERR_ALLOC;
+    float plain = 0, with = 0;
+    if (rc == CAP_OK) plain = time_batch(p, parts, lo, k, b, x, st, &rc, fk);
+    p->batch_steps = t;
+    if (rc == CAP_OK) with = time_batch(p, parts, lo, k, b, x, st, &rc, fk);
+    (void)hipStreamSynchronize(st);
+    (void)hipFree(b);
+    (void)hipFree(x);
+    if (rc != CAP_OK || with >= 0.98f * plain) {
+        p->batch_steps = nullptr;
+        steps_free(t);
+    }
+    return rc;
 }
 
 // Hybrid batch: a deep matrix (few rows per level) sets the whole batch's
@@ -3091,10 +3062,10 @@ int cap_batch_create(cap_batch *out, int n_mat, const int *row_off, const int *r
         return rc;
     }
     p->owns_matrix = true;
-    std::vector<int> lv;
-    if ((rc = batch_levels(p, &lv)) != CAP_OK ||
+    std::vector<int> lv, rp_host, ci_host;
+    if ((rc = batch_levels(p, &rp_host, &ci_host, &lv)) != CAP_OK ||
         (rc = build_batch_schedule(p, ro, lv, p->wblock >> lpr_log2_for(k), st)) != CAP_OK ||
-        (rc = ensure_segments(p, &ro)) != CAP_OK ||
+        (rc = ensure_segments(p, &ro, &rp_host, &ci_host)) != CAP_OK ||
         (rc = choose_batch_algo(p, o.algo, o.blocks_per_cu > 0, k, ro, lv, st)) != CAP_OK) {
         cap_plan_destroy(p);
         return rc;
@@ -3104,6 +3075,13 @@ int cap_batch_create(cap_batch *out, int n_mat, const int *row_off, const int *r
     Fork fork;
     if (o.algo == CAP_ALGO_AUTO &&
         (rc = choose_batch_hybrid(p, k, o.blocks_per_cu > 0, ro, lv, st, &parts, &part_lo, &fork)) != CAP_OK) {
+        cap_plan_destroy(p);
+        return rc;
+    }
+    if (o.algo == CAP_ALGO_AUTO && o.blocks_per_cu == 0 && p->sync == CAP_SYNC_VALUE && !p->count_polls &&
+        (rc = choose_batch_steps(p, k, ro, rp_host, ci_host, parts, part_lo, &fork, st)) != CAP_OK) {
+        for (cap_plan q : parts) cap_plan_destroy(q);
+        fork.release();
         cap_plan_destroy(p);
         return rc;
     }
@@ -3143,6 +3121,13 @@ int cap_batch_partitioned(cap_batch bt, int *first_rows, int capacity)
     const int cnt = (int)bt->part_lo.size();
     for (int h = 0; h < std::min(cnt, capacity); ++h) first_rows[h] = bt->part_lo[(size_t)h];
     return cnt;
+}
+
+int cap_batch_steps(cap_batch bt, int *matrices)
+{
+    if (!bt || !matrices) return CAP_ERR_ARG;
+    *matrices = bt->plan->batch_steps ? bt->plan->batch_steps->n_jobs : 0;
+    return CAP_OK;
 }
 
 int cap_batch_solve(cap_batch bt, const void *b, void *x, void *stream)

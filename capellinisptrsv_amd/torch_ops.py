@@ -223,6 +223,9 @@ class Batch:
         N.check(N.lib().cap_batch_tuning(h, byref(thr), byref(rpl), byref(npart), byref(tile)), "cap_batch_tuning")
         self.row_threads, self.rhs_per_lane, self.partitioned = thr.value, rpl.value, npart.value
         self.row_tiles = bool(tile.value)
+        steps = c_int()
+        N.check(N.lib().cap_batch_steps(h, byref(steps)), "cap_batch_steps")
+        self.step_matrices = steps.value  # solved by steps, one workgroup each (algo auto)
         rows = (c_int * max(1, npart.value))()
         got = N.lib().cap_batch_partitioned(h, rows, npart.value)
         if got < 0:

@@ -324,6 +324,12 @@ int cap_batch_info(cap_batch batch, int *algo, int *blocks_per_cu);
  * hybrid batch of CAP_ALGO_AUTO: see cap_batch_create). */
 int cap_batch_tuning(cap_batch batch, int *row_threads, int *rhs_per_lane, int *partitioned,
                      int *row_tiles);
+/* No counterpart in the reference: how many of the batch's matrices
+ * CAP_ALGO_AUTO solves by steps (CAP_ALGO_LEVEL's kernel, one workgroup per
+ * matrix and chunk of right-hand sides, bit-exact) instead of the algorithm
+ * cap_batch_info reports; all that are not partitioned, or 0.  Refined
+ * solves do not use them. */
+int cap_batch_steps(cap_batch batch, int *matrices);
 /* No counterpart in the reference: the first rows of the matrices a hybrid
  * batch solves with partitioned plans (up to `capacity` of them); returns
  * how many there are, or a negative CAP_ERR_* code. */

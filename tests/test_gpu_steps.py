@@ -1,0 +1,139 @@
+"""GPU parity of the step solve (steps.hip) where the level rule of explicit
+CAP_ALGO_LEVEL plans does not reach: autotuned plans over matrices whose
+first levels lie all over the rows, rows longer than the 16 entries a step
+carries, any number of right-hand sides, batches, and the division by a
+table reciprocal at the ends of its range.  Bar: the oracle's bits.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from capellinisptrsv_amd import api
+from conftest import random_lower
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(cuda, rp, ci, v, **kw):
+    import torch
+    from capellinisptrsv_amd import Plan
+    return Plan(*(torch.from_numpy(np.ascontiguousarray(a)).to(cuda) for a in (rp, ci, v)), **kw)
+
+
+def _solve(plan, cuda, b):
+    import torch
+    x = plan.solve(torch.from_numpy(np.ascontiguousarray(b)).to(cuda))
+    torch.cuda.synchronize()
+    assert plan.status() == 0
+    return x.cpu().numpy()
+
+
+def _ragged(n=6001, off=16, band=400, seed=3):
+    return api.generate("band_rowcount", n=n, offdiag=off, band=band, seed=seed)
+
+
+@pytest.mark.parametrize("dtype,bits", [(np.float64, np.uint64), (np.float32, np.uint32)])
+@pytest.mark.parametrize("off", [4, 8, 16, 40])
+def test_autotuned_steps_bit_exact(cuda, off, dtype, bits):
+    """4, 8 and 16 carried entries, and rows of up to 39 (the rest read from
+    the overflow table); thread-per-row kernels take about 5 x as long here."""
+    rp, ci, v = _ragged(off=off, seed=off)
+    v = v.astype(dtype)
+    n = len(rp) - 1
+    for arith, fused in (("fused", True), ("reference", False)):
+        plan = _plan(cuda, rp, ci, v, arith=arith)
+        if off != 40:
+            assert plan.info()["algo"] == "level"
+        for k in (1, 2, 3, 16):
+            b = api.uniform(5 + k, n * k).astype(dtype).reshape(n, k) if k > 1 else api.uniform(5, n).astype(dtype)
+            x = _solve(plan, cuda, b)
+            ref = oracle.csr_forward(rp, ci, v, b.reshape(-1), rhs=k, fused=fused)
+            assert np.array_equal(x.reshape(-1).view(bits), ref.view(bits)), (off, arith, k)
+        plan.close()
+
+
+def test_autotuned_steps_read_the_callers_values(cuda):
+    """Where the explicit rule refuses the matrix the autotuned plan used to
+    run kernels that read the caller's values on every solve; its steps do so
+    too."""
+    import torch
+    from capellinisptrsv_amd import Plan
+    rp, ci, v = _ragged(n=20001, seed=21)  # empty rows near the end: beyond that rule's ring
+    d = [torch.from_numpy(a).to(cuda) for a in (rp, ci, v)]
+    plan = Plan(*d)
+    b = api.uniform(6, len(rp) - 1)
+    assert np.array_equal(_solve(plan, cuda, b), oracle.csr_forward(rp, ci, v, b, fused=True))
+    d[2].mul_(0.75)
+    assert np.array_equal(_solve(plan, cuda, b), oracle.csr_forward(rp, ci, v * 0.75, b, fused=True))
+    plan.close()
+
+
+@pytest.mark.parametrize("dtype,bits,span", [(np.float64, np.uint64, 620), (np.float32, np.uint32, 80)])
+def test_step_division_range(cuda, dtype, bits, span):
+    """Diagonals and right-hand sides over powers of two beyond both ends of
+    the reciprocal's range, negative diagonals, zeros of both signs, the
+    smallest numbers: the division's bits; infinities and NaN as the
+    write-first kernel spreads them."""
+    rng = np.random.default_rng(7)
+    rp, ci, v = random_lower(4000, max_off=2, band=60, seed=8)
+    n = len(rp) - 1
+    v = v.astype(dtype)
+    last = rp[1:] - 1
+    off = np.ones(len(v), bool)
+    off[last] = False
+    v[off] = (rng.random(off.sum()) < 0.1) * v[off] * dtype(2.0) ** -3  # mostly independent rows
+    v[last] = (rng.choice([-1, 1], n) * (1 + rng.random(n)) * 2.0 ** rng.integers(-span, span, n)).astype(dtype)
+    b = ((1 + rng.random(n)) * 2.0 ** rng.integers(-span, span, n) * rng.choice([-1, 1], n)).astype(dtype)
+    b[::17] = 0.0
+    b[5::17] = -0.0
+    b[9::17] = np.finfo(dtype).smallest_subnormal
+    plan = _plan(cuda, rp, ci, v, algo="level")
+    with np.errstate(all="ignore"):
+        ref = oracle.csr_forward(rp, ci, v, b, fused=True)
+    x = _solve(plan, cuda, b)
+    ok = np.isfinite(ref)
+    assert ok.sum() > n // 2
+    assert np.array_equal(x[ok].view(bits), ref[ok].view(bits))
+    assert np.array_equal(x, ref, equal_nan=True)
+    b[3], b[500] = np.inf, np.nan
+    plain = _plan(cuda, rp, ci, v, algo="wrtfst")
+    assert np.array_equal(_solve(plan, cuda, b), _solve(plain, cuda, b), equal_nan=True)
+    plan.close()
+    plain.close()
+
+
+def _batch(seed, sizes, off, band):
+    mats = [api.generate("band_rowcount", n=n, offdiag=off, band=band, seed=seed + i) if n else
+            (np.zeros(1, np.int32), np.zeros(0, np.int32), np.zeros(0)) for i, n in enumerate(sizes)]
+    row_off = np.cumsum([0] + [len(m[0]) - 1 for m in mats]).astype(np.int32)
+    nnz_off = np.cumsum([0] + [len(m[1]) for m in mats])
+    rp = np.concatenate([m[0][:-1] + o for m, o in zip(mats, nnz_off)] + [[nnz_off[-1]]]).astype(np.int32)
+    return mats, row_off, rp, np.concatenate([m[1] for m in mats]).astype(np.int32), np.concatenate([m[2] for m in mats])
+
+
+@pytest.mark.parametrize("dtype,arith", [(np.float64, "fused"), (np.float32, "fused"), (np.float64, "reference")])
+@pytest.mark.parametrize("k", [1, 3, 4, 16])
+def test_batch_steps_bit_exact(cuda, k, dtype, arith):
+    """Matrices from empty to 9,000 rows (fewer and more than the eight of a
+    group), solved twice, and captured into a graph."""
+    import torch
+    from capellinisptrsv_amd import Batch
+    from test_gpu_capture import _replays
+    for sizes in ((9000, 0, 700, 1), tuple(2000 + 37 * i for i in range(19))):
+        mats, row_off, rp, ci, v = _batch(50 + k, sizes, 16, 300)
+        v = v.astype(dtype)
+        N = int(row_off[-1])
+        b = api.uniform(9 + k, N * k).astype(dtype)
+        bt = Batch(*(torch.from_numpy(a).to(cuda) for a in (row_off, rp, ci, v)), k=k, arith=arith)
+        assert bt.step_matrices == sum(n > 0 for n in sizes) and bt.partitioned == 0
+        bd = torch.from_numpy(b.reshape(N, k)).to(cuda)
+        x = bt.solve(bd)
+        flat = x.cpu().numpy().reshape(-1)
+        for m, (mrp, mci, mv) in enumerate(mats):
+            lo, hi = row_off[m] * k, row_off[m + 1] * k
+            if hi > lo:
+                ref = oracle.csr_forward(mrp, mci, mv.astype(dtype), b[lo:hi], rhs=k, fused=arith == "fused")
+                assert np.array_equal(flat[lo:hi], ref), m
+        out = torch.empty_like(bd)
+        _replays(lambda: bt.solve(bd, out=out, stream=torch.cuda.current_stream()), out, x)
+        bt.close()
