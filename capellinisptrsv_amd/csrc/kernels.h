@@ -1810,96 +1810,31 @@ __global__ void __launch_bounds__(kBlock)
 // For deep matrices whose lower bandwidth w = max(i - col) is at most the
 // tail width W (the dependency chain is ~n/levels rows long and no row order
 // can shorten it).  Rows are cut into P blocks of m >= W rows; block p's
-// rows only reach back into the last W rows of block p-1.  With D the
-// block-diagonal part of L, y = D^{-1} b (independent blocks) and V_p =
-// D_pp^{-1} C_p (C_p: block p's entries in the coupling columns [pm - W,
-// pm)), the exact solution is x_p = y_p - V_p t_{p-1} with t_p the last W
-// values of x_p:
-//   t_p = a_p + B_p t_{p-1},   a_p = tail(y_p),   B_p = -tail(V_p).
-// The recurrence over the Q = P - 1 tails is scanned in two levels: in
-// groups of gs consecutive tails sequentially (u_p from the group's first
-// tail on), then over the group carries T_g in ceil(log2 G) rounds, then
-// every tail is fixed up with its in-group product W_p = B_p ... B_first:
-// t_p = u_p + W_p T_{g-1}.  The matrix products are formed once per plan
-// (k_part_gemm); a solve only touches vectors.  The sums are reassociated,
-// so results match the sequential solve to rounding, not bit for bit.
-// The tail width W (the number of coupling columns, 128 or 256) is the
-// smallest of those at least the matrix's lower bandwidth; blocks hold at
-// least W rows.  Matrices are column-major W x W (element (c, k) at k * W +
-// c); V comes from W / 64 batch solves of 64 interleaved columns (n x 64
-// each, one after another).  The tables and the solve's work vectors are
-// FP64 for FP32 plans too: b is widened when the block kernel reads it and x
-// rounded once when the finish writes it.
+// rows only reach back into the last W rows of block p-1, its history.  A
+// solve sweeps all blocks at once, twice: first with the history 0, for the
+// block's last W values a_p, and then, with the blocks' true tails t_p at
+// hand, from t_{p-1}, for x.  In between the tails are joined,
+//   t_p = a_p + B_p t_{p-1},
+// with column c of B_p the tail that block p has for b = 0 and the unit
+// vector e_c as its history (W sweeps, once per plan).
+// The second sweep reads the rows again instead of adding V_p t_{p-1} with a
+// stored V_p (n x W): 4.2 KB per 8 rows at 38 entries against 8 KB, and V
+// takes no memory (half a gigabyte at n = 500,000).
+// The join is a walk (k_part_walk) where the plan finds that a block damps
+// its history, else a scan of the recurrence over the Q = P - 1 tails in two
+// levels: in groups of gs consecutive tails sequentially (u_p from the
+// group's first tail on), then over the group carries T_g in ceil(log2 G)
+// rounds, then every tail is fixed up with its in-group product W_p = B_p
+// ... B_first: t_p = u_p + W_p T_{g-1}.  The matrix products are formed once
+// per plan (k_part_gemm); a solve only touches vectors.  The sums are
+// reassociated, so results match the sequential solve to rounding, not bit
+// for bit.  The tail width W (128 or 256) is the smallest of those at least
+// the matrix's lower bandwidth; blocks hold at least W rows.  Matrices are
+// column-major W x W (element (c, k) at k * W + c).  The tables and the
+// solve's work vectors are FP64 for FP32 plans too: b is widened when a sweep
+// reads it and x rounded once when it is written.
 constexpr int kPartW = 128;     // the narrower tail width
 constexpr int kPartWMax = 256;  // the wider one
-
-// Coupling right-hand sides (W / 64 zeroed slabs of 64 interleaved columns,
-// slab h at r + h * n * 64): an entry of row i in block p >= 1 whose column c
-// lies before the block goes to column q = c - (pm - W); duplicated entries
-// add up.
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-    k_part_coupling(const int *__restrict__ rp, const int *__restrict__ ci, const T *__restrict__ val, int n, int m,
-                    int W, double *__restrict__ r)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int start = (i / m) * m;
-    if (start == 0) return;
-    const int base = start - W;
-    for (int j = rp[i]; j < rp[i + 1]; ++j) {
-        const int c = ci[j];
-        const int q = c - base;
-        if (c >= start || q < 0) continue;  // inside the block; q < 0 cannot occur (bandwidth checked on the host)
-        r[(long long)(q >> 6) * n * 64 + (long long)i * 64 + (q & 63)] += (double)val[j];
-    }
-}
-
-// V from the 64-column slabs the batch solves write (row-major, 64 per row)
-// to column-major vt (column k at k * n): the finish then reads consecutive
-// rows per column.
-__global__ void __launch_bounds__(kBlock)
-    k_part_transpose(const double *__restrict__ v, int n, int W, double *__restrict__ vt)
-{
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long long)n * W) return;
-    const int k = (int)(g / n), i = (int)(g % n);
-    vt[g] = v[(long long)(k >> 6) * n * 64 + (long long)i * 64 + (k & 63)];
-}
-
-// B_p = -(the last W rows of V_p) for p in [1, q_count), stored at index
-// p - 1 (the first round's matrices).
-__global__ void __launch_bounds__(kBlock)
-    k_part_tail_matrix(const double *__restrict__ vt, int n, int m, int q_count, int W, double *__restrict__ b0)
-{
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long long)(q_count - 1) * W * W) return;
-    const int c = (int)(g % W);
-    const int k = (int)((g / W) % W);
-    const int p = 1 + (int)(g / ((long long)W * W));
-    const long long row = (long long)(p + 1) * m - W + c;
-    b0[g] = -vt[(long long)k * n + row];
-}
-
-// y = D^{-1} b: one wavefront per block, rows in order.  A row's in-block
-// entries in columns i-1 and i-2 are kept apart (near: their values, summed
-// per column); the others (columns <= i-3) are stored ELL-style, ew <=
-// kPartEll per row (value, and the byte offset of the column's slot in the
-// LDS ring of the block's values: ((col - block start) mod 2W) * 8; pads
-// point at slot 2W, which holds 0), the rest of a longer row in
-// an overflow CSR (ov_rp per row, absolute columns).  Entry l of a row sits
-// in lane l; its products with the block's earlier values are summed through
-// LDS (8 lanes add 8 products each, then an 8-lane butterfly), and
-//   y_i = ((b_i - S_i - w2_i y_{i-2}) - w1_i y_{i-1}) / d_i
-// (as a multiplication by the reciprocal diagonal).  S_i needs only values
-// up to y_{i-3}, so it is summed two rows ahead, off the chain from one row
-// to the next.  Row data are loaded a group of kPartPre rows ahead.  The sum
-// is reassociated and the division is a multiplication (tolerance, not
-// bit-exact), like the whole partitioned solve.
-constexpr int kPartEll = 64;
-constexpr int kPartPre = 16;
-// ring slots of a tail width W (rows' values by row mod 2W)
-constexpr int part_ring(int W) { return 2 * W; }
 
 // A double moved between lanes by DPP (the GFX9 DPP set).  Lanes whose
 // source lies outside their row read 0 (bound_ctrl); lanes in rows outside
@@ -1914,16 +1849,46 @@ __device__ __forceinline__ double dpp_d(double v)
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// The sum of v over each group of 8 lanes, in all 8 of them: butterflies by
+// Each v[q] summed over groups of 8 lanes, in all 8 of them: butterflies by
 // quad_perm [1,0,3,2], quad_perm [2,3,0,1] and row_half_mirror (lane i and
 // 7 - i of each half row).  Each lane adds the same two halves, in either
-// order, so all 8 hold the same bits.
-__device__ __forceinline__ double part_sum8(double v)
+// order, so all 8 hold the same bits.  (Step by step for all q: one after
+// another their chains do not overlap.)
+template <int K>
+__device__ __forceinline__ void part_sum8(double (&v)[K])
 {
-    v += dpp_d<0xB1, 0xf>(v);
-    v += dpp_d<0x4E, 0xf>(v);
-    v += dpp_d<0x141, 0xf>(v);
-    return v;
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] += dpp_d<0xB1, 0xf>(v[q]);
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] += dpp_d<0x4E, 0xf>(v[q]);
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] += dpp_d<0x141, 0xf>(v[q]);
+}
+
+// v plus the other of its pair of rows of 16 lanes (or of halves of 32)
+template <bool HALVES>
+__device__ __forceinline__ double part_swap_add(double v)
+{
+    const unsigned long long u = as_bits(v);
+    const unsigned l = (unsigned)u, h = (unsigned)(u >> 32);
+    const auto lo = HALVES ? __builtin_amdgcn_permlane32_swap(l, l, false, false)
+                           : __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    const auto hi = HALVES ? __builtin_amdgcn_permlane32_swap(h, h, false, false)
+                           : __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    return as_val((unsigned long long)hi[0] << 32 | lo[0]) + as_val((unsigned long long)hi[1] << 32 | lo[1]);
+}
+
+// Each v[q] summed over the 8 lanes with the same lane mod 8, in all of them:
+// row_ror:8, then the rows of 16 lanes and the halves of 32 swapped.
+template <int K>
+__device__ __forceinline__ void part_sum_across(double (&v)[K])
+{
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] += dpp_d<0x128, 0xf>(v[q]);
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] = part_swap_add<false>(v[q]);
+#pragma unroll
+    for (int q = 0; q < K; ++q) v[q] = part_swap_add<true>(v[q]);
 }
 
 // v of lane `src` (0..63, may differ per lane; every lane active), through
@@ -1935,212 +1900,289 @@ __device__ __forceinline__ double lane_read(double v, int src)
     const int hi = __builtin_amdgcn_ds_bpermute(src * 4, (int)(u >> 32));
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
-
-
-template <int W, int KR, typename T>
-__global__ void __launch_bounds__(kWave)
-    k_part_block(const int *__restrict__ ell_c, const double *__restrict__ ell_v, const int *__restrict__ ov_rp,
-                 const int *__restrict__ ov_c, const double *__restrict__ ov_v, const double *__restrict__ inv_diag,
-                 const double2 *__restrict__ near, const T *__restrict__ b, double *__restrict__ y,
-                 double *__restrict__ tails, int n, int m, int ew, int k, int q_count)
+__device__ __forceinline__ float lane_read(float v, int src)
 {
-    constexpr int kRing = part_ring(W);
-    constexpr int kRow = KR + 3;  // a row's scalars in LDS: b per RHS, 1 / diagonal, near (i-1), near (i-2)
-    __shared__ double ring[KR][kRing + 1];
-    __shared__ double rowd[kPartPre][kRow];
-    __shared__ double red[2 * KR][kWave];  // a row pair's lane products, transposed for the sums
-    const int lane = threadIdx.x;
-    // right-hand sides q0 .. q0 + KR - 1 (b and y interleaved, k per row)
-    const long long q0 = (long long)blockIdx.y * KR;
-    const int start = blockIdx.x * m;
-    const int end = min(n, start + m);
-    if (lane < KR) ring[lane][kRing] = 0.0;  // the pads' slot
-    // a group's row data: entry `lane` of each of its kPartPre rows, and, in
-    // lane r, row r's b values, reciprocal diagonal, near values and
-    // overflow start (lane kPartPre: the end).  Lanes with nothing to load
-    // are masked off (loading a clamped entry instead was slower).
-    int nc[kPartPre];
-    double nv[kPartPre], nb[KR], nd = 1.0, nw1 = 0.0, nw2 = 0.0;
-    int no = 0;
-    auto fetch = [&](int g0) {
-        if (g0 + kPartPre <= end) {  // uniform: a whole group, one lane mask for all its loads
-            if (lane < ew) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(src * 4, __float_as_int(v)));
+}
+
+// A record holds up to 8 consecutive rows of one block for one step of a
+// wavefront.  Its 64 lanes are 8 segments of 8; a segment takes up to 8 J
+// entries of one row in columns before the record's first row r0 (entry e in
+// lane e mod 8), so a longer row has several.  The entries inside the record
+// are in M, the inverse of the rows' 8 x 8 triangle, a column per segment:
+//   y_j = sum over segments u of M[j][u] (b_u - S_u),
+// S_u the segment's sum of value * earlier value, b_u its row's b (0 in a
+// row's further segments).  In lane 8 u + j: M[j][u], the lane's J values, r0
+// - 1 - column per entry in a byte (columns reach back at most W <= 256 rows),
+// and 16 bits: the segment's row in the record, flags for a further segment
+// and for a segment without entries, the record's row count, and how many
+// rows on the record kPartAhead records later starts (the sweep loads that
+// far ahead).  Unused entries repeat a column of their row with the value 0:
+// they read no value that the row does not depend on.
+// NP = J / 2 + 1 pieces of 16 bytes per lane; piece i of record r at
+// (r * NP + i) * 64 + lane.
+constexpr int kPartSeg = 8;      // segments, and rows at most, of a record
+constexpr int kPartAhead = 6;    // records loaded ahead
+constexpr int kPartMaxJ = 6;     // J is 2, 4 or 6
+constexpr int kPartWaves = 4;    // wavefronts of a sweep's workgroup, at most
+constexpr unsigned kPartFurther = 8u, kPartEmpty = 16u;
+constexpr int part_pieces(int J) { return J / 2 + 1; }
+
+// The records of a plan, one wavefront each.  rows[r]: record r's first row
+// (one entry more than records); at[p]: block p's first record.
+template <int J, typename T>
+__global__ void __launch_bounds__(kWave)
+    k_part_records(const int *__restrict__ rp, const int *__restrict__ ci, const T *__restrict__ val,
+                   const int *__restrict__ rows, const int *__restrict__ at, int m, uint4 *__restrict__ rec)
+{
+    constexpr int S = kPartSeg;
+    __shared__ double tri[S][S], inv[S][S], vals[kWave][J];
+    __shared__ unsigned dist[kWave][J];
+    __shared__ int out[S], seg0[S + 1];
+    const int r = (int)blockIdx.x, lane = (int)threadIdx.x, u = lane / S, j = lane % S;
+    const int r0 = rows[r], count = rows[r + 1] - r0;
+    tri[u][j] = inv[u][j] = 0.0;
 #pragma unroll
-                for (int r = 0; r < kPartPre; ++r) {
-                    const long long e = (long long)(g0 + r) * ew + lane;
-                    nc[r] = ell_c[e];
-                    nv[r] = ell_v[e];
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < kPartPre; ++r) {
-                    nc[r] = kRing * 8;
-                    nv[r] = 0.0;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < kPartPre; ++r) {
-                const long long e = (long long)(g0 + r) * ew + lane;
-                const bool in = g0 + r < end && lane < ew;
-                nc[r] = in ? ell_c[e] : kRing * 8;
-                nv[r] = in ? ell_v[e] : 0.0;
-            }
+    for (int s = 0; s < J; ++s) vals[lane][s] = 0.0;
+    __syncthreads();
+    if (lane < count) {
+        int n_out = 0;
+        for (int e = rp[r0 + lane]; e < rp[r0 + lane + 1]; ++e) {
+            if (ci[e] < r0)
+                ++n_out;
+            else
+                tri[lane][ci[e] - r0] += (double)val[e];  // duplicated entries add up
         }
-        const int row = min(g0 + lane, end);
-        const bool mine = lane < kPartPre && row < end;
-#pragma unroll
-        for (int j = 0; j < KR; ++j) nb[j] = mine ? (double)b[(long long)row * k + q0 + j] : 0.0;
-        nd = mine ? inv_diag[row] : 1.0;
-        const double2 w = mine ? near[row] : make_double2(0.0, 0.0);
-        nw1 = w.x;
-        nw2 = w.y;
-        no = lane <= kPartPre ? ov_rp[row] : 0;
-    };
-    // The values go to y from the ring, a group at a time (one store of
-    // kPartPre x KR values at the next group's top): a store per row would
-    // make the waits for the prefetch (the memory counter covers stores too)
-    // wait for it.
-    static_assert(kPartPre * KR <= kWave, "a group's values are stored by one instruction");
-    const int wr = lane / KR, wj = lane % KR;  // the (row, RHS) this lane stores
-    auto store_group = [&](int s0) {
-        const int i = s0 + wr;
-        if (lane < kPartPre * KR && i < end) y[(long long)i * k + q0 + wj] = ring[wj][(i - start) & (kRing - 1)];
-    };
-    // Each lane carries the chain of one right-hand side, wj = lane mod KR:
-    // y_{i-1}, y_{i-2} of that RHS (0 before the block's first row, where the
-    // near values are 0 too).  Every lane still forms the products of its
-    // ELL entry for all KR right-hand sides (the sums need them).
-    double y1 = 0.0, y2 = 0.0;
-    fetch(start);
-    for (int g0 = start; g0 < end; g0 += kPartPre) {
-        int cc[kPartPre];
-        double cv[kPartPre];
-#pragma unroll
-        for (int r = 0; r < kPartPre; ++r) {
-            cc[r] = nc[r];
-            cv[r] = nv[r];
-        }
-        // the group's row scalars, read back as broadcasts row by row
-        if (lane < kPartPre) {
-#pragma unroll
-            for (int j = 0; j < KR; ++j) rowd[lane][j] = nb[j];
-            rowd[lane][KR] = nd;
-            rowd[lane][KR + 1] = nw1;
-            rowd[lane][KR + 2] = nw2;
-        }
-        const int og = no;
-        // FAST: a whole group with no overflow entries (no branch between
-        // its rows, so their sums and chains can interleave)
-        const bool fast = g0 + kPartPre <= end &&
-                          __builtin_amdgcn_readlane(og, 0) == __builtin_amdgcn_readlane(og, kPartPre);
-        auto group = [&](auto fast_tag) {
-            constexpr bool FAST = decltype(fast_tag)::value;
-            // ring values of row r's ELL entries (all in columns the ring
-            // holds; pads read the zero slot)
-            auto ring_vals = [&](int r, double (&rv)[KR]) {
-#pragma unroll
-                for (int j = 0; j < KR; ++j) rv[j] = *(const double *)((const char *)ring[j] + cc[r]);
-            };
-            // the lane products of row r's S, from its ring values (plus its
-            // overflow entries), into prod[0 .. KR)
-            auto row_prod = [&](int r, const double (&rv)[KR], double *prod) {
-#pragma unroll
-                for (int j = 0; j < KR; ++j) prod[j] = cv[r] * rv[j];
-                if constexpr (!FAST) {
-                    const int o0 = __builtin_amdgcn_readlane(og, r), o1 = __builtin_amdgcn_readlane(og, r + 1);
-                    for (int e = o0 + lane; e < o1; e += kWave) {  // rows longer than kPartEll
-                        const int c = ov_c[e];
-                        const double w = ov_v[e];
-#pragma unroll
-                        for (int j = 0; j < KR; ++j)
-                            prod[j] = __builtin_fma(w, ring[j][(c - start) & (kRing - 1)], prod[j]);
-                    }
-                }
-            };
-            // S of rows r and r + 1 (all their right-hand sides): the 2 KR
-            // sums of 64 lane products go through LDS, 8 lanes per sum add 8
-            // products each (a fixed tree), and three butterfly steps join
-            // the 8 lanes (part_sum8).  Every sum is formed the same way
-            // whatever KR, so each right-hand side keeps its one-RHS bits.
-            auto pair_sums = [&](int r, const double (&rva)[KR], const double (&rvb)[KR], double &sa, double &sb) {
-                constexpr int N = 2 * KR;
-                double prod[N];
-                row_prod(r, rva, prod);
-                row_prod(r + 1, rvb, prod + KR);
-#pragma unroll
-                for (int u = 0; u < N; ++u) red[u][lane] = prod[u];
-                const double *src = &red[min(lane >> 3, N - 1)][(lane & 7) * 8];  // lanes past 8 N: unused
-                double a[8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) a[t] = src[t];
-                const double v = part_sum8(((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])));
-                // sum u sits in lanes 8u .. 8u + 7: this lane's RHS's two
-                if constexpr (KR == 1) {
-                    sa = bcast(v, 0);
-                    sb = bcast(v, 8);
-                } else {
-                    sa = lane_read(v, 8 * wj);
-                    sb = lane_read(v, 8 * (KR + wj));
-                }
-            };
-            // the sums of the group's first two rows (columns below g0 - 1)
-            double s0, s1, rv0[KR], rv1[KR];
-            ring_vals(0, rv0);
-            ring_vals(1, rv1);
-            if (g0 + kPartPre < end) fetch(g0 + kPartPre);
-            if (g0 > start) store_group(g0 - kPartPre);
-            pair_sums(0, rv0, rv1, s0, s1);
-            // y of row r from its sum s
-            // y of row r for this lane's RHS from its sum s
-            auto finish_row = [&](int r, double s) {
-                const int i = g0 + r;
-                const double di = rowd[r][KR], w1 = rowd[r][KR + 1], w2 = rowd[r][KR + 2];
-                double t = rowd[r][wj] - s;
-                t = __builtin_fma(-w2, y2, t);
-                t = __builtin_fma(-w1, y1, t);
-                const double yi = t * di;
-                y2 = y1;
-                y1 = yi;
-                // every lane writes (the lanes of one RHS the same value to
-                // the same slot), so no lane mask splits the rows' code
-                ring[wj][(i - start) & (kRing - 1)] = yi;
-            };
-            // Rows in pairs: row r + 2's ring values (columns <= i - 1) are
-            // read before y_i is written, row r + 3's (columns <= i) before
-            // y_{i+1}; then both sums run, two independent DPP chains.
-            static_assert(kPartPre % 2 == 0, "rows go in pairs");
-#pragma unroll
-            for (int r = 0; r < kPartPre; r += 2) {
-                if constexpr (!FAST) {
-                    if (g0 + r >= end) continue;  // uniform: the block's last group
-                }
-                double rv2[KR], rv3[KR];
-                if (r + 2 < kPartPre) ring_vals(r + 2, rv2);
-                finish_row(r, s0);
-                if constexpr (!FAST) {
-                    if (g0 + r + 1 >= end) continue;
-                }
-                if (r + 2 < kPartPre) ring_vals(r + 3, rv3);
-                finish_row(r + 1, s1);
-                if (r + 2 < kPartPre) pair_sums(r + 2, rv2, rv3, s0, s1);
-            }
-        };
-        if (fast)
-            group(std::true_type{});
-        else
-            group(std::false_type{});
+        out[lane] = n_out;
     }
-    store_group(start + (end - 1 - start) / kPartPre * kPartPre);  // the last group
-    // a_p = the block's last W values, the tail scan's input (blocks p <
-    // q_count, which are whole: m >= W rows), at (p * k + q) * W + c, from
-    // the ring
-    if ((int)blockIdx.x < q_count) {
+    __syncthreads();
+    if (lane == 0) {
+        int s = 0;
+        for (int i = 0; i < count; ++i) {
+            seg0[i] = s;
+            s += max(1, (out[i] + S * J - 1) / (S * J));
+        }
+        seg0[count] = s;
+    }
+    if (lane < count) {  // column `lane` of the inverse
+        for (int i = lane; i < count; ++i) {
+            double s = i == lane ? 1.0 : 0.0;
+            for (int l = lane; l < i; ++l) s = __builtin_fma(-tri[i][l], inv[l][lane], s);
+            inv[i][lane] = s / tri[i][i];
+        }
+    }
+    __syncthreads();
+    int row = -1;
+    for (int i = 0; i < count; ++i)
+        if (u >= seg0[i] && u < seg0[i + 1]) row = i;
+    unsigned flags = kPartFurther | kPartEmpty, pad = 0;
+    if (row >= 0) {
+        const int h = u - seg0[row];
+        flags = (unsigned)row | (h > 0 ? kPartFurther : 0u) | (out[row] == 0 ? kPartEmpty : 0u);
+        int idx = 0;
+        for (int e = rp[r0 + row]; e < rp[r0 + row + 1]; ++e) {
+            if (ci[e] >= r0) continue;
+            if (idx == 0) pad = (unsigned)(r0 - 1 - ci[e]);
+            if (idx / (S * J) == h && idx % S == j) {
+                vals[lane][idx / S % J] = (double)val[e];
+                dist[lane][idx / S % J] = (unsigned)(r0 - 1 - ci[e]) + 1u;
+            }
+            ++idx;
+        }
+        // the slots past the segment's last entry
+        for (int s = 0; s < J; ++s)
+            if ((h * J + s) * S + j >= idx) dist[lane][s] = pad + 1u;
+    } else {
+        for (int s = 0; s < J; ++s) dist[lane][s] = 1u;
+    }
+    const int last = at[r0 / m + 1];
+    const unsigned ahead = r + kPartAhead < last ? (unsigned)(rows[r + kPartAhead] - r0) : 0u;
+    flags |= (unsigned)count << 5 | ahead << 9;
+    uint4 *o = rec + (long long)r * part_pieces(J) * kWave + lane;
+#pragma unroll
+    for (int s = 0; s < J; s += 2) {
+        const unsigned long long a = as_bits(vals[lane][s]), b = as_bits(vals[lane][s + 1]);
+        o[s / 2 * kWave] = make_uint4((unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32));
+    }
+    unsigned w[2] = {0u, flags << 16};
+#pragma unroll
+    for (int s = 0; s < J; ++s) w[s / 4] |= (dist[lane][s] - 1u) << (8 * (s % 4));
+    const unsigned long long mm = as_bits(row >= 0 ? inv[j][row] : 0.0);
+    o[J / 2 * kWave] = make_uint4((unsigned)mm, (unsigned)(mm >> 32), w[0], w[1]);
+}
+
+// What a sweep is for: the tails a_p of history 0 (and the largest magnitude
+// in each, the bits of a NaN above all), the B_p (right-hand side q's history
+// is e_q and b is 0), or x from the tails t.
+enum PartSweep { kPartTails, kPartUnit, kPartX };
+
+// One wavefront per block and KR right-hand sides (b and x interleaved, k per
+// row), a record per step; a workgroup's wavefronts have right-hand sides of
+// one block, so that the others find in L1 the records that one has loaded.  The block's latest values are in an LDS ring of
+// 2W slots, KR values each.  A step's chain is: the ring's values read (J per
+// lane), their sum over the segment's 8 lanes, b - S times M, the sum over
+// the 8 segments, the ring's slots written: 0.2 us for 8 rows (0.33 and 0.5
+// with 2 and 4 right-hand sides per wavefront), where a row at a time took
+// 0.2 us a row.  So the rows' bytes bound it, with records loaded kPartAhead
+// steps early: 42 and 46 us for the 250 MB of n = 500,000 at 38 entries a row
+// (97 us for a row at a time in 384 MB of padded rows, and 92 for V's 512 MB).
+// Products with a zero of M are left out: a row's infinity or NaN reaches
+// only the rows that depend on it.
+// Every right-hand side gets the same bits whatever KR.
+template <int W, int KR, int J, typename T, PartSweep MODE>
+__global__ void __launch_bounds__(kPartWaves * kWave)
+    k_part_sweep(const uint4 *__restrict__ rec, const int *__restrict__ at, const uint2 *__restrict__ first,
+                 const T *b, const double *__restrict__ hist, double *__restrict__ tails,
+                 unsigned long long *__restrict__ top, T *x, int n, int m, int k, int blocks)
+{
+    constexpr int D = kPartAhead, NP = part_pieces(J), kMask = 2 * W - 1, kRec = NP * kWave * 16;
+    const int p = (int)blockIdx.x + (MODE == kPartUnit ? 1 : 0);
+    if ((int)blockIdx.x >= blocks) return;
+    __shared__ double rings[kPartWaves][2 * W + 1][KR];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    double (&ring)[2 * W + 1][KR] = rings[wave];  // the last slot: 0
+    const int lane = (int)threadIdx.x % kWave, j = lane & 7;
+    const int q0 = ((int)blockIdx.y * ((int)blockDim.x / kWave) + wave) * KR;
+    const int start = p * m, rows = min(n - start, m);
+    const int r_at = at[p], n_rec = at[p + 1] - r_at;
+#pragma unroll
+    for (int c = lane; c < W; c += kWave) {
+#pragma unroll
+        for (int q = 0; q < KR; ++q) {
+            double v = 0.0;
+            if (MODE == kPartUnit) v = c == q0 + q ? 1.0 : 0.0;
+            if (MODE == kPartX && p > 0) v = hist[((long long)(p - 1) * k + q0 + q) * W + c];
+            ring[c][q] = 0.0;
+            ring[W + c][q] = v;
+        }
+    }
+    if (lane < KR) ring[2 * W][lane] = 0.0;
+    const unsigned row_bytes = (unsigned)(k * sizeof(T)), lane16 = 16u * (unsigned)lane;
+    const unsigned span = (unsigned)rows * row_bytes - (unsigned)(q0 * sizeof(T));
+    const Rsrc rt = make_rsrc(rec + (long long)r_at * NP * kWave, (unsigned)n_rec * kRec);
+    // records past the block's last read as 0: no rows, and nothing is stored
+    const long long at_b = uniform((long long)start * k + q0);
+    const Rsrc rb = make_rsrc(b + at_b, span), rx = make_rsrc(x + at_b, span);
+    Words4 st[D][NP];
+    T bs[D][KR];
+    auto fetch = [&](int d, int at_rec, unsigned row) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+            st[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rt, (int)(lane16 + (unsigned)(at_rec * kRec + i * kWave * 16)),
+                                                             0, 0);
+        if (MODE != kPartUnit) {
+#pragma unroll
+            for (int q = 0; q < KR; ++q)
+                load_value(rb, (row + (unsigned)j) * row_bytes, (unsigned)(q * sizeof(T)), &bs[d][q]);
+        }
+    };
+    {
+        const uint2 f = first[p];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            fetch(d, d, ((d < 4 ? f.x : f.y) >> (8 * (d % 4))) & 255u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // What the chain needs of a record, worked out during the record before:
+    // the ring slots its entries read (a segment without entries reads the
+    // zero slot), the segment's b, M, whether M is 0, the slot it writes, its
+    // place in x and its rows.
+    struct Stage {
+        int slot[J], own, count;
+        unsigned ahead, at_x;
+        double mm, bu[KR];
+        bool none;
+    };
+    auto decode = [&](int d, int lr) {
+        Stage w;
+        const Words4 head = st[d][NP - 1];
+        const unsigned flags = head.w >> 16;
+        const unsigned uni = (unsigned)__builtin_amdgcn_readfirstlane((int)flags);
+        w.count = (int)(uni >> 5 & 15u);
+        w.ahead = uni >> 9;
+#pragma unroll
+        for (int s = 0; s < J; ++s) {
+            const int back = (int)((s < 4 ? head.z : head.w) >> (8 * (s % 4)) & 255u);
+            w.slot[s] = (flags & kPartEmpty) ? 2 * W : (lr - 1 - back) & kMask;
+        }
+        w.own = (lr + j) & kMask;
+        w.at_x = lane < w.count ? (unsigned)(lr + j) * row_bytes : 0x80000000u;  // else dropped
+        w.mm = as_val((unsigned long long)head.y << 32 | head.x);
+        w.none = w.mm == 0.0;
+#pragma unroll
+        for (int q = 0; q < KR; ++q) {
+            w.bu[q] = 0.0;
+            if (MODE != kPartUnit) {
+                const double t = (double)lane_read(bs[d][q], (int)(flags & 7u));
+                w.bu[q] = (flags & kPartFurther) ? 0.0 : t;
+            }
+        }
+        return w;
+    };
+    int lr = 0;  // the record's first row in the block
+    Stage now = decode(0, 0);
+    for (int r0 = 0; r0 < n_rec; r0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            double sum[KR][2];
+#pragma unroll
+            for (int q = 0; q < KR; ++q) sum[q][0] = sum[q][1] = 0.0;
+#pragma unroll
+            for (int s = 0; s < J; ++s) {
+                const Words4 w = st[d][s / 2];
+                const double v = s & 1 ? as_val((unsigned long long)w.w << 32 | w.z)
+                                       : as_val((unsigned long long)w.y << 32 | w.x);
+#pragma unroll
+                for (int q = 0; q < KR; ++q) sum[q][s & 1] = __builtin_fma(v, ring[now.slot[s]][q], sum[q][s & 1]);
+            }
+            const unsigned ahead = (unsigned)lr + now.ahead;
+            lr += now.count;
+            const Stage next = decode((d + 1) % D, lr);
+            double y[KR];
+#pragma unroll
+            for (int q = 0; q < KR; ++q) y[q] = sum[q][0] + sum[q][1];
+            part_sum8(y);
+#pragma unroll
+            for (int q = 0; q < KR; ++q) y[q] = now.none ? 0.0 : now.mm * (now.bu[q] - y[q]);
+            part_sum_across(y);
+            // every lane writes (those of a row the same value): the slots of
+            // the rows past the record's are the next record's
+#pragma unroll
+            for (int q = 0; q < KR; ++q) ring[now.own][q] = y[q];
+            if (MODE == kPartX) {
+#pragma unroll
+                for (int q = 0; q < KR; ++q) store_value(rx, now.at_x, (unsigned)(q * sizeof(T)), (T)y[q]);
+            }
+            now = next;
+            // the loads neither before M's last use (they take its registers)
+            // nor later than here
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(d, r0 + d + D, ahead);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (MODE != kPartX) {  // the block's last W values: blocks of m >= W rows
+        const long long out = MODE == kPartUnit ? p - 1 : p;
+        unsigned long long big[KR];
+#pragma unroll
+        for (int q = 0; q < KR; ++q) big[q] = 0;
 #pragma unroll
         for (int c = lane; c < W; c += kWave) {
-            const int slot = (end - W + c - start) & (kRing - 1);
 #pragma unroll
-            for (int j = 0; j < KR; ++j) tails[((long long)blockIdx.x * k + q0 + j) * W + c] = ring[j][slot];
+            for (int q = 0; q < KR; ++q) {
+                const double v = ring[(m - W + c) & kMask][q];
+                tails[(out * k + q0 + q) * W + c] = v;
+                big[q] = max(big[q], as_bits(v) & ~(1ull << 63));
+            }
+        }
+        if (MODE == kPartTails) {
+#pragma unroll
+            for (int q = 0; q < KR; ++q) {
+#pragma unroll
+                for (int s = 1; s < kWave; s *= 2) big[q] = max(big[q], (unsigned long long)__shfl_xor((long long)big[q], s));
+                if (lane == 0) top[out * k + q0 + q] = big[q];
+            }
         }
     }
 }
@@ -2390,84 +2432,172 @@ __global__ void __launch_bounds__(W)
     }
 }
 
-// x = y - V t_{p-1} in blocks p >= 1 (t: the scan's result), x = y in
-// block 0.  One thread per (row, RHS), g = row * k + q: V column-major, so
-// for each column the lanes read consecutive rows (the k lanes of one row
-// share an element).
-template <int W, typename T>
-__global__ void __launch_bounds__(kBlock)
-    k_part_finish(const double *__restrict__ y, const double *__restrict__ vt, const double *__restrict__ t, int n,
-                  int m, int k, T *__restrict__ x)
+// The largest absolute row sum of each B_p (p = 1 + blockIdx.x), rounded up.
+template <int W>
+__global__ void __launch_bounds__(W) k_part_norm(const double *__restrict__ bm, double *__restrict__ norm)
 {
-    const long long gi = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= (long long)n * k) return;
-    const int i = k == 1 ? (int)gi : (int)(gi / k), q = k == 1 ? 0 : (int)(gi % k);
-    const int p = i / m;
-    double xi = y[gi];
-    if (p > 0) {
-        const double *tp = t + ((long long)(p - 1) * k + q) * W;
-        double s[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 8
-        for (int c = 0; c < W; c += 4)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                s[u] = __builtin_fma(__builtin_nontemporal_load(vt + (long long)(c + u) * n + i), tp[c + u], s[u]);
-        xi -= (s[0] + s[1]) + (s[2] + s[3]);
+    __shared__ double red[W];
+    const int c = (int)threadIdx.x;
+    const double *M = bm + (long long)blockIdx.x * W * W;
+    double s = 0.0;
+    for (int kk = 0; kk < W; ++kk) s += fabs(M[(long long)kk * W + c]);
+    red[c] = s;
+    __syncthreads();
+    if (c == 0) {
+        for (int i = 1; i < W; ++i) s = red[i] <= s ? s : red[i];  // a NaN stays or replaces the rest
+        norm[blockIdx.x] = s * (1.0 + 1e-9);
     }
-    x[gi] = (T)xi;
 }
 
-// The finish for chunks of KQ >= 2 right-hand sides: a workgroup takes
-// W consecutive rows (at most two blocks, as m >= W) and RHS
-// blockIdx.y * KQ + j.  It stages both blocks' t_{p-1} in LDS (RHS fastest,
-// read as broadcasts), and each thread reads its row of V once for all KQ.
-// The sums run in the single-RHS kernel's order (four partial sums by
-// column mod 4), so each RHS gets that kernel's bits.  NT: V is read with
-// non-temporal loads (one chunk covers every RHS, so V is read once; with
-// several chunks, cached reads let later chunks reuse some of it).
-template <int W, int KQ, typename T, bool NT>
-__global__ void __launch_bounds__(W)
-    k_part_finish_multi(const double *__restrict__ y, const double *__restrict__ vt, const double *__restrict__ t,
-                        int n, int m, int k, T *__restrict__ x)
+// The tails by walks, one workgroup of kPartSplit x W threads per run of
+// consecutive tails and chunk of KQ right-hand sides.  Used where blocks damp
+// their history (four in a row by kPartDamp or more) or are few.  What block p
+// - s adds to t_p is at most norm(B_p ... B_{p-s+1}) max|a_{p-s}|; the walk to
+// t_p starts at the farthest block for which a bound of that is above 2^-66
+// max|a_p| (all that is left out, 256 blocks at most, then stays below 2^-58,
+// a 32nd of the rounding of t_p's own terms) and not below the smallest
+// double.  How far that is depends on the right-hand side alone, so it gets
+// the same bits in every chunk.  Blocks are looked at kPartReach back: there
+// the factor has passed 2^-2048, the whole range of a double.  After a block
+// with an infinity or a NaN in its tail every tail is NaN (0 times an
+// infinity is NaN, and each product has all W columns).
+// The bound is taken in logarithms, whole numbers of 1 / 256 rounded up, of
+// the norms of four matrices' products, and of single matrices for the rest:
+// fade[i].x is the sum of those of B_1 ... B_i, fade[i].y of B_i ... B_{i-3},
+// B_{i-4} ... (sums whose differences are right whether or not they wrap).
+// Four matrices' product is smaller than their norms' product: 2^-58 against
+// 2^-36 at 512 rows of bandwidth 96, which is 5 products to a tail, not 8.
+// d[j] += sum over kk of m[kk] times s[j] of lane kk of the 16 lanes' row, in
+// two chains by kk mod 2
+template <int KK, int KQ>
+__device__ __forceinline__ void part_rank(const double (&m)[16], const double (&s)[KQ], double (&d)[KQ][2])
 {
-    __shared__ double st[2][W][KQ];
-    const int lo = (int)blockIdx.x * W;
-    const long long q0 = (long long)blockIdx.y * KQ;
-    const int p_lo = lo / m, p_hi = (min(n, lo + W) - 1) / m;
-    for (int e = (int)threadIdx.x; e < 2 * KQ * W; e += W) {
-        const int sblk = e / (KQ * W), j = (e / W) % KQ, c = e % W;
-        const int p = sblk == 0 ? p_lo : p_hi;
-        st[sblk][c][j] = p > 0 ? t[((long long)(p - 1) * k + q0 + j) * W + c] : 0.0;
+    if constexpr (KK < 16) {
+#pragma unroll
+        for (int j = 0; j < KQ; ++j)
+            d[j][KK % 2] = __builtin_fma(
+                m[KK], __builtin_amdgcn_update_dpp(0.0, s[j], 0x150 + KK, 0xf, 0xf, true), d[j][KK % 2]);  // row_newbcast
+        part_rank<KK + 1, KQ>(m, s, d);
+    }
+}
+
+constexpr double kPartDamp = 0x1p-32;
+constexpr int kPartReach = 4 * kWave;
+template <int W, int KQ>
+__global__ void __launch_bounds__(kPartSplit * W, W >= 256 && KQ >= 2 ? 7 : 1)
+    k_part_walk(const double *__restrict__ a, const unsigned long long *__restrict__ top,
+                const double *__restrict__ bm, const uint2 *__restrict__ fade, double *__restrict__ tail,
+                int q_count, int run, int k)
+{
+    constexpr int kLen = W / kPartSplit, kThreads = kPartSplit * W;
+    constexpr unsigned long long kInf = 0x7FF0000000000000ULL, kNormal = 0x0010000000000000ULL;
+    // neighbours read the same matrices: each of the 8 XCDs, to which
+    // workgroups go in turn, takes consecutive runs (gridDim.x is a multiple)
+    const int p0 = ((int)blockIdx.x % 8 * ((int)gridDim.x / 8) + (int)blockIdx.x / 8) * run;
+    const int p1 = min(q_count, p0 + run);
+    if (p0 >= q_count) return;
+    const int t = (int)threadIdx.x, c = t % W, kq = t / W, lane = t % kWave, wave = t / kWave;
+    __shared__ double sv[KQ][W];
+    __shared__ double red[kPartSplit][KQ][W];
+    __shared__ int from[KQ], lost[KQ];  // per right-hand side: its walk's start, the first block past repair
+    if (t < KQ) {
+        from[t] = p0;
+        lost[t] = q_count;
     }
     __syncthreads();
-    const int i = lo + (int)threadIdx.x;
-    if (i >= n) return;
-    const int p = i / m;
-    const int sblk = p == p_lo ? 0 : 1;
-    double acc[KQ][4];
+    const unsigned long long *tq = top + (long long)blockIdx.y * KQ;
+    for (int h = t; h < p1 - 1; h += kThreads) {
 #pragma unroll
-    for (int j = 0; j < KQ; ++j)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc[j][u] = 0.0;
-    if (p > 0) {
-#pragma unroll 2
-        for (int c = 0; c < W; c += 4) {
-            double mv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                mv[u] = NT ? __builtin_nontemporal_load(vt + (long long)(c + u) * n + i) : vt[(long long)(c + u) * n + i];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int j = 0; j < KQ; ++j) acc[j][u] = __builtin_fma(mv[u], st[sblk][c + u][j], acc[j][u]);
-        }
+        for (int j = 0; j < KQ; ++j)
+            if (tq[(long long)h * k + j] >= kInf) atomicMin(&lost[j], h);
     }
+    // (tail, right-hand side) pairs, one to a wavefront: lane l looks at the
+    // blocks l, l + 64, ... back
+    for (int e = wave; e < (p1 - p0) * KQ; e += kThreads / kWave) {
+        const int p = p0 + e / KQ, j = e % KQ;
+        const unsigned long long own = tq[(long long)p * k + j];
+        int far = 0;
 #pragma unroll
-    for (int j = 0; j < KQ; ++j) {
-        const long long g = (long long)i * k + q0 + j;
-        double xi = y[g];
-        if (p > 0) xi -= (acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]);
-        x[g] = (T)xi;
+        for (int i = 0; i < kPartReach; i += kWave) {
+            const int s = i + lane, h = p - s;
+            if (s == 0 || h < 0) continue;
+            const unsigned long long bits = tq[(long long)h * k + j];
+            // log2 in 256ths, the exponent biased: above the term's (an
+            // exponent and a fraction fall short of it by 0.087 at most)
+            const int mid = p - (s & ~3);
+            const int term = (int)(bits >> 44) + 24 + (int)(fade[p].y - fade[mid].y) + (int)(fade[mid].x - fade[h].x);
+            const int floor = own >= kNormal && own < kInf ? (int)(own >> 44) - 66 * 256 : -60 * 256;
+            if (bits != 0 && term > max(floor, -60 * 256)) far = s;
+        }
+#pragma unroll
+        for (int s = 1; s < kWave; s *= 2) far = max(far, __shfl_xor(far, s));
+        if (lane == 0) atomicMin(&from[j], p - far);
+    }
+    __syncthreads();
+    int h = p0;
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) h = min(h, lost[j] < p0 ? p0 : from[j]);
+    // A thread has one row and kLen columns of a product, the vectors' values
+    // 16 columns at a time, one to a lane: a lane's value goes to its row of
+    // 16 by DPP, one LDS read per lane for 16 columns.  At W = 128 the part of
+    // the next product's matrix is loaded while the current one is joined.
+    // The matrices' bytes bound it: at n = 500,000 (m = 1000, 3 products to a
+    // tail, 64 MB) 19 us; at n = 200,000 with 8 right-hand sides (m = 512, 5
+    // products) 31 us, 50 with two chunks of 4.  The scan's launches took 83
+    // and 140 (1023 tails).
+    constexpr bool kAhead = W == kPartW;
+    constexpr int kCols = 16;
+    double mat[kAhead ? kLen / kCols : 1][kCols];
+    auto load = [&](int p, int g, double (&m)[kCols]) {
+        const double *M = bm + ((long long)(p - 1) * W + kq * kLen + g * kCols) * W + c;
+#pragma unroll
+        for (int kk = 0; kk < kCols; ++kk) m[kk] = M[(long long)kk * W];
+    };
+    double v[KQ];
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) v[j] = 0.0;
+    for (bool head = true;; head = false) {
+        double mv[KQ], ah[KQ];
+        if (t < W) {
+#pragma unroll
+            for (int j = 0; j < KQ; ++j) ah[j] = a[part_vec<W, KQ>(h, k, j) + c];
+        }
+        if (!head) {
+            __syncthreads();  // sv is written, red is read
+            double d[KQ][2];
+#pragma unroll
+            for (int j = 0; j < KQ; ++j) d[j][0] = d[j][1] = 0.0;
+#pragma unroll(kAhead ? kLen / kCols : 1)
+            for (int g = 0; g < kLen / kCols; ++g) {
+                double (&m)[kCols] = mat[kAhead ? g : 0];
+                if (!kAhead) load(h, g, m);
+                double s[KQ];
+#pragma unroll
+                for (int j = 0; j < KQ; ++j) s[j] = sv[j][kq * kLen + g * kCols + t % kCols];
+                part_rank<0, KQ>(m, s, d);
+            }
+#pragma unroll
+            for (int j = 0; j < KQ; ++j) mv[j] = d[j][0] + d[j][1];
+#pragma unroll
+            for (int j = 0; j < KQ; ++j) red[kq][j][c] = mv[j];
+        }
+        if (kAhead && h + 1 < p1) {
+#pragma unroll
+            for (int g = 0; g < kLen / kCols; ++g) load(h + 1, g, mat[kAhead ? g : 0]);
+        }
+        if (!head) __syncthreads();
+        if (t < W) {
+#pragma unroll
+            for (int j = 0; j < KQ; ++j) {
+                v[j] = ah[j];
+                if (!head && h > from[j])
+                    v[j] += (red[0][j][c] + red[1][j][c]) + (red[2][j][c] + red[3][j][c]);
+                sv[j][c] = v[j];
+                if (h >= p0)
+                    tail[part_vec<W, KQ>(h, k, j) + c] = lost[j] < h ? as_val(VBits<double>::kQNaN) : v[j];
+            }
+        }
+        if (++h == p1) break;
     }
 }
 

@@ -74,26 +74,28 @@ inline int lpr_log2_for(int k)
 }  // namespace
 
 // State of a partitioned banded solve: blocks of m rows (P of them, Q = P - 1
-// coupled tails of W values, W = 128 or 256); the block-diagonal part's
-// off-diagonals in ELL slabs of ew per row plus an overflow CSR, and its
-// reciprocal diagonal; V = D^{-1} C column-major (n x W); the tail scan's
-// W x W matrices in bm: B_p at p - 1,
-// the in-group products W_p at w_off + p - gs, and for each round r of the
-// group-carry scan G - 2^r matrices from m_off[r]; the solve's work vectors.
+// coupled tails of W values, W = 128 or 256); the blocks' rows as records
+// (layout in kernels.h, k_part_records) of J entries per lane, block p's from
+// at[p], and where its first few records start; the tail scan's W x W
+// matrices in bm: B_p at p - 1 and, unless the tails are walked, the in-group
+// products W_p at w_off + p - gs, and for each round r of the group-carry
+// scan G - 2^r matrices from m_off[r]; the solve's work vectors.
 struct PartState {
-    int W = kPartW;                   // tail width: the coupling columns
-    int m = 0, P = 0, Q = 0, ew = 0;  // ew: ELL slab width (<= kPartEll)
-    int gs = 0, G = 0, rounds = 0;    // tails per group, groups, carry-scan rounds
-    int *ell_c = nullptr, *ov_rp = nullptr, *ov_c = nullptr;
-    double *ell_v = nullptr, *ov_v = nullptr, *diag = nullptr;
-    double *near = nullptr;  // per row: the entries in columns i-1 and i-2 (in-block)
-    double *vt = nullptr;
+    int W = kPartW;                 // tail width: the coupling columns
+    int m = 0, P = 0, Q = 0, J = 0;
+    bool walk = false;              // the blocks damp their history, or are few: k_part_walk
+    int gs = 0, G = 0, rounds = 0;  // tails per group, groups, carry-scan rounds
+    uint4 *rec = nullptr;
+    int *at = nullptr;
+    uint2 *first = nullptr;
     double *bm = nullptr;
+    uint2 *fade = nullptr;     // k_part_walk: how the blocks damp
     long long w_off = 0;
     std::vector<long long> m_off;
     // work vectors, sized for kcap right-hand sides (grown by a solve with more)
     int kcap = 0;
-    double *y = nullptr, *a = nullptr, *u = nullptr, *t = nullptr, *c0 = nullptr, *c1 = nullptr;
+    double *a = nullptr, *u = nullptr, *t = nullptr, *c0 = nullptr, *c1 = nullptr;
+    unsigned long long *top = nullptr;      // the largest magnitude of each a_p
     double *res = nullptr, *cor = nullptr;  // refinement: FP64 residual and correction (n * kcap)
 };
 
@@ -106,7 +108,7 @@ struct HopState {
 
 // The RHS-block pick of an autotuned plan for one right-hand-side count:
 // thread-per-row workgroups per CU, threads per workgroup and right-hand
-// sides per lane, or the partitioned block solve's right-hand sides per
+// sides per lane, or the partitioned sweeps' right-hand sides per
 // wavefront (0: the plan's).
 struct RhsPick {
     int bpc = 0, block = 0, kr = 0, rpl = 0;
@@ -147,7 +149,7 @@ struct cap_plan_s {
     // right-hand-side count on the first cap_plan_solve with that count
     bool tune_rhs = false;
     std::map<int, RhsPick> rhs_pick;
-    int part_kr = 0;  // partition block solve: right-hand sides per wavefront (0: the fixed rule)
+    int part_kr = 0;  // partition sweeps: right-hand sides per wavefront (0: the fixed rule)
     int rpl = 1;      // thread-per-row, several right-hand sides: right-hand sides per lane
     int fixed_rpl = 0;  // cap_opts.rhs_per_lane: the multi-RHS block the caller fixed (0: none)
     bool auto_algo = false;  // created with CAP_ALGO_AUTO
@@ -400,9 +402,9 @@ void free_partition(cap_plan p)
     PartState *ps = p->part;
     if (!ps) return;
     (void)hipDeviceSynchronize();
-    for (void *b : {(void *)ps->ell_c, (void *)ps->ov_rp, (void *)ps->ov_c, (void *)ps->ell_v, (void *)ps->ov_v,
-                    (void *)ps->diag, (void *)ps->near, (void *)ps->vt, (void *)ps->bm, (void *)ps->y, (void *)ps->a, (void *)ps->u,
-                    (void *)ps->t, (void *)ps->c0, (void *)ps->c1, (void *)ps->res, (void *)ps->cor})
+    for (void *b : {(void *)ps->rec, (void *)ps->at, (void *)ps->first, (void *)ps->bm, (void *)ps->fade,
+                    (void *)ps->a, (void *)ps->u, (void *)ps->t, (void *)ps->c0, (void *)ps->c1, (void *)ps->top,
+                    (void *)ps->res, (void *)ps->cor})
         if (b) (void)hipFree(b);
     delete ps;
     p->part = nullptr;
@@ -609,29 +611,29 @@ int ensure_part_rhs(cap_plan p, int k)
     PartState *ps = p->part;
     if (k <= ps->kcap) return CAP_OK;
     CAP_HIP_TRY(hipDeviceSynchronize());
-    for (double **v : {&ps->y, &ps->a, &ps->u, &ps->t, &ps->c0, &ps->c1, &ps->res, &ps->cor}) {
+    for (double **v : {&ps->a, &ps->u, &ps->t, &ps->c0, &ps->c1, &ps->res, &ps->cor}) {
         if (*v) (void)hipFree(*v);
         *v = nullptr;  // res / cor come back at the new size when a refined solve needs them
     }
+    if (ps->top) (void)hipFree(ps->top);
+    ps->top = nullptr;
     ps->kcap = 0;
     const size_t tails = (size_t)ps->Q * k * ps->W, carries = (size_t)ps->G * k * ps->W;
-    CAP_TRY(dev_alloc(&ps->y, (size_t)p->n * k));
     CAP_TRY(dev_alloc(&ps->a, tails));
-    CAP_TRY(dev_alloc(&ps->u, tails));
     CAP_TRY(dev_alloc(&ps->t, tails));
-    CAP_TRY(dev_alloc(&ps->c0, carries));
-    CAP_TRY(dev_alloc(&ps->c1, carries));
+    CAP_TRY(dev_alloc(&ps->top, (size_t)ps->Q * k));
+    if (!ps->walk) {
+        CAP_TRY(dev_alloc(&ps->u, tails));
+        CAP_TRY(dev_alloc(&ps->c0, carries));
+        CAP_TRY(dev_alloc(&ps->c1, carries));
+    }
     ps->kcap = k;
     return CAP_OK;
 }
 
-// Right-hand sides per wavefront of the block solve, at most (they share the
-// row data; each adds an independent reduction chain and 2 KB of LDS ring).
-// Below that cap a solve takes k / 2, so that the block solve runs about two
-// wavefronts per SIMD (P = 1024 blocks): on the 500 k deep band, k = 4 took
-// 0.417 ms at 2 per wavefront against 0.441 at 4, and k = 16 0.975 ms at 4
-// against 1.209 at 2.
-constexpr int kPartBlockRhs = 4;
+// Right-hand sides per wavefront of a sweep, at most (they share the row
+// data; each adds an independent chain and 2W LDS slots).
+constexpr int kPartSweepRhs = 4;
 
 // The largest power of two up to `cap` that divides k: the chunk of
 // right-hand sides one workgroup takes.
@@ -642,20 +644,46 @@ inline int part_chunk(int k, int cap)
     return c;
 }
 
-template <int W, int KR, typename T>
-void launch_part_block(cap_plan p, const T *b, int k, hipStream_t st)
+// One sweep over `blocks` blocks, k right-hand sides (KR | k) of them to a
+// wavefront.  The grid's x is rounded up to the 8 XCDs, so that the
+// wavefronts of a block's right-hand sides share an L2.
+template <int W, int KR, typename T, PartSweep MODE>
+void launch_part_sweep(const PartState *ps, int n, const T *b, const double *hist, double *tails, T *x, int k,
+                       int blocks, hipStream_t st)
 {
-    const PartState *ps = p->part;
-    k_part_block<W, KR, T><<<dim3((unsigned)ps->P, (unsigned)(k / KR)), kWave, 0, st>>>(
-        ps->ell_c, ps->ell_v, ps->ov_rp, ps->ov_c, ps->ov_v, ps->diag, (const double2 *)ps->near, b, ps->y, ps->a,
-        p->n, ps->m, ps->ew, k, ps->Q);
+    const int waves = part_chunk(k / KR, kPartWaves);
+    const dim3 grid((unsigned)((blocks + 7) / 8 * 8), (unsigned)(k / KR / waves));
+    auto go = [&](auto j) {
+        k_part_sweep<W, KR, decltype(j)::value, T, MODE>
+            <<<grid, waves * kWave, 0, st>>>(ps->rec, ps->at, ps->first, b, hist, tails, ps->top, x, n, ps->m, k, blocks);
+    };
+    switch (ps->J) {
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    default: go(std::integral_constant<int, kPartMaxJ>{}); break;
+    }
 }
+
+template <int W, typename T, PartSweep MODE>
+void part_sweep(const PartState *ps, int n, int kr, const T *b, const double *hist, double *tails, T *x, int k,
+                int blocks, hipStream_t st)
+{
+    switch (kr) {
+    case 4: launch_part_sweep<W, 4, T, MODE>(ps, n, b, hist, tails, x, k, blocks, st); break;
+    case 2: launch_part_sweep<W, 2, T, MODE>(ps, n, b, hist, tails, x, k, blocks, st); break;
+    default: launch_part_sweep<W, 1, T, MODE>(ps, n, b, hist, tails, x, k, blocks, st); break;
+    }
+}
+
+// Right-hand sides per wavefront without a tuned pick: n = 200,000, bandwidth
+// 96, four of them: one 80 us, two 100; eight: 140, two 114, four 159.
+inline int part_sweep_rhs(int k) { return part_chunk(k, std::min(kPartSweepRhs, std::max(1, k / kPartWaves))); }
 
 // Right-hand sides per workgroup of the group scan and the carry rounds, at
 // most: those grids have only G (= P / gs) workgroups per chunk, and each step
 // of a workgroup is a chain, so they keep more, smaller chunks than the
-// fix-up and the finish (Q and n / W workgroups), which take 16 (8 at W =
-// 256: the finish stages 2 x W x KQ values in LDS).
+// fix-up (Q workgroups), which takes 16 (8 at W = 256).  The walk's products
+// are a chain too.
 constexpr int kPartScanRhs = 4;
 
 // The tail scan over the group carries, KQ right-hand sides per workgroup
@@ -687,66 +715,78 @@ double *launch_part_carries(cap_plan p, int k, hipStream_t st)
     return k == KQ ? part_carries<W, KQ, true>(p, k, st) : part_carries<W, KQ, false>(p, k, st);
 }
 
-// The fix-up of every tail and the finish, KQ right-hand sides per
-// workgroup (KQ | k); `tg`: the scanned group carries.
-template <int W, int KQ, typename T>
-void launch_part_fix(cap_plan p, const double *tg, T *x, int k, hipStream_t st)
+// The fix-up of every tail, KQ right-hand sides per workgroup (KQ | k);
+// `tg`: the scanned group carries.
+template <int W, int KQ>
+void launch_part_fix(cap_plan p, const double *tg, int k, hipStream_t st)
 {
     const PartState *ps = p->part;
-    const unsigned chunks = (unsigned)(k / KQ);
-    const long long mat = (long long)W * W;
-    if (chunks == 1)  // non-temporal matrix reads when each W_p is read once
-        k_part_fixup<W, KQ, true><<<dim3(ps->Q, chunks), W, 0, st>>>(ps->u, tg, ps->bm + ps->w_off * mat, ps->gs,
-                                                                     ps->t, k);
+    const dim3 grid((unsigned)ps->Q, (unsigned)(k / KQ));
+    const double *wm = ps->bm + ps->w_off * W * W;
+    if (k == KQ)  // non-temporal matrix reads when each W_p is read once
+        k_part_fixup<W, KQ, true><<<grid, W, 0, st>>>(ps->u, tg, wm, ps->gs, ps->t, k);
     else
-        k_part_fixup<W, KQ, false><<<dim3(ps->Q, chunks), W, 0, st>>>(ps->u, tg, ps->bm + ps->w_off * mat, ps->gs,
-                                                                      ps->t, k);
-    if constexpr (KQ == 1)
-        k_part_finish<W, T><<<blocks_for((long long)p->n * k), kBlock, 0, st>>>(ps->y, ps->vt, ps->t, p->n, ps->m, k,
-                                                                               x);
-    else {  // m >= W: a workgroup's W rows span at most two blocks
-        const dim3 grid((unsigned)((p->n + W - 1) / W), chunks);
-        if (chunks == 1)
-            k_part_finish_multi<W, KQ, T, true><<<grid, W, 0, st>>>(ps->y, ps->vt, ps->t, p->n, ps->m, k, x);
-        else
-            k_part_finish_multi<W, KQ, T, false><<<grid, W, 0, st>>>(ps->y, ps->vt, ps->t, p->n, ps->m, k, x);
-    }
+        k_part_fixup<W, KQ, false><<<grid, W, 0, st>>>(ps->u, tg, wm, ps->gs, ps->t, k);
+}
+
+// Workgroups of the walks, about: one per CU.  A run of tails walks to its
+// first one and takes one product for each further one, so fewer and longer
+// runs read fewer matrices.  Whatever k: the runs set where walks start, and
+// so a right-hand side's bits.
+constexpr int kWalkGroups = 256;
+
+template <int W, int KQ>
+void launch_part_walk(cap_plan p, int k, hipStream_t st)
+{
+    const PartState *ps = p->part;
+    const int run = (ps->Q + kWalkGroups - 1) / kWalkGroups;
+    k_part_walk<W, KQ><<<dim3((unsigned)(((ps->Q + run - 1) / run + 7) / 8 * 8), (unsigned)(k / KQ)), kPartSplit * W, 0, st>>>(
+        ps->a, ps->top, ps->bm, ps->fade, ps->t, ps->Q, run, k);
 }
 
 // One solve of a partitioned plan (k FP64 right-hand sides, interleaved:
-// b[row * k + q]): y = D^{-1} b (one wavefront per block and chunk of
-// right-hand sides), the block tails, the two-level tail scan (in groups,
-// over the group carries, then the fix-up; grids over tails x chunks), then
-// x = y - V t.  Every step is on `st`; none of them waits on another
-// workgroup.  Each right-hand side gets the bits of its own one-RHS solve.
+// b[row * k + q]): the sweep for the block tails, the tails joined (walked,
+// or the scan in groups, over the group carries and the fix-up; grids over
+// tails x chunks), and the sweep for x.  Every step is on `st`; none of them
+// waits on another workgroup.  Each right-hand side gets the bits of its own
+// one-RHS solve.  x may be b: a block's rows of b are read before they are
+// written, by the same wavefront.
 template <int W, typename T>
 int launch_partition_w(cap_plan p, const T *b, T *x, int k, hipStream_t st)
 {
-    // right-hand sides per wavefront of the block solve: the plan's tuned
-    // pick for k when it has one, else the largest power of two up to
-    // min(4, k / 2) that divides k
-    int kr = part_chunk(k, std::min(kPartBlockRhs, std::max(1, k / 2)));
-    if (p->part_kr > 0 && p->part_kr <= kPartBlockRhs && k % p->part_kr == 0) kr = p->part_kr;
-    switch (kr) {
-    case 4: launch_part_block<W, 4, T>(p, b, k, st); break;
-    case 2: launch_part_block<W, 2, T>(p, b, k, st); break;
-    default: launch_part_block<W, 1, T>(p, b, k, st); break;
+    // right-hand sides per wavefront: the plan's tuned pick for k when it has
+    // one, else as many as leave a workgroup's wavefronts work
+    const PartState *ps = p->part;
+    int kr = part_sweep_rhs(k);
+    if (p->part_kr > 0 && p->part_kr <= kPartSweepRhs && k % p->part_kr == 0) kr = p->part_kr;
+    part_sweep<W, T, kPartTails>(ps, p->n, kr, b, nullptr, ps->a, (T *)nullptr, k, ps->Q, st);
+    if (ps->walk) {
+        switch (part_chunk(k, W == kPartW ? 2 * kPartScanRhs : kPartScanRhs)) {
+        case 8:
+            if constexpr (W == kPartW) launch_part_walk<W, 8>(p, k, st);
+            break;
+        case 4: launch_part_walk<W, 4>(p, k, st); break;
+        case 2: launch_part_walk<W, 2>(p, k, st); break;
+        default: launch_part_walk<W, 1>(p, k, st); break;
+        }
+    } else {
+        const double *tg = nullptr;
+        switch (part_chunk(k, kPartScanRhs)) {
+        case 4: tg = launch_part_carries<W, 4>(p, k, st); break;
+        case 2: tg = launch_part_carries<W, 2>(p, k, st); break;
+        default: tg = launch_part_carries<W, 1>(p, k, st); break;
+        }
+        switch (part_chunk(k, W == kPartW ? 16 : 8)) {
+        case 16:
+            if constexpr (W == kPartW) launch_part_fix<W, 16>(p, tg, k, st);
+            break;
+        case 8: launch_part_fix<W, 8>(p, tg, k, st); break;
+        case 4: launch_part_fix<W, 4>(p, tg, k, st); break;
+        case 2: launch_part_fix<W, 2>(p, tg, k, st); break;
+        default: launch_part_fix<W, 1>(p, tg, k, st); break;
+        }
     }
-    const double *tg = nullptr;
-    switch (part_chunk(k, kPartScanRhs)) {
-    case 4: tg = launch_part_carries<W, 4>(p, k, st); break;
-    case 2: tg = launch_part_carries<W, 2>(p, k, st); break;
-    default: tg = launch_part_carries<W, 1>(p, k, st); break;
-    }
-    switch (part_chunk(k, W == kPartW ? 16 : 8)) {
-    case 16:
-        if constexpr (W == kPartW) launch_part_fix<W, 16, T>(p, tg, x, k, st);
-        break;
-    case 8: launch_part_fix<W, 8, T>(p, tg, x, k, st); break;
-    case 4: launch_part_fix<W, 4, T>(p, tg, x, k, st); break;
-    case 2: launch_part_fix<W, 2, T>(p, tg, x, k, st); break;
-    default: launch_part_fix<W, 1, T>(p, tg, x, k, st); break;
-    }
+    part_sweep<W, T, kPartX>(ps, p->n, kr, b, ps->t, nullptr, x, k, ps->P, st);
     CAP_HIP_TRY(hipGetLastError());
     return CAP_OK;
 }
@@ -1136,7 +1176,7 @@ int time_candidate(cap_plan p, int algo, int sync, const void *b, void *x, int r
 // lanes, poll at once), 1024-thread workgroups with 1, 2, 4 (8 in FP32)
 // right-hand sides per lane, and the pick again with readiness in x;
 // partitioned plans time 1, 2 and 4 right-hand sides per wavefront of the
-// block solve (the ones that divide k).  Every candidate gives the same
+// sweeps (the ones that divide k).  Every candidate gives the same
 // bits.  The plan's own settings are timed first and another must be 2 %
 // faster to win.  Waits for the device (events).
 int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
@@ -1160,7 +1200,7 @@ int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
             if (k >= 4) cands.push_back({1, kBlock, 0, 4, -1, 0, 0});
         }
     } else if (algo == CAP_ALGO_PARTITION) {
-        const int dflt = part_chunk(k, std::min(kPartBlockRhs, std::max(1, k / 2)));
+        const int dflt = part_sweep_rhs(k);
         cands.push_back({0, 0, dflt});
         for (int kr : {1, 2, 4})
             if (kr != dflt && k % kr == 0) cands.push_back({0, 0, kr});
@@ -1230,58 +1270,209 @@ void apply_choice(cap_plan p, const TuneChoice &c)
 // Tables of the partitioned banded solve (CAP_ALGO_PARTITION), built once:
 // plans whose lower bandwidth is at most kPartWMax and that split into at
 // least two blocks; CAP_ERR_UNSUPPORTED otherwise.  The tail width W is 128
-// when the bandwidth allows, else 256; blocks hold m = max(W, ceil(n /
-// kPartBlocks)) rows.  The host lays out the block-diagonal part (ELL slabs
-// + overflow CSR + reciprocal diagonal); V = D^{-1} C comes from W / 64
-// 64-RHS solves of a batch over the blocks (dropped afterwards) and is
-// stored column-major; the scan's matrices are formed round by round.
+// when the bandwidth allows, else 256.  Blocks hold at least W and n /
+// kPartBlocks rows, and more, kPartRows or n / kPartSpread, where that leaves
+// 16 blocks: a sweep takes about 0.2 us per 8 rows of a block, 14 us for 512
+// rows, and its bytes take 0.1 us per 1000 rows of the matrix, so up to n /
+// kPartSpread rows cost nothing, while fewer blocks are fewer matrices to
+// read and more damping in each.  Blocks that damp too little to be walked
+// are made longer, up to kPartLongest rows, when that is enough (n = 200,000,
+// bandwidth 128, 13 entries a row: 640 rows and the scan 107 us, 720 rows and
+// the walk 72, 1440 rows 96).  A matrix whose blocks grow (refused at that
+// size) is tried with the smallest.
+// The host groups the rows into records; the records are filled, the B_p
+// swept and the scan's matrices formed on the device.
 constexpr int kPartBlocks = 1024;
+constexpr int kPartRows = 512;
+constexpr int kPartSpread = 500;
+constexpr int kPartLongest = 1280;
 // largest relative max-norm difference from the sequential solve accepted
 // when the tables are checked at plan creation (the FP64 bar is 1e-12)
 constexpr double kPartStableTol = 1e-13;
 constexpr int kPartGroup = 8;  // tails per group of the scan's first level
-// Largest table set a partitioned plan may hold (device; the host builds the
-// same tables once): larger matrices are refused rather than risk exhausting
-// memory behind the caller's back.
+// Largest table set a partitioned plan may hold: larger matrices are refused
+// rather than risk exhausting memory behind the caller's back.
 constexpr double kPartMaxBytes = 16.0 * (1ull << 30);
 
-int build_partition_tables(cap_plan p, const std::vector<int> &rp_host, hipStream_t st);
+// The matrix a plan's records are made of: the plan's own, or, when a row has
+// more entries than a record (duplicates), a copy with the duplicates added up.
+struct PartRows {
+    std::vector<int> rp, ci;
+    std::vector<double> v;
+};
+
+int build_partition_tables(cap_plan p, const PartRows &mat, int w, int m, bool merged, int *longer, hipStream_t st);
 
 int build_partition(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
 {
+    if (p->part) return CAP_OK;
     try {
-        return build_partition_tables(p, rp_host, st);
+        const int n = p->n, nnz = p->nnz;
+        PartRows mat;
+        mat.rp = rp_host;
+        mat.ci.resize((size_t)nnz);
+        CAP_HIP_TRY(hipMemcpy(mat.ci.data(), p->ci, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost));
+        int w = 0, longest = 0;
+        for (int i = 0; i < n; ++i) {
+            longest = std::max(longest, mat.rp[i + 1] - mat.rp[i]);
+            for (int j = mat.rp[i]; j < mat.rp[i + 1]; ++j) w = std::max(w, i - mat.ci[j]);
+        }
+        if (w > kPartWMax) return CAP_ERR_UNSUPPORTED;
+        mat.v.resize((size_t)nnz);  // FP32 values widen exactly
+        if (p->vt == CAP_F64) {
+            CAP_HIP_TRY(hipMemcpy(mat.v.data(), p->val, sizeof(double) * (size_t)nnz, hipMemcpyDeviceToHost));
+        } else {
+            std::vector<float> vf((size_t)nnz);
+            CAP_HIP_TRY(hipMemcpy(vf.data(), p->val, sizeof(float) * (size_t)nnz, hipMemcpyDeviceToHost));
+            for (size_t e = 0; e < vf.size(); ++e) mat.v[e] = (double)vf[e];
+        }
+        const bool merged = longest > kPartSeg * kPartSeg * kPartMaxJ;
+        if (merged) {
+            PartRows u;
+            std::vector<double> sum((size_t)w + 1);
+            std::vector<char> has((size_t)w + 1);
+            u.rp.push_back(0);
+            for (int i = 0; i < n; ++i) {
+                std::fill(sum.begin(), sum.end(), 0.0);
+                std::fill(has.begin(), has.end(), 0);
+                for (int j = mat.rp[i]; j < mat.rp[i + 1]; ++j) {
+                    sum[(size_t)(i - mat.ci[j])] += mat.v[(size_t)j];
+                    has[(size_t)(i - mat.ci[j])] = 1;
+                }
+                for (int d = std::min(i, w); d >= 0; --d) {
+                    if (!has[(size_t)d]) continue;
+                    u.ci.push_back(i - d);
+                    u.v.push_back(sum[(size_t)d]);
+                }
+                u.rp.push_back((int)u.ci.size());
+            }
+            mat = std::move(u);
+        }
+        const int W = w <= kPartW ? kPartW : kPartWMax;
+        const int least = std::max(W, (n + kPartBlocks - 1) / kPartBlocks);
+        const int m = std::max(least, std::min(std::max(kPartRows, n / kPartSpread), (n + 15) / 16));
+        int longer = 0;
+        int rc = build_partition_tables(p, mat, w, m, merged, &longer, st);
+        if (longer > 0) rc = build_partition_tables(p, mat, w, longer, merged, nullptr, st);
+        if (rc == CAP_ERR_UNSUPPORTED && m > least) rc = build_partition_tables(p, mat, w, least, merged, nullptr, st);
+        return rc;
     } catch (const std::bad_alloc &) {
         free_partition(p);
         return CAP_ERR_ALLOC;
     }
 }
 
-int build_partition_tables(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
+template <int J, typename T>
+void fill_records(const int *rp, const int *ci, const T *val, const int *rows, int count, PartState *ps, hipStream_t st)
 {
-    if (p->part) return CAP_OK;
-    const int n = p->n, nnz = p->nnz;
-    std::vector<int> ci((size_t)nnz);
-    CAP_HIP_TRY(hipMemcpy(ci.data(), p->ci, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost));
-    int w = 0;
-    for (int i = 0; i < n; ++i)
-        for (int j = rp_host[i]; j < rp_host[i + 1]; ++j) w = std::max(w, i - ci[j]);
-    if (w > kPartWMax) return CAP_ERR_UNSUPPORTED;
-    const int W = w <= kPartW ? kPartW : kPartWMax, ring = 2 * W;
-    const int m = std::max(W, (n + kPartBlocks - 1) / kPartBlocks);
+    k_part_records<J, T><<<(unsigned)count, kWave, 0, st>>>(rp, ci, val, rows, ps->at, ps->m, ps->rec);
+}
+template <typename T>
+void fill_records(const int *rp, const int *ci, const T *val, const int *rows, int count, PartState *ps, hipStream_t st)
+{
+    switch (ps->J) {
+    case 2: fill_records<2, T>(rp, ci, val, rows, count, ps, st); break;
+    case 4: fill_records<4, T>(rp, ci, val, rows, count, ps, st); break;
+    default: fill_records<kPartMaxJ, T>(rp, ci, val, rows, count, ps, st); break;
+    }
+}
+
+// The norms of B_q (one[q], q >= 1) and of B_q B_{q-1} B_{q-2} B_{q-3}
+// (four[q], q >= 4); B_q at bm + (q - 1) W^2.  Waits for st.
+template <int W>
+int part_norms(const double *bm, int Q, double *one, double *four, hipStream_t st)
+{
+    double *prod = nullptr, *norm = nullptr;
+    int3 *d_ops = nullptr;
+    const long long mat = (long long)W * W;
+    const int B = Q - 1;
+    std::vector<int3> ops;  // pairs behind the copies of the B_q, then fours behind the pairs
+    for (int q = 2; q < Q; ++q) ops.push_back(make_int3(B + q - 1, q - 1, q - 2));
+    const int pairs = (int)ops.size();
+    for (int q = 4; q < Q; ++q) ops.push_back(make_int3(2 * B + q - 1, B + q - 1, B + q - 3));
+    const int fours = (int)ops.size() - pairs;
+    int rc = CAP_OK;
+    do {
+        if ((rc = dev_alloc(&norm, (size_t)(2 * B))) || (rc = dev_alloc(&prod, (size_t)(3 * B * mat))) ||
+            (rc = dev_alloc(&d_ops, std::max<size_t>(1, ops.size()))))
+            break;
+        rc = CAP_ERR_HIP;
+        if (hipMemcpyAsync(prod, bm, sizeof(double) * (size_t)(B * mat), hipMemcpyDeviceToDevice, st) != hipSuccess ||
+            hipMemcpy(d_ops, ops.data(), sizeof(int3) * ops.size(), hipMemcpyHostToDevice) != hipSuccess)
+            break;
+        const unsigned quads = (W / 128) * (W / 128);
+        if (pairs > 0) k_part_gemm<W><<<dim3((unsigned)pairs, quads), 256, 0, st>>>(d_ops, prod);
+        if (fours > 0) k_part_gemm<W><<<dim3((unsigned)fours, quads), 256, 0, st>>>(d_ops + pairs, prod);
+        k_part_norm<W><<<(unsigned)B, W, 0, st>>>(prod, norm);
+        if (fours > 0) k_part_norm<W><<<(unsigned)fours, W, 0, st>>>(prod + (2LL * B + 3) * mat, norm + B);
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess ||
+            hipMemcpy(one + 1, norm, sizeof(double) * (size_t)B, hipMemcpyDeviceToHost) != hipSuccess ||
+            (fours > 0 &&
+             hipMemcpy(four + 4, norm + B, sizeof(double) * (size_t)fours, hipMemcpyDeviceToHost) != hipSuccess))
+            break;
+        rc = CAP_OK;
+    } while (0);
+    (void)hipStreamSynchronize(st);
+    for (void *t : {(void *)norm, (void *)prod, (void *)d_ops})
+        if (t) (void)hipFree(t);
+    return rc;
+}
+int part_norms(const double *bm, int W, int Q, double *one, double *four, hipStream_t st)
+{
+    if (Q < 2) return hipGetLastError() == hipSuccess && hipStreamSynchronize(st) == hipSuccess ? CAP_OK : CAP_ERR_HIP;
+    return W == kPartWMax ? part_norms<kPartWMax>(bm, Q, one, four, st) : part_norms<kPartW>(bm, Q, one, four, st);
+}
+
+int build_partition_tables(cap_plan p, const PartRows &mat, int w, int m, bool merged, int *longer, hipStream_t st)
+{
+    const int n = p->n, nnz = (int)mat.ci.size();
+    const std::vector<int> &rp_host = mat.rp, &ci = mat.ci;
+    const std::vector<double> &v = mat.v;
+    const int W = w <= kPartW ? kPartW : kPartWMax;
     const int P = n > 0 ? (n + m - 1) / m : 0;
     if (P < 2) return CAP_ERR_UNSUPPORTED;
-    // ELL slab width: the longest row's in-block off-diagonals in columns
-    // <= i - 3 (columns i-1 and i-2 go to the near table), rounded up to 8,
-    // at most kPartEll (the rest of a longer row goes to the overflow)
-    int longest = 1;
-    for (int i = 0; i < n; ++i) {
-        const int start = (i / m) * m;
-        int cnt = 0;
-        for (int j = rp_host[i]; j < rp_host[i + 1] - 1; ++j) cnt += ci[j] >= start && ci[j] < i - 2;
-        longest = std::max(longest, cnt);
+    // entries per lane: the fewest bytes, as if all of a row's entries but
+    // the last were outside its record; a row fits one record
+    int J = 0;
+    double best = 0.0;
+    for (int j = 2; j <= kPartMaxJ; j += 2) {
+        double segs = 0.0;
+        int most = 0;
+        for (int i = 0; i < n; ++i) {
+            const int s = std::max(1, (rp_host[i + 1] - rp_host[i] - 2 + kPartSeg * j - 1) / (kPartSeg * j));
+            segs += s;
+            most = std::max(most, (rp_host[i + 1] - rp_host[i] - 1 + kPartSeg * j - 1) / (kPartSeg * j));
+        }
+        const double cost = segs * part_pieces(j);
+        if (most <= kPartSeg && (J == 0 || cost < best)) {
+            J = j;
+            best = cost;
+        }
     }
-    const int ew = std::min(kPartEll, (longest + 7) / 8 * 8);
+    if (J == 0) return CAP_ERR_UNSUPPORTED;
+    // the records: as many of a block's next rows as their segments fit
+    std::vector<int> rows, at{0};
+    std::vector<uint2> first;
+    for (int q = 0; q < P; ++q) {
+        const int end = (int)std::min<long long>(n, (long long)(q + 1) * m);
+        for (int i = q * m; i < end;) {
+            const int r0 = i;
+            rows.push_back(r0);
+            for (int segs = 0; i < end && i < r0 + kPartSeg; ++i) {
+                int out = 0;
+                for (int j = rp_host[i]; j < rp_host[i + 1]; ++j) out += ci[j] < r0;
+                segs += std::max(1, (out + kPartSeg * J - 1) / (kPartSeg * J));
+                if (segs > kPartSeg) break;
+            }
+        }
+        unsigned f[2] = {0, 0};
+        for (int d = 0; d < kPartAhead && at.back() + d < (int)rows.size(); ++d)
+            f[d / 4] |= (unsigned)(rows[(size_t)(at.back() + d)] - q * m) << (8 * (d % 4));
+        first.push_back(make_uint2(f[0], f[1]));
+        at.push_back((int)rows.size());
+    }
+    const int n_rec = (int)rows.size();
+    rows.push_back(n);
     // the tail scan's matrix count: B (Q - 1), W (Q - gs), carry rounds
     const int Q = P - 1, gs = kPartGroup, G = (Q + gs - 1) / gs;
     int rounds = 0;
@@ -1290,64 +1481,15 @@ int build_partition_tables(cap_plan p, const std::vector<int> &rp_host, hipStrea
     const long long w_off = Q - 1;
     m_off[0] = w_off + std::max(0, Q - gs);
     for (int r = 0; r < rounds; ++r) m_off[(size_t)r + 1] = m_off[(size_t)r] + (G - (1 << r));
-    const long long n_mat = m_off[(size_t)rounds];
-    {
-        const double bytes = (double)n * (12.0 * ew + 8.0 * W + 40.0) + (double)n_mat * W * W * 8.0 + 12.0 * nnz;
-        if (bytes > kPartMaxBytes) return CAP_ERR_UNSUPPORTED;
-    }
-    std::vector<double> v((size_t)nnz);  // FP32 values widen exactly
-    if (p->vt == CAP_F64) {
-        CAP_HIP_TRY(hipMemcpy(v.data(), p->val, sizeof(double) * (size_t)nnz, hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float> vf((size_t)nnz);
-        CAP_HIP_TRY(hipMemcpy(vf.data(), p->val, sizeof(float) * (size_t)nnz, hipMemcpyDeviceToHost));
-        for (size_t e = 0; e < vf.size(); ++e) v[e] = (double)vf[e];
-    }
-    // the block-diagonal part: in-block off-diagonals in columns i-1 and i-2
-    // summed into the near table (two per row), the others in stored order,
-    // the first ew of a row in its ELL slab (as the byte offset of the
-    // column's slot in the block kernel's LDS ring; pads point at the ring's
-    // zero slot), the rest in the overflow CSR (absolute columns); and, for
-    // the coupling solves, all of them as a batch with local column indices
-    std::vector<int> ell_c((size_t)n * ew, ring * 8), ov_rp((size_t)n + 1), ov_c, ro((size_t)P + 1),
-        rpd((size_t)n + 1), cid;
-    std::vector<double> ell_v((size_t)n * ew, 0.0), ov_v, dg((size_t)n), vd, nr((size_t)n * 2, 0.0);
-    cid.reserve((size_t)nnz);
-    vd.reserve((size_t)nnz);
-    for (int q = 0; q <= P; ++q) ro[(size_t)q] = (int)std::min<long long>(n, (long long)q * m);
-    for (int i = 0; i < n; ++i) {
-        const int start = (i / m) * m, d = rp_host[i + 1] - 1;
-        ov_rp[(size_t)i] = (int)ov_c.size();
-        rpd[(size_t)i] = (int)cid.size();
-        int used = 0;
-        for (int j = rp_host[i]; j < d; ++j) {
-            if (ci[j] < start) continue;
-            cid.push_back(ci[j] - start);
-            vd.push_back(v[j]);
-            if (ci[j] >= i - 2) {  // column i-1 or i-2
-                nr[(size_t)i * 2 + (size_t)(i - 1 - ci[j])] += v[j];
-                continue;
-            }
-            if (used < ew) {
-                ell_c[(size_t)i * ew + used] = ((ci[j] - start) & (ring - 1)) * 8;  // ring slot byte offset
-                ell_v[(size_t)i * ew + used] = v[j];
-            } else {
-                ov_c.push_back(ci[j]);
-                ov_v.push_back(v[j]);
-            }
-            ++used;
-        }
-        dg[(size_t)i] = 1.0 / v[(size_t)d];
-        cid.push_back(i - start);
-        vd.push_back(v[(size_t)d]);
-    }
-    ov_rp[(size_t)n] = (int)ov_c.size();
-    rpd[(size_t)n] = (int)cid.size();
+    const long long n_mat = m_off[(size_t)rounds], mat_len = (long long)W * W;
+    const size_t rec_len = (size_t)n_rec * part_pieces(J) * kWave;
+    if ((double)rec_len * 16.0 + (double)n_mat * mat_len * 8.0 + 12.0 * nnz > kPartMaxBytes)
+        return CAP_ERR_UNSUPPORTED;
     PartState *ps = new PartState();
     p->part = ps;  // freed by free_partition on every failure from here on
     ps->W = W;
     ps->m = m;
-    ps->ew = ew;
+    ps->J = J;
     ps->P = P;
     ps->Q = Q;
     ps->gs = gs;
@@ -1355,119 +1497,128 @@ int build_partition_tables(cap_plan p, const std::vector<int> &rp_host, hipStrea
     ps->rounds = rounds;
     ps->w_off = w_off;
     ps->m_off = m_off;
-    // plan-time products, launch by launch (each list depends on the one
-    // before): the in-group products W_p = B_p W_{p-1} (W_first = B_first)
-    // for groups g >= 1, the carries' first-round matrices (the W of each
-    // group's last tail), then each carry round's products
-    std::vector<std::vector<int3>> launches;
-    for (int j = 0; j < gs; ++j) {
-        std::vector<int3> ops;
-        for (int g = 1; g * gs + j < Q; ++g) {
-            const int q = g * gs + j;
-            ops.push_back(j == 0 ? make_int3((int)(w_off + q - gs), q - 1, -1)
-                                 : make_int3((int)(w_off + q - gs), q - 1, (int)(w_off + q - 1 - gs)));
-        }
-        if (!ops.empty()) launches.push_back(ops);
-    }
-    {
-        std::vector<int3> ops;
-        for (int g = 1; g < G; ++g) {
-            const int last = std::min(Q, (g + 1) * gs) - 1;
-            ops.push_back(make_int3((int)(m_off[0] + g - 1), (int)(w_off + last - gs), -1));
-        }
-        if (!ops.empty()) launches.push_back(ops);
-    }
-    for (int r = 0; r + 1 < rounds; ++r) {
-        std::vector<int3> ops;
-        const int s = 1 << r;
-        for (int g = 2 * s; g < G; ++g)
-            ops.push_back(make_int3((int)(m_off[(size_t)r + 1] + g - 2 * s), (int)(m_off[(size_t)r] + g - s),
-                                    (int)(m_off[(size_t)r] + g - 2 * s)));
-        if (!ops.empty()) launches.push_back(ops);
-    }
-    std::vector<int3> all_ops;
-    std::vector<size_t> op_start;
-    for (const auto &l : launches) {
-        op_start.push_back(all_ops.size());
-        all_ops.insert(all_ops.end(), l.begin(), l.end());
-    }
+    int *d_rows = nullptr, *d_rp = nullptr, *d_ci = nullptr;
+    double *d_v = nullptr, *bm = nullptr;
     int3 *d_ops = nullptr;
-    cap_opts o;
-    cap_opts_default(&o);
-    o.host_inputs = 1;
-    o.validate = 0;
-    o.spin_limit = p->spin_limit;
-    o.wait_limit_ms = p->wait_ticks > 0 ? p->wait_ticks / 100000 : -1;
-    o.readiness = CAP_READY_IN_PLACE;  // plan-time only: keep the uncached pool at the solves' size
-    cap_batch b64 = nullptr;
-    double *rr = nullptr, *vv = nullptr;  // W / 64 slabs of n x 64 coupling columns, and their solves
-    const size_t slab = (size_t)n * 64, slabs = (size_t)W / 64;
-    const long long mat = (long long)W * W;
-    const size_t n_ov = std::max<size_t>(1, ov_c.size());
     int rc = CAP_OK;
     do {
-        if ((rc = dev_alloc(&ps->ell_c, ell_c.size())) || (rc = dev_alloc(&ps->ell_v, ell_v.size())) ||
-            (rc = dev_alloc(&ps->ov_rp, ov_rp.size())) || (rc = dev_alloc(&ps->ov_c, n_ov)) ||
-            (rc = dev_alloc(&ps->ov_v, n_ov)) || (rc = dev_alloc(&ps->diag, (size_t)n)) ||
-            (rc = dev_alloc(&ps->near, (size_t)n * 2)) ||
-            (rc = dev_alloc(&ps->vt, (size_t)n * W)) || (rc = ensure_part_rhs(p, 1)))
+        if ((rc = dev_alloc(&ps->rec, rec_len)) || (rc = dev_alloc(&ps->at, at.size())) ||
+            (rc = dev_alloc(&ps->first, first.size())) || (rc = dev_alloc(&d_rows, rows.size())) ||
+            (rc = dev_alloc(&ps->fade, (size_t)Q)) ||
+            (Q > 1 && (rc = dev_alloc(&bm, (size_t)((Q - 1) * mat_len)))))
             break;
-        if (n_mat > 0 && (rc = dev_alloc(&ps->bm, (size_t)(n_mat * mat)))) break;
-        if (!all_ops.empty() && (rc = dev_alloc(&d_ops, all_ops.size()))) break;
-        if (hipMemcpy(ps->ell_c, ell_c.data(), sizeof(int) * ell_c.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(ps->ell_v, ell_v.data(), sizeof(double) * ell_v.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(ps->ov_rp, ov_rp.data(), sizeof(int) * ov_rp.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            (!ov_c.empty() &&
-             (hipMemcpy(ps->ov_c, ov_c.data(), sizeof(int) * ov_c.size(), hipMemcpyHostToDevice) != hipSuccess ||
-              hipMemcpy(ps->ov_v, ov_v.data(), sizeof(double) * ov_v.size(), hipMemcpyHostToDevice) != hipSuccess)) ||
-            hipMemcpy(ps->diag, dg.data(), sizeof(double) * dg.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(ps->near, nr.data(), sizeof(double) * nr.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        ps->bm = bm;
+        rc = CAP_ERR_HIP;
+        if (hipMemcpy(ps->at, at.data(), sizeof(int) * at.size(), hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(ps->first, first.data(), sizeof(uint2) * first.size(), hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(d_rows, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice) != hipSuccess)
+            break;
+        if (merged) {
+            if ((rc = dev_alloc(&d_rp, rp_host.size())) || (rc = dev_alloc(&d_ci, ci.size())) ||
+                (rc = dev_alloc(&d_v, v.size())))
+                break;
             rc = CAP_ERR_HIP;
-            break;
+            if (hipMemcpy(d_rp, rp_host.data(), sizeof(int) * rp_host.size(), hipMemcpyHostToDevice) != hipSuccess ||
+                hipMemcpy(d_ci, ci.data(), sizeof(int) * ci.size(), hipMemcpyHostToDevice) != hipSuccess ||
+                hipMemcpy(d_v, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
+                break;
+            fill_records<double>(d_rp, d_ci, d_v, d_rows, n_rec, ps, st);
+        } else if (p->vt == CAP_F64) {
+            fill_records<double>(p->rp, p->ci, (const double *)p->val, d_rows, n_rec, ps, st);
+        } else {
+            fill_records<float>(p->rp, p->ci, (const float *)p->val, d_rows, n_rec, ps, st);
         }
-        // V = D^{-1} C: the coupling columns as W / 64 64-RHS solves of the blocks
-        if ((rc = cap_batch_create(&b64, P, ro.data(), rpd.data(), cid.data(), vd.data(), CAP_F64, 64, &o, st)))
-            break;
-        if ((rc = dev_alloc(&rr, slab * slabs)) || (rc = dev_alloc(&vv, slab * slabs))) break;
-        if (hipMemsetAsync(rr, 0, slab * slabs * sizeof(double), st) != hipSuccess) {
-            rc = CAP_ERR_HIP;
-            break;
+        if (Q > 1) {
+            if (W == kPartWMax)
+                launch_part_sweep<kPartWMax, kPartSweepRhs, double, kPartUnit>(ps, n, nullptr, nullptr, bm, nullptr, W,
+                                                                               Q - 1, st);
+            else
+                launch_part_sweep<kPartW, kPartSweepRhs, double, kPartUnit>(ps, n, nullptr, nullptr, bm, nullptr, W,
+                                                                            Q - 1, st);
         }
-        if (p->vt == CAP_F64)
-            k_part_coupling<double><<<blocks_for(n), kBlock, 0, st>>>(p->rp, p->ci, (const double *)p->val, n, m, W, rr);
-        else
-            k_part_coupling<float><<<blocks_for(n), kBlock, 0, st>>>(p->rp, p->ci, (const float *)p->val, n, m, W, rr);
-        if (hipGetLastError() != hipSuccess) {
-            rc = CAP_ERR_HIP;
-            break;
-        }
-        for (size_t h = 0; h < slabs && rc == CAP_OK; ++h) rc = cap_batch_solve(b64, rr + h * slab, vv + h * slab, st);
-        if (rc != CAP_OK || (rc = cap_plan_status(b64->plan, st)) != CAP_OK) break;
-        k_part_transpose<<<blocks_for((long long)n * W), kBlock, 0, st>>>(vv, n, W, ps->vt);
-        if (Q > 1)
-            k_part_tail_matrix<<<blocks_for((long long)(Q - 1) * mat), kBlock, 0, st>>>(ps->vt, n, m, Q, W, ps->bm);
-        if (!all_ops.empty()) {
-            if (hipMemcpy(d_ops, all_ops.data(), sizeof(int3) * all_ops.size(), hipMemcpyHostToDevice) !=
-                hipSuccess) {
-                rc = CAP_ERR_HIP;
+        std::vector<double> one((size_t)Q), four((size_t)Q);
+        if ((rc = part_norms(bm, W, Q, one.data(), four.data(), st)) != CAP_OK) break;
+        double worst = 0.0;  // of four blocks in a row
+        for (int q = 4; q < Q; ++q) worst = four[(size_t)q] <= worst ? worst : four[(size_t)q];
+        bool finite = true;
+        for (int q = 1; q < Q; ++q) finite = finite && one[(size_t)q] < 0x1p1000 && four[(size_t)q] < 0x1p1000;
+        ps->walk = finite && (worst <= kPartDamp || Q <= kPartGroup);
+        if (!ps->walk && longer && worst < 0.0625 && n >= 16 * kPartLongest) {
+            const int rows_of = (int)std::ceil(m * 36.0 / -std::log2(worst));
+            if (rows_of <= kPartLongest) {
+                *longer = rows_of;
+                rc = CAP_ERR_UNSUPPORTED;
                 break;
             }
-            const unsigned quads = (unsigned)((W / 128) * (W / 128));
-            for (size_t l = 0; l < launches.size(); ++l) {
-                const dim3 grid((unsigned)launches[l].size(), quads);
-                if (W == kPartWMax)
-                    k_part_gemm<kPartWMax><<<grid, 256, 0, st>>>(d_ops + op_start[l], ps->bm);
-                else
-                    k_part_gemm<kPartW><<<grid, 256, 0, st>>>(d_ops + op_start[l], ps->bm);
-            }
         }
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) rc = CAP_ERR_HIP;
+        std::vector<uint2> fade((size_t)Q, make_uint2(0u, 0u));
+        auto log256 = [](double v) { return (unsigned)(int)std::ceil(256.0 * std::log2(std::max(v, 0x1p-1022))); };
+        for (int q = 1; q < Q && ps->walk; ++q) {
+            fade[(size_t)q].x = fade[(size_t)q - 1].x + log256(one[(size_t)q]);
+            if (q >= 4) fade[(size_t)q].y = fade[(size_t)q - 4].y + log256(four[(size_t)q]);
+        }
+        rc = CAP_ERR_HIP;
+        if (hipMemcpy(ps->fade, fade.data(), sizeof(uint2) * (size_t)Q, hipMemcpyHostToDevice) != hipSuccess) break;
+        rc = CAP_OK;
+        if (ps->walk) break;
+        // the scan's products, launch by launch (each list depends on the one
+        // before): the in-group products W_p = B_p W_{p-1} (W_first = B_first)
+        // for groups g >= 1, the carries' first-round matrices (the W of each
+        // group's last tail), then each carry round's products
+        std::vector<std::vector<int3>> launches;
+        for (int j = 0; j < gs; ++j) {
+            std::vector<int3> ops;
+            for (int g = 1; g * gs + j < Q; ++g) {
+                const int q = g * gs + j;
+                ops.push_back(j == 0 ? make_int3((int)(w_off + q - gs), q - 1, -1)
+                                     : make_int3((int)(w_off + q - gs), q - 1, (int)(w_off + q - 1 - gs)));
+            }
+            if (!ops.empty()) launches.push_back(ops);
+        }
+        {
+            std::vector<int3> ops;
+            for (int g = 1; g < G; ++g) {
+                const int last = std::min(Q, (g + 1) * gs) - 1;
+                ops.push_back(make_int3((int)(m_off[0] + g - 1), (int)(w_off + last - gs), -1));
+            }
+            if (!ops.empty()) launches.push_back(ops);
+        }
+        for (int r = 0; r + 1 < rounds; ++r) {
+            std::vector<int3> ops;
+            const int s = 1 << r;
+            for (int g = 2 * s; g < G; ++g)
+                ops.push_back(make_int3((int)(m_off[(size_t)r + 1] + g - 2 * s), (int)(m_off[(size_t)r] + g - s),
+                                        (int)(m_off[(size_t)r] + g - 2 * s)));
+            if (!ops.empty()) launches.push_back(ops);
+        }
+        std::vector<int3> all_ops;
+        std::vector<size_t> op_start;
+        for (const auto &l : launches) {
+            op_start.push_back(all_ops.size());
+            all_ops.insert(all_ops.end(), l.begin(), l.end());
+        }
+        if (all_ops.empty()) break;
+        // the same B_p, at the head of a larger set
+        if ((rc = dev_alloc(&ps->bm, (size_t)(n_mat * mat_len)))) break;
+        if ((rc = dev_alloc(&d_ops, all_ops.size()))) break;
+        rc = CAP_ERR_HIP;
+        if (hipMemcpy(ps->bm, bm, sizeof(double) * (size_t)((Q - 1) * mat_len), hipMemcpyDeviceToDevice) != hipSuccess ||
+            hipMemcpy(d_ops, all_ops.data(), sizeof(int3) * all_ops.size(), hipMemcpyHostToDevice) != hipSuccess)
+            break;
+        const unsigned quads = (unsigned)((W / 128) * (W / 128));
+        for (size_t l = 0; l < launches.size(); ++l) {
+            const dim3 grid((unsigned)launches[l].size(), quads);
+            if (W == kPartWMax)
+                k_part_gemm<kPartWMax><<<grid, 256, 0, st>>>(d_ops + op_start[l], ps->bm);
+            else
+                k_part_gemm<kPartW><<<grid, 256, 0, st>>>(d_ops + op_start[l], ps->bm);
+        }
+        if (hipGetLastError() == hipSuccess && hipStreamSynchronize(st) == hipSuccess) rc = CAP_OK;
     } while (0);
     (void)hipStreamSynchronize(st);
-    if (b64) cap_batch_destroy(b64);
-    for (double *t : {rr, vv})
+    for (void *t : {(void *)d_rows, (void *)d_rp, (void *)d_ci, (void *)d_v, (void *)d_ops})
         if (t) (void)hipFree(t);
-    if (d_ops) (void)hipFree(d_ops);
+    if (bm && bm != ps->bm) (void)hipFree(bm);
     // Accuracy check against the sequential solve.  The block solves and V
     // multiply by block inverses, which the sequential solve never forms;
     // when the blocks are not diagonally dominant their entries grow along a

@@ -169,40 +169,6 @@ struct StepStage {
     T v[E], d, r, bo[K];
 };
 
-// Loads and stores through buffer descriptors: a uniform byte offset in a
-// scalar register plus the thread's own 32-bit offset, so walking the tables
-// costs no vector instruction.  Reads past the descriptor's bytes give 0 and
-// writes there are dropped.
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-typedef unsigned Words4 __attribute__((ext_vector_type(4)));
-typedef unsigned Words2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ Rsrc make_rsrc(const void *p, unsigned bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ void load_value(Rsrc r, unsigned own, unsigned off, double *v)
-{
-    const Words2 w = __builtin_amdgcn_raw_buffer_load_b64(r, (int)own, (int)off, 0);
-    __builtin_memcpy(v, &w, 8);
-}
-__device__ __forceinline__ void load_value(Rsrc r, unsigned own, unsigned off, float *v)
-{
-    const unsigned w = __builtin_amdgcn_raw_buffer_load_b32(r, (int)own, (int)off, 0);
-    __builtin_memcpy(v, &w, 4);
-}
-__device__ __forceinline__ void store_value(Rsrc r, unsigned own, unsigned off, double v)
-{
-    Words2 w;
-    __builtin_memcpy(&w, &v, 8);
-    __builtin_amdgcn_raw_buffer_store_b64(w, r, (int)own, (int)off, 0);
-}
-__device__ __forceinline__ void store_value(Rsrc r, unsigned own, unsigned off, float v)
-{
-    unsigned w;
-    __builtin_memcpy(&w, &v, 4);
-    __builtin_amdgcn_raw_buffer_store_b32(w, r, (int)own, (int)off, 0);
-}
-
 // off: the step's first piece (uniform), t16 = 16 * thread, pb = 16 * block
 // bytes from piece to piece; row_bytes: the row's offset in b and x.
 template <typename T, int E, int K>
