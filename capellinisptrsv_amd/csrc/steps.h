@@ -21,6 +21,7 @@ struct StepTables {
     int vt = 0, E = 4, n_jobs = 0, block = 64, ring = 0, max_rhs = 1;
     int tallest = 0;  // rows of the largest matrix
     int cus = 256;    // compute units of the device
+    size_t lds = 0;   // bytes of LDS a workgroup may have
     bool long_rows = false;
     long long slots = 0;
     std::vector<StepJob> jobs;

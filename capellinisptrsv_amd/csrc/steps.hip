@@ -319,6 +319,166 @@ __global__ void __launch_bounds__(kStepBlock)
     }
 }
 
+// The same steps, for rows of up to 4 entries and one right-hand side, with
+// the loads in wavefronts of their own.  Issuing a step's loads is half of a
+// step's time where a wavefront does both (194 ns a step, 99 without its
+// loads), and a compute unit has room for more wavefronts.  Thread B + t loads
+// what thread t solves: its row data D steps ahead into registers, and two
+// steps ahead of the solve from there into one of two LDS buffers; thread t
+// reads its next step's data while it solves this one.  A head's unused word
+// carries the row's offset in b and x.  Both sides meet at the one barrier
+// per step.
+// What bounds it: with one solving wavefront its chain (107 ns a step, 159
+// with k_step: 24.6 against 34.1 us for n = 2,000 in 193 steps), with more
+// the LDS traffic of the steps' data too: 194 / 279 / 333 ns with two, three
+// and four (k_step 221 / 303 / 355; n = 100,000 in 807 steps 156 against 178
+// us).  With 8 or 16 entries a row the data through LDS costs more than its
+// loads (n = 68,170, 7 entries: 163 against 140 us; n = 60,000, 15 entries:
+// 231 against 212), and where there are more workgroups than compute units
+// the loads of one overlap the chains of the others: those keep k_step.
+constexpr int kSplitEntries = 4;
+constexpr int kSplitDepth = 10;
+
+template <typename T>
+constexpr int split_bytes()  // of a step's data in LDS, per thread
+{
+    return 16 * StepLayout<T, kSplitEntries>::P + (int)sizeof(T);
+}
+
+template <typename T, bool UNFUSED>
+__global__ void __launch_bounds__(2 * kStepBlock)
+    k_step_split(const StepJob *__restrict__ jobs, int n_jobs, const uint4 *__restrict__ tab,
+                 const unsigned *__restrict__ rows, const T *__restrict__ b, T *__restrict__ x, int k)
+{
+    constexpr int E = kSplitEntries, D = kSplitDepth;
+    typedef StepLayout<T, E> L;
+    const int which = blockIdx.z * gridDim.x + blockIdx.x;
+    if (which >= n_jobs) return;
+    const StepJob job = jobs[which];
+    const int q0 = blockIdx.y, B = job.block;
+    if ((int)threadIdx.x >= 2 * B) return;  // whole wavefronts; barriers count the others
+    typedef __attribute__((address_space(3))) T LdsVal;
+    typedef __attribute__((address_space(3))) Words4 LdsWords;
+    auto value = [](unsigned byte) -> LdsVal * { return (LdsVal *)byte; };
+    auto words = [](unsigned byte) -> LdsWords * { return (LdsWords *)byte; };
+    const bool loads = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >= B;
+    const unsigned t = loads ? threadIdx.x - B : threadIdx.x, pb = 16u * B;
+    // after the ring: two buffers of a step's pieces, then its values of b
+    const unsigned buf0 = ((unsigned)(job.ring + 1) * sizeof(T) + 15u) & ~15u, size = (unsigned)split_bytes<T>() * B;
+    const unsigned my_piece = buf0 + 16 * t, my_b = buf0 + L::P * pb + (unsigned)sizeof(T) * t;
+    const unsigned kb = (unsigned)(k * sizeof(T));
+    const unsigned span = (unsigned)job.rows_of * kb - q0 * (unsigned)sizeof(T);
+    const int total = (job.steps + 1) & ~1;  // the solving side unrolls by two
+    if (loads) {
+        const unsigned t16 = 16 * t, t4 = 4 * t;
+        const Rsrc rb = make_rsrc(b + (size_t)job.row0 * k + q0, span);
+        const unsigned step16 = 16u * L::P * B, step4 = 4u * B;
+        const Rsrc rt = make_rsrc(tab + job.tab, (unsigned)(job.steps + kStepTail) * step16);
+        const Rsrc rr = make_rsrc(rows + job.rows, (unsigned)(job.steps + kStepTail) * step4);
+        Words4 w[D][L::P];
+        T bo[D];
+        unsigned xo[D], ahead[D];
+        unsigned next = 0, nrow = 0;
+        auto fetch = [&](int d, unsigned row) {
+            xo[d] = __umul24(row, kb);
+#pragma unroll
+            for (int q = 0; q < L::P; ++q)
+                w[d][q] = __builtin_amdgcn_raw_buffer_load_b128(rt, (int)t16, (int)(next + q * pb), 0);
+            load_value(rb, xo[d], 0, &bo[d]);
+            next += step16;
+        };
+        auto fetch_row = [&](int d) {
+            ahead[d] = __builtin_amdgcn_raw_buffer_load_b32(rr, (int)t4, (int)nrow, 0);
+            nrow += step4;
+        };
+        auto pass_on = [&](int d, unsigned at) {  // into the buffer `at` bytes on, then the next step but D - 1
+            Words4 head = w[d][0];
+            head.y = xo[d];
+            *words(my_piece + at) = head;
+#pragma unroll
+            for (int q = 1; q < L::P; ++q) *words(my_piece + at + q * pb) = w[d][q];
+            *value(my_b + at) = bo[d];
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(d, ahead[d]);
+            fetch_row(d);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        unsigned first[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            first[d] = __builtin_amdgcn_raw_buffer_load_b32(rr, (int)t4, (int)nrow, 0);
+            nrow += step4;
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) fetch_row(d);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            fetch(d, first[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        pass_on(0, 0);
+        pass_on(1, size);
+        lds_barrier();
+        lds_barrier();  // step 0 is read
+        unsigned at = 0;
+        for (int s0 = 0; s0 < total; s0 += D) {
+#pragma unroll
+            for (int h = 0; h < D; ++h) {
+                if (s0 + h >= total) return;
+                pass_on((h + 2) % D, at);  // step s0 + h + 2
+                at = size - at;
+                lds_barrier();
+            }
+        }
+        return;
+    }
+    const Rsrc rx = make_rsrc(x + (size_t)job.row0 * k + q0, span);
+    if (t == 0) *value((unsigned)job.ring * sizeof(T)) = (T)0;
+    struct Step {
+        Words4 w[L::P];
+        T bo;
+    };
+    auto read = [&](Step &n, unsigned at) {
+#pragma unroll
+        for (int q = 0; q < L::P; ++q) n.w[q] = *words(my_piece + at + q * pb);
+        n.bo = *value(my_b + at);
+    };
+    auto slots = [&](const Step &n, unsigned (&at)[E]) {
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            const unsigned pair = u < 2 ? n.w[0].z : n.w[0].w;
+            at[u] = ((u & 1) ? pair >> 16 : pair & 0xffffu) * (unsigned)sizeof(T);
+        }
+    };
+    Step st[2];
+    unsigned at[E];
+    lds_barrier();
+    read(st[0], 0);
+    slots(st[0], at);
+    lds_barrier();
+    for (int s0 = 0; s0 < total; s0 += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const Step &w = st[h];
+            T xv[E], v[E], dr[16 / sizeof(T)], sum = (T)0;
+#pragma unroll
+            for (int u = 0; u < E; ++u) xv[u] = *value(at[u]);
+            __builtin_amdgcn_sched_barrier(0);
+            read(st[1 - h], (1 - h) * size);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_memcpy(v, &w.w[1], sizeof(v));
+            __builtin_memcpy(dr, &w.w[L::P - 1], 16);
+#pragma unroll
+            for (int u = 0; u < E; ++u) sum = UNFUSED ? sum + v[u] * xv[u] : fmac(v[u], xv[u], sum);
+            const T xi = step_divide(w.bo - sum, dr[0], dr[1]);
+            *value((w.w[0].x & 0xffffu) * (unsigned)sizeof(T)) = xi;
+            store_value(rx, w.w[0].y, 0, xi);
+            slots(st[1 - h], at);
+            lds_barrier();
+        }
+    }
+}
+
 // ----------------------------------------------------------- schedule
 namespace {
 
@@ -535,21 +695,32 @@ template <typename T, int E, bool LONG, int K>
 int launch_k(const StepTables *t, const T *b, T *x, int k, bool unfused, hipStream_t st, int allow_lds)
 {
     constexpr int D = step_depth<E, K>();
-    const size_t bytes = (size_t)(t->ring + 1) * K * sizeof(T);
-    auto go = [&](auto kernel) {
-        if (allow_lds) {  // once, when the tables are built
-            CAP_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, allow_lds));
-            return (int)CAP_OK;
-        }
-        const int group = std::min(t->n_jobs, kXcds);
-        const dim3 grid((unsigned)group, (unsigned)(k / K), (unsigned)((t->n_jobs + group - 1) / group));
-        kernel<<<grid, t->block, bytes, st>>>(t->d_jobs, t->n_jobs, t->tab, t->rows, t->ov_c, (const T *)t->ov_v, b, x,
-                                              k);
-        CAP_HIP_TRY(hipGetLastError());
-        return (int)CAP_OK;
+    const size_t ring = (size_t)(t->ring + 1) * K * sizeof(T);
+    const int group = std::min(t->n_jobs, kXcds);
+    const dim3 grid((unsigned)group, (unsigned)(k / K), (unsigned)((t->n_jobs + group - 1) / group));
+    auto allow = [&](auto kernel) {  // once, when the tables are built
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   allow_lds);
     };
-    return unfused ? go(k_step<T, E, D, true, LONG, K>) : go(k_step<T, E, D, false, LONG, K>);
+    if constexpr (K == 1 && E == kSplitEntries) {
+        auto kernel = unfused ? k_step_split<T, true> : k_step_split<T, false>;
+        const size_t bytes = (ring + 15) / 16 * 16 + 2 * (size_t)split_bytes<T>() * t->block;
+        if (allow_lds) {
+            CAP_HIP_TRY(allow(kernel));
+        } else if (bytes <= t->lds && (long long)t->n_jobs * k <= t->cus) {
+            kernel<<<grid, 2 * t->block, bytes, st>>>(t->d_jobs, t->n_jobs, t->tab, t->rows, b, x, k);
+            CAP_HIP_TRY(hipGetLastError());
+            return CAP_OK;
+        }
+    }
+    auto kernel = unfused ? k_step<T, E, D, true, LONG, K> : k_step<T, E, D, false, LONG, K>;
+    if (allow_lds) {
+        CAP_HIP_TRY(allow(kernel));
+        return CAP_OK;
+    }
+    kernel<<<grid, t->block, ring, st>>>(t->d_jobs, t->n_jobs, t->tab, t->rows, t->ov_c, (const T *)t->ov_v, b, x, k);
+    CAP_HIP_TRY(hipGetLastError());
+    return CAP_OK;
 }
 
 // Right-hand sides per thread for k of them: fewer mean more workgroups, each
@@ -615,6 +786,7 @@ int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<
     if (!t) return CAP_ERR_ALLOC;
     t->vt = vt;
     t->cus = std::max(1, cus);
+    t->lds = (size_t)std::max(0, lds_bytes);
     int rc;
     try {
         rc = build(t, rp, ci, mats, want_rhs, lds_bytes, pad_max);

@@ -137,3 +137,28 @@ def test_batch_steps_bit_exact(cuda, k, dtype, arith):
         out = torch.empty_like(bd)
         _replays(lambda: bt.solve(bd, out=out, stream=torch.cuda.current_stream()), out, x)
         bt.close()
+
+
+@pytest.mark.parametrize("dtype,bits", [(np.float64, np.uint64), (np.float32, np.uint32)])
+@pytest.mark.parametrize("n,width", [(1, 1), (2, 1), (9, 1), (10, 1), (11, 1), (12, 1), (13, 1), (21, 1), (640, 63),
+                                     (650, 65), (2000, 130), (3003, 250), (3000, 600)])
+def test_loads_in_their_own_wavefronts(cuda, n, width, dtype, bits):
+    """Up to 4 entries a row: step counts around the 10 steps that the loading
+    wavefronts are ahead, odd and even, and steps of one to four wavefronts
+    (rows of level l read level l - 1)."""
+    rng = np.random.default_rng(n)
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        first = i // width * width
+        if first:
+            ci += sorted(rng.choice(np.arange(first - width, first), size=min(width, 1 + i % 4), replace=False))
+        ci.append(i)
+        v += list(rng.uniform(-1, 1, len(ci) - 1 - rp[-1])) + [3.0]
+        rp.append(len(ci))
+    rp, ci, v = np.array(rp, np.int32), np.array(ci, np.int32), np.array(v).astype(dtype)
+    plan = _plan(cuda, rp, ci, v, algo="level")
+    b = api.uniform(6, n).astype(dtype)
+    for x in (_solve(plan, cuda, b) for _ in range(2)):
+        ref = oracle.csr_forward(rp, ci, v, b, rhs=1, fused=True)
+        assert np.array_equal(x.view(bits), ref.view(bits))
+    plan.close()
