@@ -2505,7 +2505,18 @@ int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st
                                      p->norms);
     };
     const bool small = block == kBlockSmall;
-    if (block == kBlockLarge)
+    if (hop_takes(p, rhs)) {
+        const HopTab tab{p->hop->base, p->hop->ex, p->hop->npad};
+        auto look = [&](auto kernel) {
+            kernel<<<nb, block, 0, st>>>(tab, val, b, x, pr, sc, p->n, p->ticket, p->norms);
+        };
+        if (p->hop->E == 2)
+            small ? look(k_refine_hop<2, kBlockSmall>) : look(k_refine_hop<2, kBlock>);
+        else if (p->hop->E == 3)
+            small ? look(k_refine_hop<3, kBlockSmall>) : look(k_refine_hop<3, kBlock>);
+        else
+            small ? look(k_refine_hop<4, kBlockSmall>) : look(k_refine_hop<4, kBlock>);
+    } else if (block == kBlockLarge)
         go(k_refine2<0, kBlockLarge>);
     else if (p->lds)
         small ? go(k_refine2<1, kBlockSmall>) : go(k_refine2<1, kBlock>);

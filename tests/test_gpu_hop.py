@@ -141,3 +141,26 @@ def test_hop_refusals_and_replay(cuda):
     _replays(lambda: plan.solve(b, out=out, stream=torch.cuda.current_stream()), out, eager)
     assert plan.status() == 0
     plan.close()
+
+
+@pytest.mark.parametrize("threads", [128, 256])
+@pytest.mark.parametrize("name,mat", MATS, ids=[m[0] for m in MATS])
+def test_refined_sweep_bit_exact(cuda, name, mat, threads):
+    """The refinement's first two steps over the same tables: the oracle's
+    two-step result bit for bit (a looked-through row's pair is worked out
+    again with the row's own operations)."""
+    import torch
+    rp, ci, v = mat
+    n = len(rp) - 1
+    plan = _plan(cuda, rp, ci, v, algo="hop", row_threads=threads)
+    b = api.uniform(9, n)
+    _, _, want = oracle.refine2(rp, ci, v, b, rhs=1, rcp=True)
+    bt = torch.from_numpy(b).to(cuda)
+    out = torch.empty_like(bt)
+    for rep in range(2):  # the second call replays the captured graph
+        x, iters, rel = plan.solve_refined(bt, tol=1e-9, out=out)
+        torch.cuda.synchronize()
+        assert plan.status() == 0
+        assert iters == 2, (rep, iters, rel)
+        assert np.array_equal(x.cpu().numpy(), want), rep
+    plan.close()
