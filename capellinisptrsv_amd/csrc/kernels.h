@@ -981,6 +981,15 @@ __device__ __forceinline__ void block_max_to(unsigned long long v, unsigned long
     }
 }
 
+// The two norms into the host's memory, then the count they belong to.
+__global__ void k_echo(const unsigned long long *__restrict__ norms, unsigned long long *echo, unsigned long long count)
+{
+    if (threadIdx.x != 0) return;
+    __hip_atomic_store(echo, norms[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(echo + 1, norms[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(echo + 2, count, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------ fused refinement sweep
 // The first two steps of mixed-precision refinement in one dependency sweep.
 // Row i computes, from the pairs (x0_j, d_j) of its dependencies j:

@@ -190,6 +190,9 @@ struct cap_plan_s {
     unsigned long long *pair = nullptr;  // fused refinement pairs when readiness is in place
     long long pair_len = 0;
     unsigned long long *norms = nullptr;  // inside ctrl
+    // the norms for the host: pinned memory, two norms and the count of the
+    // read they belong to
+    unsigned long long *echo = nullptr, echoes = 0;
     hipGraphExec_t refine_graph = nullptr;
     const void *graph_b = nullptr;
     void *graph_x = nullptr;
@@ -450,6 +453,10 @@ void plan_free(cap_plan p)
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (p->refine_graph) (void)hipGraphExecDestroy(p->refine_graph);
+    if (p->echo) {
+        (void)hipDeviceSynchronize();
+        (void)hipHostFree(p->echo);
+    }
     delete p;
 }
 
@@ -1754,33 +1761,37 @@ int build_hop(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci
     for (int i = 0; i < n; ++i) most = std::max(most, rp[i + 1] - 1 - rp[i]);
     if (n < 1 || most > kHopMax) return CAP_ERR_UNSUPPORTED;
     const int E = std::max(2, most);
-    std::vector<int> hop, look, order;  // look: the hop a looked-through row is ready in
+    struct Ready {
+        int hop, look;  // look: the hop in which all the row's entries are there, were it looked through
+    };
+    std::vector<Ready> at_row;
+    std::vector<int> order;
     std::vector<unsigned char> bits;
     int hops = 0;
     try {
-        hop.resize((size_t)n);
-        look.resize((size_t)n);
+        at_row.resize((size_t)n);
         order.resize((size_t)n);
         bits.resize((size_t)n);
         for (int i = 0; i < n; ++i) {
-            const int lo = rp[i], hi = rp[i + 1] - 1;
-            int ready = 0, newest = 0;
-            for (int j = lo; j < hi; ++j) {
-                newest = std::max(newest, hop[(size_t)ci[j]]);
-                ready = std::max(ready, std::min(hop[(size_t)ci[j]], look[(size_t)ci[j]]));
+            const int lo = rp[i], cnt = rp[i + 1] - 1 - lo;
+            int ready = 0, newest = 0, of[kHopMax];
+            for (int j = 0; j < cnt; ++j) {
+                const Ready e = at_row[(size_t)ci[(size_t)(lo + j)]];
+                of[j] = e.hop;
+                newest = std::max(newest, e.hop);
+                ready = std::max(ready, std::min(e.hop, e.look));
             }
             unsigned m = 0;
-            for (int j = lo; j < hi; ++j) m |= (unsigned)(hop[(size_t)ci[j]] > ready) << (j - lo);
-            hop[(size_t)i] = ready + 1;
-            look[(size_t)i] = newest;
+            for (int j = 0; j < cnt; ++j) m |= (unsigned)(of[j] > ready) << j;
+            at_row[(size_t)i] = Ready{ready + 1, newest};
             bits[(size_t)i] = (unsigned char)m;
             hops = std::max(hops, ready + 1);
         }
         // rows in hop order, by index within a hop
         std::vector<int> at((size_t)hops + 2, 0);
-        for (int i = 0; i < n; ++i) ++at[(size_t)hop[(size_t)i] + 1];
+        for (int i = 0; i < n; ++i) ++at[(size_t)at_row[(size_t)i].hop + 1];
         for (int h = 0; h <= hops; ++h) at[(size_t)h + 1] += at[(size_t)h];
-        for (int i = 0; i < n; ++i) order[(size_t)at[(size_t)hop[(size_t)i]]++] = i;
+        for (int i = 0; i < n; ++i) order[(size_t)at[(size_t)at_row[(size_t)i].hop]++] = i;
     } catch (const std::bad_alloc &) {
         return CAP_ERR_ALLOC;
     }
@@ -2526,6 +2537,31 @@ int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st
     return CAP_OK;
 }
 
+// The refinement norms, once everything before on `st` is done.  A kernel
+// writes them into pinned memory with a count, which the host watches for: a
+// refined solve of n = 1,000,000 takes 102.5 us, and 118.7 with a copy to the
+// stack and a stream synchronization.  After 2 ms the host waits for the
+// stream.
+int read_norms(cap_plan p, unsigned long long *nb, hipStream_t st)
+{
+    if (!p->echo) {
+        CAP_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&p->echo), 64, hipHostMallocDefault));
+        std::memset(p->echo, 0, 64);  // memory of a freed plan's counts may come back
+    }
+    const unsigned long long count = ++p->echoes;
+    k_echo<<<1, kWave, 0, st>>>(p->norms, p->echo, count);
+    CAP_HIP_TRY(hipGetLastError());
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    while (__atomic_load_n(p->echo + 2, __ATOMIC_ACQUIRE) != count) {
+        if (std::chrono::steady_clock::now() < until) continue;
+        CAP_HIP_TRY(hipStreamSynchronize(st));
+        break;
+    }
+    nb[0] = p->echo[0];
+    nb[1] = p->echo[1];
+    return CAP_OK;
+}
+
 // One refinement step on `st`: r32 = b - L x (or b when first), d = L32^{-1} r32
 // in FP32 (value protocol), x += d; norms[0] = max|d| bits, norms[1] = max|x|.
 int refine_step(cap_plan p, const double *b, double *x, int rhs, bool first, hipStream_t st)
@@ -2611,8 +2647,7 @@ int refined_partition(cap_plan p, const double *b, double *x, int k, double tol,
         CAP_HIP_TRY(hipGetLastError());
         ++it;
         unsigned long long nbits[2];
-        CAP_HIP_TRY(hipMemcpyAsync(nbits, p->norms, sizeof(nbits), hipMemcpyDeviceToHost, st));
-        CAP_HIP_TRY(hipStreamSynchronize(st));
+        CAP_TRY(read_norms(p, nbits, st));
         double dmax, xmax;
         std::memcpy(&dmax, &nbits[0], 8);
         std::memcpy(&xmax, &nbits[1], 8);
@@ -2692,8 +2727,7 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
     if (join) CAP_TRY(join_parts(join, st));
     it = 2;
     while (true) {
-        CAP_HIP_TRY(hipMemcpyAsync(nb, p->norms, sizeof(nb), hipMemcpyDeviceToHost, st));
-        CAP_HIP_TRY(hipStreamSynchronize(st));
+        CAP_TRY(read_norms(p, nb, st));
         double dmax, xmax;
         std::memcpy(&dmax, &nb[0], 8);
         std::memcpy(&xmax, &nb[1], 8);
