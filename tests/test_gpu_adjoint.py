@@ -121,3 +121,37 @@ def test_adjoint_finite_differences_n1m(cuda):
         fd = dloss(plan.solve(bp), plan.solve(bm)) / (2 * h)
         an = float(gb[i])
         assert abs(fd - an) <= 1e-5 * max(1.0, abs(an)), (i, fd, an)
+
+
+def _hubs(n, hubs, seed):
+    """Rows of up to 3 entries, and columns that many further rows read."""
+    rp, ci, v = random_lower(n, max_off=2, band=300, seed=seed)
+    rng = np.random.default_rng(seed)
+    rows = [list(zip(ci[rp[i]:rp[i + 1]], v[rp[i]:rp[i + 1]])) for i in range(n)]
+    for col, many in hubs:
+        for r in rng.choice(np.arange(col + 1, n), size=many, replace=False):
+            rows[r].insert(0, (col, rng.uniform(-0.1, 0.1)))
+    rp = np.r_[0, np.cumsum([len(r) for r in rows])].astype(np.int32)
+    flat = [e for r in rows for e in r]
+    return rp, np.array([c for c, _ in flat], np.int32), np.array([w for _, w in flat])
+
+
+@pytest.mark.parametrize("n,hubs", [(1, []), (64, []), (257, [(3, 6)]), (5000, [(10, 50), (2000, 9), (2001, 5),
+                                                                            (2002, 8), (4990, 4)]),
+                                    (30_000, [(c, 1 + c % 14) for c in range(5, 29_000, 40)])])
+def test_value_gradients_bit_exact(cuda, n, hubs):
+    """The oracle's backward order bit for bit, and the value gradients of
+    rows that start and end anywhere in a workgroup's 256 rows."""
+    import torch
+    rp, ci, v = _hubs(n, hubs, seed=n)
+    plan = _plan(cuda, rp, ci, v, adjoint="gather")[0]
+    b, g = api.uniform(1, n), api.uniform(2, n)
+    x = plan.solve(torch.from_numpy(b).to(cuda))
+    for _ in range(2):
+        gb, gv = plan.adjoint(torch.from_numpy(g).to(cuda), x)
+        torch.cuda.synchronize()
+        assert plan.status() == 0
+        y = oracle.adjoint(rp, ci, v, g, fused=True)
+        assert np.array_equal(gb.cpu().numpy(), y)
+        assert np.array_equal(gv.cpu().numpy(), oracle.grad_val(rp, ci, y, oracle.csr_forward(rp, ci, v, b, fused=True)))
+    plan.close()
