@@ -1285,14 +1285,19 @@ void apply_choice(cap_plan p, const TuneChoice &c)
 // read and more damping in each.  Blocks that damp too little to be walked
 // are made longer, up to kPartLongest rows, when that is enough (n = 200,000,
 // bandwidth 128, 13 entries a row: 640 rows and the scan 107 us, 720 rows and
-// the walk 72, 1440 rows 96).  A matrix whose blocks grow (refused at that
-// size) is tried with the smallest.
+// the walk 72, 1440 rows 96).  The blocks' number is brought down to a whole
+// multiple of the compute units where that takes a quarter more rows at most,
+// as the last round of workgroups is as long as a full one: n = 140,000, 274
+// or 256 blocks: 63 and 59 us, with 8 right-hand sides 112 and 87; half as
+// many rows again did not pay (n = 200,000, 391 or 256 blocks: 66 and 74).  A
+// matrix whose blocks grow (refused at that size) is tried with the smallest.
 // The host groups the rows into records; the records are filled, the B_p
 // swept and the scan's matrices formed on the device.
 constexpr int kPartBlocks = 1024;
 constexpr int kPartRows = 512;
 constexpr int kPartSpread = 500;
 constexpr int kPartLongest = 1280;
+constexpr int kPartCus = 256;
 // largest relative max-norm difference from the sequential solve accepted
 // when the tables are checked at plan creation (the FP64 bar is 1e-12)
 constexpr double kPartStableTol = 1e-13;
@@ -1357,7 +1362,13 @@ int build_partition(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
         }
         const int W = w <= kPartW ? kPartW : kPartWMax;
         const int least = std::max(W, (n + kPartBlocks - 1) / kPartBlocks);
-        const int m = std::max(least, std::min(std::max(kPartRows, n / kPartSpread), (n + 15) / 16));
+        int m = std::max(least, std::min(std::max(kPartRows, n / kPartSpread), (n + 15) / 16));
+        // whole rounds of the compute units, where a quarter more rows give them
+        const int rounds = n / m / kPartCus;
+        if (rounds > 0 && n / m % kPartCus > 0) {
+            const int even = (n + rounds * kPartCus - 1) / (rounds * kPartCus);
+            if (even <= m + m / 4) m = std::max(m, even);
+        }
         int longer = 0;
         int rc = build_partition_tables(p, mat, w, m, merged, &longer, st);
         if (longer > 0) rc = build_partition_tables(p, mat, w, longer, merged, nullptr, st);
