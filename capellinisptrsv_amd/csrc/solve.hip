@@ -1278,8 +1278,9 @@ void apply_choice(cap_plan p, const TuneChoice &c)
 // plans whose lower bandwidth is at most kPartWMax and that split into at
 // least two blocks; CAP_ERR_UNSUPPORTED otherwise.  The tail width W is 128
 // when the bandwidth allows, else 256.  Blocks hold at least W and n /
-// kPartBlocks rows, and more, kPartRows or n / kPartSpread, where that leaves
-// 16 blocks: a sweep takes about 0.2 us per 8 rows of a block, 14 us for 512
+// kPartBlocks rows, and more, kPartRows (twice that at W = 256, whose matrices
+// are four times the bytes: n = 158,094, 16 right-hand sides 640 -> 277 us) or
+// n / kPartSpread, where that leaves 16 blocks: a sweep takes about 0.2 us per 8 rows of a block, 14 us for 512
 // rows, and its bytes take 0.1 us per 1000 rows of the matrix, so up to n /
 // kPartSpread rows cost nothing, while fewer blocks are fewer matrices to
 // read and more damping in each.  Blocks that damp too little to be walked
@@ -1362,7 +1363,7 @@ int build_partition(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
         }
         const int W = w <= kPartW ? kPartW : kPartWMax;
         const int least = std::max(W, (n + kPartBlocks - 1) / kPartBlocks);
-        int m = std::max(least, std::min(std::max(kPartRows, n / kPartSpread), (n + 15) / 16));
+        int m = std::max(least, std::min(std::max(kPartRows * (W / kPartW), n / kPartSpread), (n + 15) / 16));
         // whole rounds of the compute units, where a quarter more rows give them
         const int rounds = n / m / kPartCus;
         if (rounds > 0 && n / m % kPartCus > 0) {
@@ -2500,7 +2501,11 @@ int ensure_refine(cap_plan p, int rhs, hipStream_t st)
 // the pair array (staged: the readiness array; else the plan's own) reset
 // with the tickets, then the thread-per-row launch with the plan's grid,
 // LDS window and batch schedule.
-int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st)
+// join (hybrid batches): side streams that end before the sweep starts.  Its
+// persistent workgroups need a compute unit each: started while others still
+// hold some, two of them shared one for all of the sweep (256 matrices, 16
+// right-hand sides: sweep 9.55 ms instead of 9.25).
+int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st, const Fork *join = nullptr)
 {
     typedef unsigned long long U;
     const long long len = (long long)p->n * rhs;
@@ -2510,6 +2515,7 @@ int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st
     const unsigned nbp = std::max(1u, std::min(blocks_for(len), 2048u));
     k_prepare_norms<U><<<nbp, kBlock, 0, st>>>(pr, len, VBits<double>::kSentinel, p->ticket, kTickets, p->norms);
     CAP_HIP_TRY(hipGetLastError());
+    if (join) CAP_TRY(join_parts(join, st));
     if (p->n == 0) return CAP_OK;
     const int l = lpr_log2_for(rhs);
     // the sweep's own sizes: 128 or 256 threads, or 1024 for a batch that
@@ -2676,10 +2682,11 @@ int refined_partition(cap_plan p, const double *b, double *x, int k, double tol,
     return rc;
 }
 
-// join (hybrid batches): side streams whose partitioned solves run
-// alongside the first two steps, which touch only the plan's scheduled rows;
-// they are joined into st before the convergence readback, since the later
-// steps read and update every row of x.
+// join (hybrid batches): side streams whose partitioned solves run beside the
+// fused sweep's reset (or the first two steps, which touch only the plan's
+// scheduled rows); they are joined into st before the sweep, at the latest
+// before the convergence readback, since the later steps read and update
+// every row of x.
 int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, int max_iter, int *iters,
                  double *last_rel, hipStream_t st, const Fork *join = nullptr)
 {
@@ -2703,8 +2710,12 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
         p->refine_graph = nullptr;
     }
     // The first two steps (solve from b, one correction) are one graph:
-    // captured once per (b, x, rhs), replayed on later calls.
-    if (!p->refine_graph || p->graph_b != b || p->graph_x != x || p->graph_rhs != rhs) {
+    // captured once per (b, x, rhs), replayed on later calls; with side
+    // streams to join, two launches.
+    const bool plain = fused && join;
+    if (plain) {
+        CAP_TRY(refine_fused(p, b, x, rhs, st, join));
+    } else if (!p->refine_graph || p->graph_b != b || p->graph_x != x || p->graph_rhs != rhs) {
         if (p->refine_graph) CAP_HIP_TRY(hipGraphExecDestroy(p->refine_graph));
         p->refine_graph = nullptr;
         hipStream_t cs;
@@ -2734,7 +2745,7 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
     int it = 0;
     unsigned long long nb[2];
     int rc = CAP_OK;
-    CAP_HIP_TRY(hipGraphLaunch(p->refine_graph, st));
+    if (!plain) CAP_HIP_TRY(hipGraphLaunch(p->refine_graph, st));
     if (join) CAP_TRY(join_parts(join, st));
     it = 2;
     while (true) {
