@@ -60,7 +60,7 @@ extern "C" {
                               resolved inside one compute unit: deep matrices
                               (few rows per level); value protocol on x itself */
 #define CAP_ALGO_PARTITION 6 /* lower bandwidth <= 256: row blocks solved
-                              independently, joined by a scan over the block
+                              independently, joined through the block
                               tails of W = 128 values (bandwidth <= 128) or
                               256 (FP64 tables built at plan creation;
                               FP32 plans widen b and round x once); sums are
@@ -71,9 +71,9 @@ extern "C" {
                               which waits for the device); the refined solve
                               uses FP64 partitioned solves (no FP32 tables)
                               with one FP64 correction. */
-#define CAP_ALGO_LEVEL 7     /* one workgroup walks the levels: a level's rows
-                              in parallel (thread per row, steps of 64 to 256
-                              rows, the workgroup size chosen by the plan),
+#define CAP_ALGO_LEVEL 7     /* one workgroup walks steps of rows whose
+                              dependencies earlier steps solved (thread per
+                              row, 64 to 256 rows a step, chosen by the plan),
                               a workgroup barrier between steps, values in an
                               LDS ring; no polling.  Needs every dependency
                               within a ring of <= 64 KiB of the newest row of
