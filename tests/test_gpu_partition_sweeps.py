@@ -147,4 +147,18 @@ def test_one_nonzero_row(cuda, name):
             assert 0.5 * w <= a <= 2.0 * w, lo
             far = lo
     assert far > 2000
+    # beside others, dense ones and ones with nonzeros elsewhere: the same bits
+    beside = np.zeros((n, 8))
+    beside[:, 2] = beside[:, 7] = api.uniform(52, n)
+    beside[[n // 2, n // 2 + 300, n - 5], 3] = 1.0
+    beside[5, 4] = 1e-200
+    for at, col in ((0, 0), (6, 0), (1, 1)):
+        beside[100 + col, at] = 1.0
+    xs = plan.solve(torch.from_numpy(beside).to(cuda)).cpu().numpy()
+    assert np.array_equal(xs[:, 0], x) and np.array_equal(xs[:, 6], x)
+    for q in range(8):
+        alone = plan.solve(torch.from_numpy(beside[:, q].copy()).to(cuda)).cpu().numpy()
+        assert np.array_equal(xs[:, q], alone), q
+        ref = oracle.csr_forward(*mat, beside[:, q].copy(), fused=True)
+        assert rel_maxnorm(xs[:, q], ref) <= FP64_TOL, q
     plan.close()
