@@ -201,7 +201,7 @@ struct cap_plan_s {
     struct PartState *part = nullptr;
     // steps in one workgroup (CAP_ALGO_LEVEL).  lvl_rhs: right-hand sides per
     // solve an explicit plan takes (1, 2 or 4; 0: any).  lvl_live: the tables
-    // take the caller's values again on every solve
+    // take the caller's values again on every solve (autotuned plans)
     StepTables *lvl = nullptr;
     int lvl_rhs = 0;
     bool lvl_live = false;
@@ -1745,20 +1745,20 @@ int level_accepts(cap_plan p, const std::vector<int> &rp, const std::vector<int>
     return CAP_OK;
 }
 
-// The plan's step tables.  An explicit plan is held to level_accepts.  An
-// autotuned plan whose matrix that rule refuses, over the caller's own
-// values, copies them into the tables again on every solve (about 10 us):
-// the kernels it would run otherwise read them there.
+// The plan's step tables.  An explicit plan is held to level_accepts and
+// keeps the values of its creation.  An autotuned plan over the caller's own
+// values copies them into the tables again on every solve (6 us at n = 2,000,
+// 8 at n = 100,000): the kernels it would run otherwise read them there, and
+// which of them wins is a matter of microseconds.
 int build_level(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, bool explicit_algo, hipStream_t st)
 {
-    int rule_rhs = 0;
-    const int rule = level_accepts(p, rp, ci, &rule_rhs);
-    if (explicit_algo && rule != CAP_OK) return rule;
+    int rhs = 0;
+    if (explicit_algo) CAP_TRY(level_accepts(p, rp, ci, &rhs));
     free_level(p);
-    CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rule_rhs : 4, p->lds_max,
-                        kStepPadMax, p->rp, p->ci, p->val, st));
-    p->lvl_rhs = explicit_algo ? rule_rhs : 0;
-    p->lvl_live = rule != CAP_OK && !p->owns_matrix;
+    CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rhs : 4, p->lds_max, kStepPadMax,
+                        p->rp, p->ci, p->val, st));
+    p->lvl_rhs = rhs;
+    p->lvl_live = !explicit_algo && !p->owns_matrix;
     return CAP_OK;
 }
 

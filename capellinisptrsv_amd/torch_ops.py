@@ -38,7 +38,10 @@ class Plan:
 
     row_ptr/col_idx: int32 CUDA tensors; values: float64/float32 CUDA tensor.
     The plan keeps references to the three tensors (their memory is used in
-    place).  algo: auto|wrtfst|twopart|mix|csc|local|partition|level|hop; sync:
+    place).  Values changed in place reach the next solve, except where the
+    plan holds tables of them: partition (also as auto's pick, see info()),
+    algo="level", upper and unit_diagonal plans keep the values of creation,
+    the gather adjoint and solve_refined those of their first call.  algo: auto|wrtfst|twopart|mix|csc|local|partition|level|hop; sync:
     auto|value|flag.
     row_threads: 128 or 256 threads per workgroup of the thread-per-row
     kernels (0: tuned with algo auto, else 256).

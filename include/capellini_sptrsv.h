@@ -204,6 +204,11 @@ void cap_opts_default(cap_opts *o);
  * the plan keeps the caller's device pointers (they must outlive the plan);
  * with host_inputs = 1 it copies them to the device.  Analysis (validation,
  * the mix chunk table, the CSC in-degree) runs once at creation.
+ * Values changed in place behind the kept pointer reach the next solve,
+ * except where a plan holds tables of them: CAP_ALGO_PARTITION (explicit or
+ * AUTO's pick, cap_plan_info) and explicit CAP_ALGO_LEVEL plans, upper or
+ * unit-diagonal ones, and host inputs solve with the values of plan creation;
+ * the gather adjoint and refined solves keep those of their first call.
  * cap_plan_solve is asynchronous on `stream`; b and x are device pointers of
  * n*rhs values interleaved as x[i*rhs + k] (serialref.h:57-60 layout). */
 typedef struct cap_plan_s *cap_plan;

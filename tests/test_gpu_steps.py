@@ -68,6 +68,40 @@ def test_autotuned_steps_read_the_callers_values(cuda):
     plan.close()
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_autotuned_steps_read_values_where_the_rule_accepts(cuda, dtype):
+    """The same on bands that explicit level plans take, for every number of
+    right-hand sides, and through the module whose values an optimizer
+    changes."""
+    import torch
+    from capellinisptrsv_amd import Plan
+    from capellinisptrsv_amd.torch_ops import TriangularSolve
+    rp, ci, v = api.generate("band", n=5000, offdiag=8, band=400, seed=23)  # beyond the partition's bandwidth
+    v = v.astype(dtype)
+    n = len(rp) - 1
+    _plan(cuda, rp, ci, v, algo="level").close()  # accepted
+    d = [torch.from_numpy(a).to(cuda) for a in (rp, ci, v)]
+    plan = Plan(*d)
+    assert plan.info()["algo"] == "level"
+    module = TriangularSolve(d[0], d[1], d[2].clone())
+    assert module.plan.info()["algo"] == "level"
+    scale = 1.0
+    for _ in range(2):
+        vs = v * dtype(scale)
+        for k in (1, 2, 3, 8):
+            b = api.uniform(30 + k, n * k).astype(dtype).reshape(n, k) if k > 1 else api.uniform(30, n).astype(dtype)
+            ref = oracle.csr_forward(rp, ci, vs, b.reshape(-1), rhs=k, fused=True)
+            assert np.array_equal(_solve(plan, cuda, b).reshape(-1), ref), (scale, k)
+        x = module(torch.from_numpy(b[:, 0].copy()).to(cuda))
+        ref = oracle.csr_forward(rp, ci, vs, b[:, 0].copy(), fused=True)
+        assert np.array_equal(x.detach().cpu().numpy(), ref), scale
+        d[2].mul_(0.75)
+        with torch.no_grad():
+            module.values.mul_(0.75)
+        scale *= 0.75
+    plan.close()
+
+
 @pytest.mark.parametrize("dtype,bits,span", [(np.float64, np.uint64, 620), (np.float32, np.uint32, 80)])
 def test_step_division_range(cuda, dtype, bits, span):
     """Diagonals and right-hand sides over powers of two beyond both ends of
