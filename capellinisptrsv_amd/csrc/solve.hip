@@ -1144,6 +1144,20 @@ unsigned long long fingerprint(const std::vector<int> &rp, const std::vector<int
     return h;
 }
 
+// The right-hand side candidates are timed on: all ones.  The dependency
+// structure sets most kernels' time, but a partitioned solve of b = 0 has no
+// tails to join: n = 2,000, bandwidth 250: under 36 us, and 67 with a dense b,
+// against 36 by steps.
+int tuning_rhs(cap_plan p, void *b, long long count, hipStream_t st)
+{
+    const unsigned nb = std::max(1u, std::min(blocks_for(count), 2048u));
+    if (p->vt == CAP_F64)
+        k_fill<unsigned long long><<<nb, kBlock, 0, st>>>((unsigned long long *)b, count, 0x3FF0000000000000ULL);
+    else
+        k_fill<unsigned><<<nb, kBlock, 0, st>>>((unsigned *)b, count, 0x3F800000u);
+    return hipGetLastError() == hipSuccess ? CAP_OK : CAP_ERR_HIP;
+}
+
 // Best of three timed solves after one warm-up; stops early once a run is
 // 1.5x slower than `bound` (the best candidate so far).
 int time_candidate(cap_plan p, int algo, int sync, const void *b, void *x, int rhs, hipStream_t st, float bound,
@@ -1838,13 +1852,12 @@ int build_hop(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci
     return rc;
 }
 
-// Candidates are timed on the plan's own matrix (b = 0; the dependency
-// structure, not the values, sets the time) and the fastest is cached per
-// matrix shape: thread-per-row with and without the LDS window, at 1 or 2
-// workgroups per CU, with the staged or the in-place readiness array, the
-// flag protocol, and mix at three thresholds when the rows are long enough
-// for wavefront mode to matter.  A plan created with readiness in place keeps
-// it in every candidate.
+// Candidates are timed on the plan's own matrix (b = 1, tuning_rhs) and the
+// fastest is cached per matrix shape: thread-per-row with and without the LDS
+// window, at 1 or 2 workgroups per CU, with the staged or the in-place
+// readiness array, the flag protocol, and mix at three thresholds when the
+// rows are long enough for wavefront mode to matter.  A plan created with
+// readiness in place keeps it in every candidate.
 int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int> &ci, hipStream_t st)
 {
     const int levels = p->n ? cap_matrix_layer(p->n, rp_host.data(), ci.data(), nullptr, nullptr, nullptr) : 1;
@@ -1868,7 +1881,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
     void *b = nullptr, *x = nullptr;
     CAP_HIP_TRY(hipMalloc(&b, (size_t)p->n * p->vbytes + 8));
     CAP_HIP_TRY(hipMalloc(&x, (size_t)p->n * p->vbytes + 8));
-    CAP_HIP_TRY(hipMemsetAsync(b, 0, (size_t)p->n * p->vbytes, st));
+    CAP_TRY(tuning_rhs(p, b, p->n, st));
     const int stg = p->staged;
     constexpr int B = kBlock, S = kBlockSmall;
     std::vector<TuneChoice> cands = {{CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, 0, stg, B},
@@ -2853,7 +2866,7 @@ int batch_refine_rows(cap_plan p, int k) { return refine_block(p, k) >> lpr_log2
 
 // A batch runs either the scheduled thread-per-row kernel over all matrices
 // or one workgroup per matrix; unless the caller named one, both are timed
-// on the batch itself (b = 0) and the faster is kept.  Unless the caller set
+// on the batch itself (b = 1) and the faster is kept.  Unless the caller set
 // blocks_per_cu, the thread-per-row grid is timed at 1, 2 and 4 workgroups
 // per compute unit (the schedule's pace depends on how many blocks are in
 // flight); a size must be 2% faster than a smaller one to win.
@@ -2872,7 +2885,7 @@ int choose_batch_algo(cap_plan p, int requested, int bpc_fixed, int k, const std
         (void)hipFree(b);
         return CAP_ERR_ALLOC;
     }
-    int rc = hipMemsetAsync(b, 0, bytes, st) == hipSuccess ? CAP_OK : CAP_ERR_HIP;
+    int rc = tuning_rhs(p, b, (long long)p->n * k, st);
     float t_w = 1e30f, t_l = 1e30f;
     int best_bpc = p->bpc;
     std::vector<int> sizes = {1, 2, 4};
@@ -3031,7 +3044,7 @@ int choose_batch_steps(cap_plan p, int k, const std::vector<int> &ro, const std:
     const size_t bytes = (size_t)p->n * k * p->vbytes + 8;
     void *b = nullptr, *x = nullptr;
     if (hipMalloc(&b, bytes) != hipSuccess || hipMalloc(&x, bytes) != hipSuccess ||
-        hipMemsetAsync(b, 0, bytes, st) != hipSuccess)
+        tuning_rhs(p, b, (long long)p->n * k, st) != CAP_OK)
         rc = CAP_ERR_ALLOC;
     float plain = 0, with = 0;
     if (rc == CAP_OK) plain = time_batch(p, parts, lo, k, b, x, st, &rc, fk);
@@ -3056,7 +3069,7 @@ int choose_batch_steps(cap_plan p, int k, const std::vector<int> &ro, const std:
 // rows are handed out (one ticket atomic per block, ~12 ns each), so its
 // thread-per-row shape is timed again: 1, 2 and 4 workgroups of 256 threads
 // per CU, and 1024-thread workgroups with 1, 2 or 4 right-hand sides per
-// lane, each over a schedule without the partitioned matrices (b = 0).  The
+// lane, each over a schedule without the partitioned matrices.  The
 // fastest hybrid is kept when 2 % faster than the plain batch as it
 // resolved (thread-per-row or one workgroup per matrix).  The kept plans go
 // to *parts.  With several right-hand sides the rest is also timed with
@@ -3126,7 +3139,7 @@ int choose_batch_hybrid(cap_plan p, int k, bool bpc_fixed, const std::vector<int
     const size_t bytes = (size_t)p->n * k * p->vbytes + 8;
     void *b = nullptr, *x = nullptr;
     if (hipMalloc(&b, bytes) != hipSuccess || hipMalloc(&x, bytes) != hipSuccess ||
-        hipMemsetAsync(b, 0, bytes, st) != hipSuccess)
+        tuning_rhs(p, b, (long long)p->n * k, st) != CAP_OK)
         rc = CAP_ERR_ALLOC;
     struct Shape {
         int bpc, block, rpl;
