@@ -1852,6 +1852,15 @@ int build_hop(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci
     return rc;
 }
 
+// The partition keeps the values of plan creation, the other candidates read
+// the caller's on every solve.  Over the caller's own values it is the pick
+// only where it takes less than half their time: matrices of short chains
+// (n = 20,000, bandwidth 120, 89 levels: 45 us, 51 by look-through) stay with a
+// kernel that follows the values.  Bands that explicit level plans take are
+// compared as they are: long chains of narrow levels, where only the steps,
+// which held the values too until they were made to follow them, come near.
+constexpr float kPartLiveFactor = 2.0f;
+
 // Candidates are timed on the plan's own matrix (b = 1, tuning_rhs) and the
 // fastest is cached per matrix shape: thread-per-row with and without the LDS
 // window, at 1 or 2 workgroups per CU, with the staged or the in-place
@@ -1901,6 +1910,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
     for (int lds : {0, 1})
         for (int blk : {B, S}) cands.push_back({CAP_ALGO_WRTFST, CAP_SYNC_VALUE, 0, 1, lds, stg, blk, 1});
     const double avg = (double)p->nnz / std::max(1, p->n);
+    float part_factor = 1.0f;
     // one workgroup per matrix pays off only with few rows per level
     {
         // timed first: on such matrices it sets a low bound that lets the
@@ -1909,8 +1919,11 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             cands.insert(cands.begin(), {CAP_ALGO_LOCAL, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
             // deep and narrow-banded: the partitioned solve, timed before all
             // (reassociated sums: not a candidate in the reference arithmetic)
-            if (!p->unfused && build_partition(p, rp_host, st) == CAP_OK)
+            if (!p->unfused && build_partition(p, rp_host, st) == CAP_OK) {
                 cands.insert(cands.begin(), {CAP_ALGO_PARTITION, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
+                int rhs = 0;
+                if (!p->owns_matrix && level_accepts(p, rp_host, ci, &rhs) != CAP_OK) part_factor = kPartLiveFactor;
+            }
         }
         // steps in one workgroup, where the ring and the padding allow: up to
         // a few thousand rows per level a step per 256 rows can still beat a
@@ -1940,6 +1953,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
         if (c.algo == CAP_ALGO_LOCAL && (rc = ensure_segments(p, nullptr)) != CAP_OK) break;
         float t = 0;
         if ((rc = time_candidate(p, c.algo, c.sync, b, x, 1, st, best, &t)) != CAP_OK) break;
+        if (c.algo == CAP_ALGO_PARTITION) t *= part_factor;
         // a later (less preferred) candidate must be 2% faster to win, so
         // near-ties resolve the same way from run to run
         if (t < (pick_set ? 0.98f : 1.0f) * best) {

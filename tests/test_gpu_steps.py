@@ -102,6 +102,21 @@ def test_autotuned_steps_read_values_where_the_rule_accepts(cuda, dtype):
     plan.close()
 
 
+def test_autotuned_short_chains_follow_the_callers_values(cuda):
+    """The partition holds the values of plan creation: on short chains, where
+    it wins by little, auto keeps a kernel that reads them."""
+    import torch
+    from capellinisptrsv_amd import Plan
+    rp, ci, v = api.generate("band_rowcount", n=20000, offdiag=3, band=120, seed=20120)  # 89 levels
+    d = [torch.from_numpy(a).to(cuda) for a in (rp, ci, v)]
+    plan = Plan(*d)
+    assert plan.info()["algo"] != "partition"
+    d[2].mul_(0.75)
+    b = api.uniform(7, 20000)
+    assert np.array_equal(_solve(plan, cuda, b), oracle.csr_forward(rp, ci, v * 0.75, b, fused=True))
+    plan.close()
+
+
 def test_autotuned_pick_is_timed_with_a_dense_right_hand_side(cuda):
     """A partitioned solve of b = 0 has no tails to join and takes half of
     what a dense b does (67 us here, against 36 by steps)."""
