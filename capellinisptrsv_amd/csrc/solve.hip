@@ -331,6 +331,7 @@ int dev_alloc(P **p, size_t count)
     *p = nullptr;
     if (count == 0) count = 1;
     if (hipMalloc((void **)p, count * sizeof(P)) != hipSuccess) {
+        (void)hipGetLastError();  // not for the next launch's check: callers may go on without
         *p = nullptr;
         return CAP_ERR_ALLOC;
     }
@@ -1113,16 +1114,17 @@ int ensure_csc(cap_plan p, hipStream_t st)
 
 // ----------------------------------------------------------- autotuner
 // A pick is cached per matrix shape: size, value type, readiness, the
-// dependency depth (level count) and a hash of sampled row pointers and
-// column indices.  Two matrices with one row-length profile but different
+// dependency depth (level count), whether the plan owns the values (steps
+// over the caller's copy them on every solve) and a hash of sampled row
+// pointers and column indices.  Two matrices with one row-length profile but different
 // dependencies (a chain and a wide-level matrix) never share a pick.
 struct TuneKey {
-    int n, nnz, vt, staged, unfused, count_polls, levels;
+    int n, nnz, vt, staged, unfused, count_polls, levels, owned;
     unsigned long long fp;
     bool operator<(const TuneKey &o) const
     {
-        return std::tie(n, nnz, vt, staged, unfused, count_polls, levels, fp) <
-               std::tie(o.n, o.nnz, o.vt, o.staged, o.unfused, o.count_polls, o.levels, o.fp);
+        return std::tie(n, nnz, vt, staged, unfused, count_polls, levels, owned, fp) <
+               std::tie(o.n, o.nnz, o.vt, o.staged, o.unfused, o.count_polls, o.levels, o.owned, o.fp);
     }
 };
 std::mutex g_tune_mu;
@@ -1870,21 +1872,27 @@ constexpr float kPartLiveFactor = 2.0f;
 int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int> &ci, hipStream_t st)
 {
     const int levels = p->n ? cap_matrix_layer(p->n, rp_host.data(), ci.data(), nullptr, nullptr, nullptr) : 1;
-    const TuneKey key{p->n, p->nnz, p->vt, p->staged, p->unfused, p->count_polls, levels, fingerprint(rp_host, ci)};
+    const TuneKey key{p->n,           p->nnz,         p->vt,  p->staged,
+                      p->unfused,     p->count_polls, levels, p->owns_matrix,
+                      fingerprint(rp_host, ci)};
     {
         std::lock_guard<std::mutex> g(g_tune_mu);
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
-            apply_choice(p, it->second);
-            if (p->algo == CAP_ALGO_MIX) return build_mix(p, rp_host, it->second.border);
-            if (p->algo == CAP_ALGO_LOCAL) return ensure_segments(p, nullptr);
-            if (p->algo == CAP_ALGO_LEVEL) return build_level(p, rp_host, ci, false, st);
-            if (it->second.hop) return build_hop(p, rp_host, ci, st);
-            if (p->algo != CAP_ALGO_PARTITION) return CAP_OK;
-            // the pick was cached for this structure; these values may not
-            // keep the partition stable, and then the plan is tuned afresh
-            const int rc = build_partition(p, rp_host, st);
-            if (rc != CAP_ERR_UNSUPPORTED) return rc;
+            const TuneChoice &c = it->second;
+            apply_choice(p, c);
+            int rc = CAP_OK;
+            if (c.algo == CAP_ALGO_MIX) rc = build_mix(p, rp_host, c.border);
+            else if (c.algo == CAP_ALGO_LOCAL) rc = ensure_segments(p, nullptr);
+            else if (c.algo == CAP_ALGO_LEVEL) rc = build_level(p, rp_host, ci, false, st);
+            else if (c.algo == CAP_ALGO_PARTITION) rc = build_partition(p, rp_host, st);
+            else if (c.hop) rc = build_hop(p, rp_host, ci, st);
+            // The key samples the pattern: this matrix may have a row too long
+            // for the look-through tables or reach beyond the steps' ring, its
+            // values may not keep the partition stable, its tables may not
+            // fit.  Then it is tuned afresh.
+            if (rc != CAP_ERR_UNSUPPORTED && rc != CAP_ERR_ALLOC) return rc;
+            p->staged = key.staged;
         }
     }
     void *b = nullptr, *x = nullptr;

@@ -799,6 +799,7 @@ int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<
     if (rc == CAP_OK) rc = fill_any(t, d_rp, d_ci, d_val, false, st);
     if (rc == CAP_OK && hipStreamSynchronize(st) != hipSuccess) rc = CAP_ERR_HIP;
     if (rc != CAP_OK) {
+        (void)hipGetLastError();  // not for the next launch's check: callers go on without the tables
         steps_free(t);
         return rc;
     }

@@ -164,3 +164,64 @@ def test_refined_sweep_bit_exact(cuda, name, mat, threads):
         assert iters == 2, (rep, iters, rel)
         assert np.array_equal(x.cpu().numpy(), want), rep
     plan.close()
+
+
+def _same_samples(a, b):
+    """Equal in what the autotuner's cache key holds of the pattern."""
+    at = [[(len(x) - 1) * s // 256 for s in range(257)] for x in a[:2]]
+    return (all(len(x) == len(y) and np.array_equal(x[i], y[i]) for x, y, i in zip(a, b, at)) and
+            oracle.row_levels(len(a[0]) - 1, *a[:2]).max() == oracle.row_levels(len(b[0]) - 1, *b[:2]).max())
+
+
+def _longer_row(rp, ci, v):
+    """Four neighbouring rows of two entries each become rows of 5, 1, 1, 1."""
+    n = len(rp) - 1
+    used = {(n) * s // 256 for s in range(257)}
+    for i in range(n // 2, n - 4):
+        if (np.diff(rp[i:i + 5]) == 3).all() and not used & set(range(i, i + 5)):
+            rows = [list(ci[rp[r]:rp[r + 1] - 1]) for r in range(i, i + 4)]
+            five = sorted(rows[0] + rows[1][1:] + rows[2][1:] + rows[3][1:])
+            new = [five + [i]] + [[rows[t][0], i + t] for t in (1, 2, 3)]
+            rp2, ci2 = rp.copy(), ci.copy()
+            ci2[rp[i]:rp[i + 4]] = np.concatenate(new)
+            rp2[i + 1:i + 5] = rp[i] + np.cumsum([len(r) for r in new])
+            v2 = v.copy()
+            v2[rp2[i + 1:i + 5] - 1] = 6.0
+            if five[-1] < i and len(set(five)) == 5 and _same_samples((rp, ci, v), (rp2, ci2, v2)):
+                return rp2, ci2, v2
+    raise AssertionError("no place found")
+
+
+def _far_column(rp, ci, v):
+    """One entry of a row in the last tenth moves to the first column."""
+    n = len(rp) - 1
+    for i in range(n * 9 // 10, n):
+        if rp[i + 1] - rp[i] == 4:
+            ci2 = ci.copy()
+            ci2[rp[i]] = 0
+            if _same_samples((rp, ci, v), (rp, ci2, v)):
+                return rp, ci2, v
+    raise AssertionError("no place found")
+
+
+@pytest.mark.parametrize("kind", ["hop", "level"])
+def test_cached_pick_that_does_not_fit_is_tuned_afresh(cuda, kind):
+    """The autotuner's cache knows a pattern by samples: a matrix with a row
+    too long for the look-through tables, or with an entry beyond the steps'
+    ring, may be taken for one that has neither."""
+    if kind == "hop":
+        first = api.generate("level", n=100_000, levels=20, width=5000, depth=3, offdiag=2, seed=31)
+        second = _longer_row(*first)
+        assert np.diff(first[0]).max() == 3 and np.diff(second[0]).max() == 6
+    else:
+        first = api.generate("band", n=100_000, offdiag=3, band=1000, seed=32)
+        second = _far_column(*first)
+    n = len(first[0]) - 1
+    b = api.uniform(26, n)
+    plan = _plan(cuda, *first)
+    assert plan.hops() > 0 if kind == "hop" else plan.info()["algo"] == "level"
+    for m in (second, first):
+        other = _plan(cuda, *m)
+        assert np.array_equal(_run(other, cuda, b), oracle.csr_forward(*m, b, fused=True))
+        other.close()
+    plan.close()
