@@ -42,6 +42,14 @@ namespace {
 constexpr int kMixWideLevel = 200;    // rows per level from which levels count as wide
 constexpr int kMixBorderWide = 4;     // threshold where they are
 constexpr int kMixBorderNarrow = 32;  // threshold where they are not
+// Workgroups of mix per CU, whatever cap_opts.blocks_per_cu says.  Two of 1024
+// threads fill all 32 wave slots of a CU, 524,288 polling lanes on the chip,
+// and in FP32 without row tiles a 777,001-row wide-level matrix then made no
+// progress for the whole wait limit (10 s), as a batch of thread-per-row
+// workgroups once did at 8 per CU, the same number of lanes.  By tickets
+// alone either must progress; why polls starve there is not known.  Where two
+// did run they gave nothing: 268 us against 270 (row tiles).
+constexpr int kMixBlocks = 1;
 inline int mix_border_for(int n, int levels)
 {
     return (long long)n >= (long long)kMixWideLevel * std::max(1, levels) ? kMixBorderWide : kMixBorderNarrow;
@@ -963,7 +971,8 @@ int launch_kernel(cap_plan p, int algo, int sync, const T *val, const T *b, T *x
     } else if (algo == CAP_ALGO_MIX) {
         if (rhs != 1) return CAP_ERR_UNSUPPORTED;
         constexpr int kMixBlock = 1024;  // 16 units per ticket share an LDS window
-        const unsigned nb = grid_for(p, ((long long)p->n_units * kWave + kMixBlock - 1) / kMixBlock);
+        const unsigned nb = std::min(grid_for(p, ((long long)p->n_units * kWave + kMixBlock - 1) / kMixBlock),
+                                     (unsigned)(p->ncu * kMixBlocks));
         if (sync == CAP_SYNC_VALUE && p->tile)
             k_mix<T, 1, kMixBlock, true><<<nb, kMixBlock, 0, st>>>(p->rp, p->ci, val, b, x, sc, p->unit,
                                                                    p->n_units, p->ticket);
@@ -1940,15 +1949,11 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             cands.insert(cands.begin(), {CAP_ALGO_LEVEL, CAP_SYNC_VALUE, 0, 1, 0, 0, B});
     }
     // thresholds 4 and 32 (see mix_border_for) always; 16 where the mean row
-    // length is at least 4 (some chunks may then reach it).  One workgroup per
-    // CU: two of its 1024-thread workgroups fill every wave slot, and in FP32,
-    // where they do fit, the untiled kernel on a 777,001-row wide-level matrix
-    // stalled until its waits gave up (10 s of plan creation); with row tiles
-    // two gave 268 us against one's 270.
+    // length is at least 4 (some chunks may then reach it)
     for (int bd : {kMixBorderWide, 16, kMixBorderNarrow})
         if (bd != 16 || avg * 4 >= bd) {
-            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 1, 0, stg, B});
-            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, 1, 0, stg, B, 1});
+            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, kMixBlocks, 0, stg, B});
+            cands.push_back({CAP_ALGO_MIX, CAP_SYNC_VALUE, bd, kMixBlocks, 0, stg, B, 1});
         }
     float best = 1e30f;
     TuneChoice pick = cands[0];
@@ -2435,7 +2440,7 @@ int cap_plan_tuning(cap_plan p, int *blocks_per_cu, int *lds_window, int *adjoin
 {
     if (!p) return CAP_ERR_ARG;
     if (row_tiles) *row_tiles = p->tile;
-    if (blocks_per_cu) *blocks_per_cu = p->bpc;
+    if (blocks_per_cu) *blocks_per_cu = p->algo == CAP_ALGO_MIX ? kMixBlocks : p->bpc;
     if (row_threads) *row_threads = p->algo == CAP_ALGO_LEVEL && p->lvl ? p->lvl->block : p->wblock;
     if (lds_window) *lds_window = p->lds;
     if (adjoint) *adjoint = p->adjoint_mode;

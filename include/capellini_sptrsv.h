@@ -156,7 +156,8 @@ typedef struct cap_opts {
                          (0 = no count bound, the default; the wall-time
                          bound below still applies) */
     int blocks_per_cu; /* persistent grid size in workgroups per compute unit
-                          (0 = tuned / default 1; at most 4) */
+                          (0 = tuned / default 1; at most 4; CAP_ALGO_MIX,
+                          whose workgroups have 1024 threads, runs one) */
     int adjoint;       /* CAP_ADJOINT_* (0 = gather) */
     int lds_window;    /* 1 = thread-per-row kernels resolve dependencies on
                           rows of their own workgroup in LDS (value protocol) */

@@ -217,6 +217,24 @@ def test_mix_row_tiles_bit_exact(cuda, border, name, mat):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("bpc", [2, 4])
+def test_mix_runs_one_workgroup_per_cu(cuda, bpc, dtype):
+    """Two of mix's 1024-thread workgroups on every CU stalled: a plan asked
+    for more runs one, and says so."""
+    import torch
+    from capellinisptrsv_amd import Plan
+    rp, ci, v = MATS[2][1]
+    v = v.astype(dtype)
+    b = api.uniform(4, len(rp) - 1).astype(dtype)
+    plan = Plan(*(torch.from_numpy(a).to(cuda) for a in (rp, ci, v)), algo="mix", blocks_per_cu=bpc)
+    assert plan.info()["blocks_per_cu"] == 1
+    x = plan.solve(torch.from_numpy(b).to(cuda)).cpu().numpy()
+    assert plan.status() == 0
+    plan.close()
+    assert np.array_equal(x, oracle.csr_forward(rp, ci, v, b, fused=True))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("name,mat", [MATS[0], MATS[3], MATS[4], MATS[5]],
                          ids=["band", "cfg1_small", "cfg2_small", "chain"])
 def test_row_tiles_1024_threads_bit_exact(cuda, name, mat, dtype):
