@@ -230,11 +230,11 @@ inline bool hop_takes(const cap_plan_s *p, int rhs)
 
 // Right-hand-side counts a plan's steps solve: an explicit level plan's 1,
 // and 2 or 4 where its rule allows; any of an autotuned one's.
-inline bool level_takes(const cap_plan_s *p, int rhs)
+inline bool level_allows(const cap_plan_s *p, int rhs)
 {
-    if (!steps_take(p->lvl, rhs)) return false;
     return p->lvl_rhs == 0 || rhs == 1 || ((rhs == 2 || rhs == 4) && rhs <= p->lvl_rhs);
 }
+inline bool level_takes(const cap_plan_s *p, int rhs) { return steps_take(p->lvl, rhs) && level_allows(p, rhs); }
 
 // Side streams of a hybrid batch: its partitioned matrices' solves run
 // concurrently with each other (and with the rest's reset), forked from and
@@ -1050,9 +1050,12 @@ int reset_t(cap_plan p, int algo, int sync, void *x, int rhs, hipStream_t st)
 // The algorithm and protocol that solve rhs right-hand sides: the plan's,
 // except that an autotuned plan whose pick has no multi-RHS form (mix,
 // two-part, CSC, level steps) solves several with the write-first kernel in the value
-// protocol (its RHS block tuned like any other).
+// protocol (its RHS block tuned like any other).  So do level plans whose b
+// and x are more bytes than the steps address.
 inline int algo_for(cap_plan p, int rhs)
 {
+    if (p->algo == CAP_ALGO_LEVEL && level_allows(p, rhs) && !steps_take(p->lvl, rhs) && rhs >= 1 && rhs <= kWave)
+        return CAP_ALGO_WRTFST;
     if (rhs > 1 && p->auto_algo &&
         (p->algo == CAP_ALGO_MIX || p->algo == CAP_ALGO_TWOPART || p->algo == CAP_ALGO_CSC ||
          (p->algo == CAP_ALGO_LEVEL && !level_takes(p, rhs))))
@@ -1732,6 +1735,8 @@ constexpr int kLevelPadMax = 4;
 // level a step still costs a third of what the one-workgroup kernel spends
 // on them one by one.
 constexpr int kStepPadMax = 16;
+// Largest step tables a plan or batch makes without being asked for them.
+constexpr double kStepMaxBytes = 4.0 * (1ull << 30);
 
 int level_accepts(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, int *max_rhs)
 {
@@ -1762,7 +1767,9 @@ int level_accepts(cap_plan p, const std::vector<int> &rp, const std::vector<int>
     const long long full = steps_for(B);
     for (int cand = B - kWave; cand >= kWave; cand -= kWave)
         if (steps_for(cand) <= full + full / 8) B = cand;
-    if (steps_for(B) * B > std::max((long long)kLevelPadMax * n, 1LL << 16)) return CAP_ERR_UNSUPPORTED;
+    const long long slots = steps_for(B) * B;
+    if (slots > std::max((long long)kLevelPadMax * n, 1LL << 16)) return CAP_ERR_UNSUPPORTED;
+    if (slots * (maxoff <= 4 ? 4 : 8) > INT32_MAX) return CAP_ERR_UNSUPPORTED;
     *max_rhs = maxoff > 4                              ? 1
                : (R + 2) * 4 * vb <= (long long)p->lds_max ? 4
                : (R + 2) * 2 * vb <= (long long)p->lds_max ? 2
@@ -1781,7 +1788,7 @@ int build_level(cap_plan p, const std::vector<int> &rp, const std::vector<int> &
     if (explicit_algo) CAP_TRY(level_accepts(p, rp, ci, &rhs));
     free_level(p);
     CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rhs : 4, p->lds_max, kStepPadMax,
-                        p->rp, p->ci, p->val, st));
+                        explicit_algo ? HUGE_VAL : kStepMaxBytes, p->rp, p->ci, p->val, st));
     p->lvl_rhs = rhs;
     p->lvl_live = !explicit_algo && !p->owns_matrix;
     return CAP_OK;
@@ -3061,7 +3068,7 @@ int choose_batch_steps(cap_plan p, int k, const std::vector<int> &ro, const std:
             mats.push_back(make_int2(ro[m], ro[m + 1]));
     if (mats.empty()) return CAP_OK;
     StepTables *t = nullptr;
-    int rc = steps_build(&t, rp, ci, mats, p->vt, 4, p->lds_max, kStepPadMax, p->rp, p->ci, p->val, st);
+    int rc = steps_build(&t, rp, ci, mats, p->vt, 4, p->lds_max, kStepPadMax, kStepMaxBytes, p->rp, p->ci, p->val, st);
     if (rc == CAP_ERR_UNSUPPORTED || rc == CAP_ERR_ALLOC) return CAP_OK;  // the plain batch stays
     if (rc != CAP_OK) return rc;
     if (!steps_take(t, k)) {

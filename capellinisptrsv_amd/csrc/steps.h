@@ -39,10 +39,11 @@ struct StepTables {
 // sides a thread should solve (4, 2 or 1); fewer where the ring does not
 // fit lds_bytes (max_rhs says how many).  CAP_ERR_UNSUPPORTED when a matrix's
 // dependencies reach further back than any ring, or its steps would be mostly
-// padding (more than pad_max slots per row).
+// padding (more than pad_max slots per row), or the tables more than
+// max_bytes.
 int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<int> &ci,
-                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, const int *d_rp,
-                const int *d_ci, const void *d_val, hipStream_t st);
+                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, double max_bytes,
+                const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st);
 // Copies the values into the tables again (they changed in place).
 int steps_refresh(const StepTables *t, const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st);
 // Solves k right-hand sides (interleaved, row * k + q), 1, 2 or 4 of them per

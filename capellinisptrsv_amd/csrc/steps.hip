@@ -245,7 +245,12 @@ __global__ void __launch_bounds__(kStepBlock)
     const unsigned span = (unsigned)job.rows_of * kb - q0 * (unsigned)sizeof(T);
     const Rsrc rb = make_rsrc(b + (size_t)job.row0 * k + q0, span), rx = make_rsrc(x + (size_t)job.row0 * k + q0, span);
     const unsigned step16 = 16u * L::P * B, step4 = 4u * B;
-    const Rsrc rt = make_rsrc(tab + job.tab, (unsigned)(job.steps + kStepTail) * step16);
+    // a window of the pieces, moved with the steps: they may be more bytes
+    // than a descriptor holds
+    auto window = [&](int step) {
+        return make_rsrc(tab + uniform((long long)(job.tab + (unsigned long long)step * (L::P * B))), 3 * D * step16);
+    };
+    Rsrc rt = window(0);
     const Rsrc rr = make_rsrc(rows + job.rows, (unsigned)(job.steps + kStepTail) * step4);
     auto row_at = [&](unsigned off) { return __builtin_amdgcn_raw_buffer_load_b32(rr, (int)t4, (int)off, 0); };
     StepStage<T, E, K> st[D];
@@ -255,17 +260,19 @@ __global__ void __launch_bounds__(kStepBlock)
 #pragma unroll
     for (int r = 0; r < D; ++r) ahead[r] = row_at((D + r) * step4);
 #pragma unroll
-    for (int r = 0; r < D; ++r) step_load<T, E, K>(st[r], rt, r * step16, t16, pb, rb, __umul24(first[r], kb));
+    for (int r = 0; r < D; ++r) step_load<T, E, K>(st[r], rt, r * step16, t16, pb, rb, first[r] * kb);
     if (t == 0) *ring((unsigned)job.ring * kSlot) = Vals(0);
     unsigned at[E];
 #pragma unroll
     for (int u = 0; u < E; ++u) at[u] = ((u & 1) ? st[0].c[u / 2] >> 16 : st[0].c[u / 2] & 0xffffu) * kSlot;
     lds_barrier();
-    unsigned next = D * step16, nrow = 2 * D * step4;  // pieces of step s + D, rows of step s + 2D
+    unsigned nrow = 2 * D * step4;  // rows of step s + 2D
     // two rounds of the D stages per iteration: the compiler's load-counter
     // waits are exact in the second round (the first round's, merged at the
     // loop head, assume about half the loads in flight)
     for (int s0 = 0; s0 < job.steps; s0 += 2 * D) {
+        rt = window(s0);
+        unsigned next = D * step16;  // pieces of step s + D
 #pragma unroll
         for (int h = 0; h < 2 * D; ++h) {
             constexpr int kD = D;
@@ -306,7 +313,7 @@ __global__ void __launch_bounds__(kStepBlock)
             // parks in-flight load results in accumulation registers, and
             // each such move waits for its load
             __builtin_amdgcn_sched_barrier(0);
-            step_load<T, E, K>(w, rt, next, t16, pb, rb, __umul24(ahead[h % kD], kb));
+            step_load<T, E, K>(w, rt, next, t16, pb, rb, ahead[h % kD] * kb);
             ahead[h % kD] = row_at(nrow);
             next += step16;
             nrow += step4;
@@ -373,14 +380,18 @@ __global__ void __launch_bounds__(2 * kStepBlock)
         const unsigned t16 = 16 * t, t4 = 4 * t;
         const Rsrc rb = make_rsrc(b + (size_t)job.row0 * k + q0, span);
         const unsigned step16 = 16u * L::P * B, step4 = 4u * B;
-        const Rsrc rt = make_rsrc(tab + job.tab, (unsigned)(job.steps + kStepTail) * step16);
+        auto window = [&](int step) {  // see k_step
+            return make_rsrc(tab + uniform((long long)(job.tab + (unsigned long long)step * (L::P * B))),
+                             (2 * D + 2) * step16);
+        };
+        Rsrc rt = window(0);
         const Rsrc rr = make_rsrc(rows + job.rows, (unsigned)(job.steps + kStepTail) * step4);
         Words4 w[D][L::P];
         T bo[D];
         unsigned xo[D], ahead[D];
         unsigned next = 0, nrow = 0;
         auto fetch = [&](int d, unsigned row) {
-            xo[d] = __umul24(row, kb);
+            xo[d] = row * kb;
 #pragma unroll
             for (int q = 0; q < L::P; ++q)
                 w[d][q] = __builtin_amdgcn_raw_buffer_load_b128(rt, (int)t16, (int)(next + q * pb), 0);
@@ -422,6 +433,8 @@ __global__ void __launch_bounds__(2 * kStepBlock)
         lds_barrier();  // step 0 is read
         unsigned at = 0;
         for (int s0 = 0; s0 < total; s0 += D) {
+            rt = window(s0);
+            next = (D + 2) * step16;  // step s0 + D + 2
 #pragma unroll
             for (int h = 0; h < D; ++h) {
                 if (s0 + h >= total) return;
@@ -583,10 +596,8 @@ int fill_any(const StepTables *t, const int *d_rp, const int *d_ci, const void *
                             : fill_tables_t<float>(t, d_rp, d_ci, d_val, values_only, st);
 }
 
-constexpr double kStepMaxBytes = 4.0 * (1ull << 30);
-
 int build(StepTables *t, const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<int2> &mats,
-          int want_rhs, int lds_bytes, int pad_max)
+          int want_rhs, int lds_bytes, int pad_max, double max_bytes)
 {
     const int vb = t->vt == CAP_F64 ? 8 : 4;
     int longest = 0, reach = 0, tallest = 0;
@@ -599,7 +610,7 @@ int build(StepTables *t, const std::vector<int> &rp, const std::vector<int> &ci,
             for (int j = rp[(size_t)i]; j < rp[(size_t)i + 1] - 1; ++j) reach = std::max(reach, i - ci[(size_t)j]);
         }
     }
-    if (tallest < 1 || tallest >= 1 << 24 || mats.size() > 65535) return CAP_ERR_UNSUPPORTED;  // 24-bit row offsets
+    if (tallest < 1 || mats.size() > 65535) return CAP_ERR_UNSUPPORTED;
     t->tallest = tallest;
     t->E = longest <= 4 ? 4 : longest <= 8 ? 8 : 16;
     t->long_rows = longest > t->E;
@@ -668,7 +679,8 @@ int build(StepTables *t, const std::vector<int> &rp, const std::vector<int> &ci,
         t->jobs.push_back(StepJob{(unsigned long long)pieces, (unsigned)first, steps, R, B, lo, n});
         pieces += (long long)count * P;
         t->block = std::max(t->block, B);
-        if (rows.size() > (size_t)INT32_MAX || (double)pieces * 16 > kStepMaxBytes) return CAP_ERR_UNSUPPORTED;
+        // a job's row table is addressed by 32-bit byte offsets
+        if (rows.size() >= (size_t)1 << 30 || (double)pieces * 16 > max_bytes) return CAP_ERR_UNSUPPORTED;
     }
     if (t->jobs.empty() || padded > std::max((long long)pad_max * total, 1LL << 16)) return CAP_ERR_UNSUPPORTED;
     // the longest chains start first
@@ -775,8 +787,8 @@ int launch_any(const StepTables *t, const void *b, void *x, int k, bool unfused,
 }  // namespace
 
 int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<int> &ci,
-                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, const int *d_rp,
-                const int *d_ci, const void *d_val, hipStream_t st)
+                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, double max_bytes,
+                const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st)
 {
     *out = nullptr;
     int dev = 0, cus = 0;
@@ -789,7 +801,7 @@ int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<
     t->lds = (size_t)std::max(0, lds_bytes);
     int rc;
     try {
-        rc = build(t, rp, ci, mats, want_rhs, lds_bytes, pad_max);
+        rc = build(t, rp, ci, mats, want_rhs, lds_bytes, pad_max, max_bytes);
     } catch (const std::bad_alloc &) {
         rc = CAP_ERR_ALLOC;
     }

@@ -82,9 +82,12 @@ extern "C" {
                               1 right-hand side per solve, or 2 or 4 when
                               rows hold at most 4 off-diagonals and the wider
                               ring fits LDS; bit-exact (the
-                              thread-per-row sum order).  Timed by algo AUTO
-                              with the few-rows-per-level candidates; its
-                              refined solves use the write-first kernels. */
+                              thread-per-row sum order).  b and x of 4 GiB or
+                              more go through CAP_ALGO_WRTFST.  Timed by algo
+                              AUTO with the few-rows-per-level candidates
+                              (tables up to 4 GiB, any number of right-hand
+                              sides); its refined solves use the write-first
+                              kernels. */
 
 #define CAP_ALGO_HOP 8       /* the thread-per-row write-first solve with
                               look-through tables: a row whose dependency is

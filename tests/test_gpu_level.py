@@ -276,3 +276,23 @@ def test_level_several_rhs_reference_arith_and_autotuned(cuda):
         for q in range(k):
             assert np.array_equal(x[:, q], oracle.csr_forward(rp, ci, v, bk[:, q].copy(), fused=True)), (k, q)
     plan.close()
+
+
+def test_level_tables_beyond_4_gib(cuda):
+    """2^24 + 32 rows in levels of 16: row numbers of more than 24 bits, and
+    tables of more bytes than a 32-bit offset reaches (64 bytes for each of
+    4 slots per row)."""
+    import torch
+    n, w = (1 << 24) + 32, 16
+    cnt = np.where(np.arange(n) < w, 1, 2)
+    rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    ci = np.empty(rp[-1], np.int32)
+    v = np.empty(rp[-1])
+    ci[rp[1:] - 1], v[rp[1:] - 1] = np.arange(n), 1.5
+    ci[rp[w:-1]], v[rp[w:-1]] = np.arange(n - w), api.uniform(40, n - w)
+    plan = _plan(cuda, rp, ci, v, algo="level")
+    b = api.uniform(41, n)
+    x = _run(plan, cuda, b)
+    plan.close()
+    torch.cuda.empty_cache()
+    assert np.array_equal(x, oracle.csr_forward(rp, ci, v, b, fused=True))
