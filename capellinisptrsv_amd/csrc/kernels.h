@@ -2158,8 +2158,9 @@ __global__ void __launch_bounds__(kWave)
     o[J / 2 * kWave] = make_uint4((unsigned)mm, (unsigned)(mm >> 32), w[0], w[1]);
 }
 
-// What a sweep is for: the tails a_p of history 0 (and the largest magnitude
-// in each, the bits of a NaN above all), the B_p (right-hand side q's history
+// What a sweep is for: the tails a_p of history 0 (and of each the bits of the
+// largest magnitude, a NaN's above all, and of the smallest that is not 0, 0
+// for none: top[2i], top[2i + 1]), the B_p (right-hand side q's history
 // is e_q and b is 0), or x from the tails t.
 enum PartSweep { kPartTails, kPartUnit, kPartX };
 
@@ -2311,24 +2312,35 @@ __global__ void __launch_bounds__(kPartWaves * kWave)
     }
     if (MODE != kPartX) {  // the block's last W values: blocks of m >= W rows
         const long long out = MODE == kPartUnit ? p - 1 : p;
-        unsigned long long big[KR];
+        unsigned long long big[KR], low[KR];  // low: less 1, so that 0 is above all
 #pragma unroll
-        for (int q = 0; q < KR; ++q) big[q] = 0;
+        for (int q = 0; q < KR; ++q) {
+            big[q] = 0;
+            low[q] = ~0ull;
+        }
 #pragma unroll
         for (int c = lane; c < W; c += kWave) {
 #pragma unroll
             for (int q = 0; q < KR; ++q) {
                 const double v = ring[(m - W + c) & kMask][q];
                 tails[(out * k + q0 + q) * W + c] = v;
-                big[q] = max(big[q], as_bits(v) & ~(1ull << 63));
+                const unsigned long long u = as_bits(v) & ~(1ull << 63);
+                big[q] = max(big[q], u);
+                low[q] = min(low[q], u - 1);
             }
         }
         if (MODE == kPartTails) {
 #pragma unroll
             for (int q = 0; q < KR; ++q) {
 #pragma unroll
-                for (int s = 1; s < kWave; s *= 2) big[q] = max(big[q], (unsigned long long)__shfl_xor((long long)big[q], s));
-                if (lane == 0) top[out * k + q0 + q] = big[q];
+                for (int s = 1; s < kWave; s *= 2) {
+                    big[q] = max(big[q], (unsigned long long)__shfl_xor((long long)big[q], s));
+                    low[q] = min(low[q], (unsigned long long)__shfl_xor((long long)low[q], s));
+                }
+                if (lane == 0) {
+                    top[2 * (out * k + q0 + q)] = big[q];
+                    top[2 * (out * k + q0 + q) + 1] = low[q] + 1;
+                }
             }
         }
     }
@@ -2600,10 +2612,15 @@ __global__ void __launch_bounds__(W) k_part_norm(const double *__restrict__ bm, 
 // consecutive tails and chunk of KQ right-hand sides.  Used where blocks damp
 // their history (four in a row by kPartDamp or more) or are few.  What block p
 // - s adds to t_p is at most norm(B_p ... B_{p-s+1}) max|a_{p-s}|; the walk to
-// t_p starts at the farthest block for which a bound of that is above 2^-66
-// max|a_p| (all that is left out, 256 blocks at most, then stays below 2^-58,
-// a 32nd of the rounding of t_p's own terms) and not below the smallest
-// double.  How far that is depends on the right-hand side alone, so it gets
+// t_p starts at the farthest block for which a bound of that is above
+// 2^-(57 + s/2) of the smallest magnitude in a_p that is not 0, and not below
+// the smallest double.  All that is left out then stays below 2^-55.7 of each
+// of them, a sixth of the rounding of t_p's own terms, also where the tail's
+// rows belong to systems that do not touch each other: measured against the
+// largest magnitude, one huge row of b took the digits of all the others in
+// its block's tail (4e-10 of the largest, now 4e-16).  The smallest is about
+// 9 bits below it with a dense right-hand side: 18.8 -> 19.6 us at n =
+// 500,000.  How far that is depends on the right-hand side alone, so it gets
 // the same bits in every chunk.  Blocks are looked at kPartReach back: there
 // the factor has passed 2^-2048, the whole range of a double.  After a block
 // with an infinity or a NaN in its tail every tail is NaN (0 times an
@@ -2652,28 +2669,28 @@ __global__ void __launch_bounds__(kPartSplit * W, W >= 256 && KQ >= 2 ? 7 : 1)
         lost[t] = q_count;
     }
     __syncthreads();
-    const unsigned long long *tq = top + (long long)blockIdx.y * KQ;
+    const unsigned long long *tq = top + 2LL * blockIdx.y * KQ;
     for (int h = t; h < p1 - 1; h += kThreads) {
 #pragma unroll
         for (int j = 0; j < KQ; ++j)
-            if (tq[(long long)h * k + j] >= kInf) atomicMin(&lost[j], h);
+            if (tq[2 * ((long long)h * k + j)] >= kInf) atomicMin(&lost[j], h);
     }
     // (tail, right-hand side) pairs, one to a wavefront: lane l looks at the
     // blocks l, l + 64, ... back
     for (int e = wave; e < (p1 - p0) * KQ; e += kThreads / kWave) {
         const int p = p0 + e / KQ, j = e % KQ;
-        const unsigned long long own = tq[(long long)p * k + j];
+        const unsigned long long own = tq[2 * ((long long)p * k + j) + 1];
         int far = 0;
 #pragma unroll
         for (int i = 0; i < kPartReach; i += kWave) {
             const int s = i + lane, h = p - s;
             if (s == 0 || h < 0) continue;
-            const unsigned long long bits = tq[(long long)h * k + j];
+            const unsigned long long bits = tq[2 * ((long long)h * k + j)];
             // log2 in 256ths, the exponent biased: above the term's (an
             // exponent and a fraction fall short of it by 0.087 at most)
             const int mid = p - (s & ~3);
             const int term = (int)(bits >> 44) + 24 + (int)(fade[p].y - fade[mid].y) + (int)(fade[mid].x - fade[h].x);
-            const int floor = own >= kNormal && own < kInf ? (int)(own >> 44) - 66 * 256 : -60 * 256;
+            const int floor = own >= kNormal && own < kInf ? (int)(own >> 44) - 57 * 256 - 128 * s : -60 * 256;
             if (bits != 0 && term > max(floor, -60 * 256)) far = s;
         }
 #pragma unroll

@@ -103,7 +103,7 @@ struct PartState {
     // work vectors, sized for kcap right-hand sides (grown by a solve with more)
     int kcap = 0;
     double *a = nullptr, *u = nullptr, *t = nullptr, *c0 = nullptr, *c1 = nullptr;
-    unsigned long long *top = nullptr;      // the largest magnitude of each a_p
+    unsigned long long *top = nullptr;      // the largest and smallest magnitude of each a_p
     double *res = nullptr, *cor = nullptr;  // refinement: FP64 residual and correction (n * kcap)
 };
 
@@ -637,7 +637,7 @@ int ensure_part_rhs(cap_plan p, int k)
     const size_t tails = (size_t)ps->Q * k * ps->W, carries = (size_t)ps->G * k * ps->W;
     CAP_TRY(dev_alloc(&ps->a, tails));
     CAP_TRY(dev_alloc(&ps->t, tails));
-    CAP_TRY(dev_alloc(&ps->top, (size_t)ps->Q * k));
+    CAP_TRY(dev_alloc(&ps->top, (size_t)ps->Q * k * 2));
     if (!ps->walk) {
         CAP_TRY(dev_alloc(&ps->u, tails));
         CAP_TRY(dev_alloc(&ps->c0, carries));

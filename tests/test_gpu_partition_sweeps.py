@@ -162,3 +162,28 @@ def test_one_nonzero_row(cuda, name):
         ref = oracle.csr_forward(*mat, beside[:, q].copy(), fused=True)
         assert rel_maxnorm(xs[:, q], ref) <= FP64_TOL, q
     plan.close()
+
+
+@pytest.mark.parametrize("huge", [1e6, 1e25])
+def test_a_huge_row_does_not_reach_rows_that_do_not_depend_on_it(cuda, huge):
+    """Even and odd rows are systems of their own, and even rows of b at the
+    blocks' ends are huge: the odd rows keep the accuracy they have without."""
+    import torch
+    n, w = 100_000, 50
+    rng = np.random.default_rng(5)
+    rows = np.repeat(np.arange(n), 2)
+    cols = rows - 2 * rng.integers(w - 10, w + 1, len(rows))
+    key = np.unique(rows[cols >= 0] * np.int64(n) + cols[cols >= 0])
+    rp = np.r_[0, np.cumsum(np.bincount(key // n, minlength=n) + 1)].astype(np.int32)
+    ci, v = np.empty(rp[-1], np.int32), np.empty(rp[-1])
+    at = np.arange(len(key)) + key // n
+    ci[at], v[at] = key % n, rng.uniform(0.5, 1.0, len(key))
+    ci[rp[1:] - 1], v[rp[1:] - 1] = np.arange(n), 4.5
+    plan = _plan(cuda, (rp, ci, v))
+    b = api.uniform(3, n)
+    b[np.arange(500, n, 1000) // 2 * 2] = huge
+    x = plan.solve(torch.from_numpy(b).to(cuda)).cpu().numpy()
+    want = oracle.csr_forward(rp, ci, v, b, fused=True)
+    assert rel_maxnorm(x, want) <= FP64_TOL
+    assert rel_maxnorm(x[1::2], want[1::2]) <= FP64_TOL
+    plan.close()
