@@ -780,10 +780,11 @@ __global__ void __launch_bounds__(BLOCK)
             for (int t = 0; t < E; ++t) vv[j][t] = val[fj + min(t, nn)];
         }
         Idle idle;
+        int missing = -1;
         bool done = !in;
         do {  // wave-uniform exit: see wrtfst_row
             if (!done) {
-                bool all = true;
+                int left = 0;  // values still missing
 #pragma unroll
                 for (int j = 0; j < E; ++j)
 #pragma unroll
@@ -792,9 +793,11 @@ __global__ void __launch_bounds__(BLOCK)
 #pragma unroll
                 for (int j = 0; j < E; ++j)
 #pragma unroll
-                    for (int t = 0; t < E; ++t) all = all && r[j][t] != kS;
-                const bool failed = !all && give_up(sc, idle);
-                if (all || failed) {
+                    for (int t = 0; t < E; ++t) left += r[j][t] == kS;
+                if (left != missing) idle.progress();
+                const bool failed = left != 0 && left == missing && give_up(sc, idle);
+                missing = left;
+                if (left == 0 || failed) {
                     T sum = (T)0;
 #pragma unroll
                     for (int j = 0; j < E; ++j) {
@@ -1206,10 +1209,11 @@ __global__ void __launch_bounds__(BLOCK)
             return u == kS ? (U)kPairQNaN : u;
         };
         Idle idle;
+        int missing = -1;
         bool done = !in;
         do {  // wave-uniform exit: see wrtfst_row
             if (!done) {
-                bool all = true;
+                int left = 0;  // values still missing
 #pragma unroll
                 for (int j = 0; j < E; ++j)
 #pragma unroll
@@ -1218,9 +1222,11 @@ __global__ void __launch_bounds__(BLOCK)
 #pragma unroll
                 for (int j = 0; j < E; ++j)
 #pragma unroll
-                    for (int t = 0; t < E; ++t) all = all && r[j][t] != kS;
-                const bool failed = !all && give_up(sc, idle);
-                if (all || failed) {
+                    for (int t = 0; t < E; ++t) left += r[j][t] == kS;
+                if (left != missing) idle.progress();
+                const bool failed = left != 0 && left == missing && give_up(sc, idle);
+                missing = left;
+                if (left == 0 || failed) {
                     float s0 = 0.0f, s1 = 0.0f;
                     double sum = 0.0;
 #pragma unroll

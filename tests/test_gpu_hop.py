@@ -225,3 +225,50 @@ def test_cached_pick_that_does_not_fit_is_tuned_afresh(cuda, kind):
         assert np.array_equal(_run(other, cuda, b), oracle.csr_forward(*m, b, fused=True))
         other.close()
     plan.close()
+
+
+@pytest.mark.parametrize("call", ["solve", "refined"])
+def test_spin_limit_counts_polls_without_progress(cuda, call):
+    """A chain whose rows also read the rows at 1/4, 1/2 and 3/4 of the way
+    sees a value arrive in every quarter of its wait; one whose other entries
+    are the first rows waits all along for the last.  Bounded in polls without
+    progress, the first needs about a quarter of the second's limit (bar: 0.6,
+    between the 0.25 and the 1 of a bound on all of a row's polls)."""
+    import torch
+    n = 1536
+
+    def chain(spread):
+        rp, ci = [0], []
+        for i in range(n):
+            cs = {i - 1, 3 * i // 4, i // 2, i // 4} if spread else {i - 1, 0, 1, 2}
+            ci += sorted(c for c in cs if 0 <= c < i) + [i]
+            rp.append(len(ci))
+        rp, ci = np.array(rp, np.int32), np.array(ci, np.int32)
+        return rp, ci, np.where(ci == np.repeat(np.arange(n), np.diff(rp)), 4.0, 0.5)
+
+    b = torch.from_numpy(api.uniform(27, n)).to(cuda)
+
+    def ends(mat, limit):
+        plan = _plan(cuda, *mat, algo="hop", spin_limit=limit)
+        ok = []
+        for _ in range(3):
+            if call == "solve":
+                plan.solve(b)
+            else:
+                try:
+                    plan.solve_refined(b, tol=1e-9)
+                except _native.CapError:
+                    pass
+            ok.append(plan.status() == 0)
+        plan.close()
+        return all(ok)
+
+    def least(mat):
+        lo, hi = 1.0, 2.0 ** 17
+        assert ends(mat, int(hi))
+        while hi > 1.1 * lo:
+            mid = (lo * hi) ** 0.5
+            lo, hi = (lo, mid) if ends(mat, int(mid)) else (mid, hi)
+        return hi
+
+    assert least(chain(True)) <= 0.6 * least(chain(False))
