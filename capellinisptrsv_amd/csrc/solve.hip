@@ -219,6 +219,7 @@ struct cap_plan_s {
     // write-first solve of one right-hand side with look-through tables
     // (autotuned plans, value protocol, staged readiness)
     HopState *hop = nullptr;
+    bool hop_reset = false;  // reversed plans: a solve or reset over the tables has run
 };
 
 // One right-hand side of a plan whose pick has look-through tables.  The
@@ -2339,6 +2340,7 @@ int cap_plan_solve(cap_plan p, const void *b, void *x, int rhs, void *stream)
     if (p->tune_rhs && rhs > 1 && rhs <= kWave && !p->reversed && !p->rhs_pick.count(rhs))
         CAP_TRY(tune_rhs_block(p, b, x, rhs, S(stream)));
     const int algo = algo_for(p, rhs), sync = sync_for(p, rhs);
+    if (hop_takes(p, rhs)) p->hop_reset = true;
     if (!p->reversed || hop_takes(p, rhs)) return plan_solve_with(p, algo, sync, b, x, rhs, S(stream));
     CAP_TRY(ensure_reversal(p, rhs));
     CAP_TRY(reverse_rows(p, b, p->rev_b, rhs, S(stream)));
@@ -2349,7 +2351,9 @@ int cap_plan_solve(cap_plan p, const void *b, void *x, int rhs, void *stream)
 int cap_plan_reset(cap_plan p, void *x, int rhs, void *stream)
 {
     if (!p || !x || rhs < 1) return CAP_ERR_ARG;
-    if (p->reversed && !hop_takes(p, rhs)) {
+    if (hop_takes(p, rhs)) {
+        p->hop_reset = true;
+    } else if (p->reversed) {
         CAP_TRY(ensure_reversal(p, rhs));
         x = p->rev_x;
     }
@@ -2361,6 +2365,7 @@ int cap_plan_reset(cap_plan p, void *x, int rhs, void *stream)
 int cap_plan_launch(cap_plan p, const void *b, void *x, int rhs, void *stream)
 {
     if (!p || !b || !x || rhs < 1) return CAP_ERR_ARG;
+    if (p->reversed && hop_takes(p, rhs) && !p->hop_reset) return CAP_ERR_ARG;  // launch without its reset
     if (!p->reversed || hop_takes(p, rhs)) return launch_plain(p, b, x, rhs, S(stream));
     if (p->rev_bytes < (size_t)p->n * rhs * p->vbytes) return CAP_ERR_ARG;  // launch without its reset
     CAP_TRY(reverse_rows(p, b, p->rev_b, rhs, S(stream)));

@@ -102,6 +102,23 @@ def test_hop_triangular_kinds(cuda, kind):
     plan.close()
 
 
+def test_upper_launch_without_reset_is_refused(cuda):
+    """As for the other kernels of upper-triangular plans: a launch that no
+    reset or solve came before is an argument error."""
+    import torch
+    rp, ci, v = upper_from_lower(*random_lower(500, max_off=3, band=100, seed=12, dup=False))
+    b = torch.from_numpy(api.uniform(28, 500)).to(cuda)
+    x = torch.zeros_like(b)
+    for algo in ("wrtfst", "hop"):
+        plan = _plan(cuda, rp, ci, v, algo=algo, upper=True)
+        with pytest.raises(_native.CapError, match=str(_native.CAP_ERR_ARG)):
+            plan.launch(b, x)
+        plan.reset(x)
+        plan.launch(b, x)
+        assert np.array_equal(x.cpu().numpy(), oracle.csr_solve(rp, ci, v, b.cpu().numpy(), upper=True, fused=True))
+        plan.close()
+
+
 def test_hop_reads_the_callers_values_and_special_values(cuda):
     """The tables hold the pattern only: values changed in place between two
     solves count.  Infinities, NaN and the sentinel's own bits in b spread
