@@ -393,6 +393,46 @@ void ready_release(void *ptr)
         if (r.ptr == ptr) r.used = false;
 }
 
+// ------------------------------------------------------------ pinned words
+// What refined solves read their norms from, 64 bytes a plan.  A pinned
+// allocation takes 25 us, inside a new plan's first refined solve, so up to
+// kEchoKept of them stay for later plans.
+constexpr size_t kEchoKept = 16;
+std::mutex g_echo_mu;
+std::vector<unsigned long long *> g_echo_free;
+
+int echo_acquire(unsigned long long **out)
+{
+    {
+        std::lock_guard<std::mutex> g(g_echo_mu);
+        if (!g_echo_free.empty()) {
+            *out = g_echo_free.back();
+            g_echo_free.pop_back();
+        }
+    }
+    if (!*out && hipHostMalloc(reinterpret_cast<void **>(out), 64, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        *out = nullptr;
+        return CAP_ERR_ALLOC;
+    }
+    std::memset(*out, 0, 64);  // another plan's counts
+    return CAP_OK;
+}
+
+// After the last kernel that writes the words.
+void echo_release(unsigned long long *words)
+{
+    if (!words) return;
+    {
+        std::lock_guard<std::mutex> g(g_echo_mu);
+        if (g_echo_free.size() < kEchoKept) {
+            g_echo_free.push_back(words);
+            return;
+        }
+    }
+    (void)hipHostFree(words);
+}
+
 // The plan's staged readiness array holds at least `bytes`.  Growing it
 // waits for the device (kernels in flight may still poll the old block) and
 // drops the captured refinement graph, which has the old block's address.
@@ -465,7 +505,7 @@ void plan_free(cap_plan p)
     if (p->refine_graph) (void)hipGraphExecDestroy(p->refine_graph);
     if (p->echo) {
         (void)hipDeviceSynchronize();
-        (void)hipHostFree(p->echo);
+        echo_release(p->echo);
     }
     delete p;
 }
@@ -2524,6 +2564,8 @@ inline unsigned stream_blocks(const cap_plan p, long long count)
 // separate one-workgroup solves.
 inline bool refine_fuses(const cap_plan p) { return p->algo != CAP_ALGO_LOCAL && p->algo != CAP_ALGO_PARTITION; }
 
+// What the steps after a fused sweep, or all of them, work on: the FP32
+// values, residual and correction.
 int ensure_refine(cap_plan p, int rhs, hipStream_t st)
 {
     const long long len = (long long)p->n * rhs;
@@ -2540,12 +2582,19 @@ int ensure_refine(cap_plan p, int rhs, hipStream_t st)
         CAP_TRY(dev_alloc(&p->d32, (size_t)len));
         p->refine_len = len;
     }
-    if (refine_fuses(p) && !p->staged && p->pair_len < len) {
-        if (p->pair) CAP_HIP_TRY(hipFree(p->pair));
-        p->pair = nullptr;
-        CAP_TRY(dev_alloc(&p->pair, (size_t)len));
-        p->pair_len = len;
-    }
+    return CAP_OK;
+}
+
+// Where the fused sweep publishes its pairs, when readiness is in place.
+int ensure_pairs(cap_plan p, int rhs)
+{
+    const long long len = (long long)p->n * rhs;
+    if (p->staged || p->pair_len >= len) return CAP_OK;
+    if (p->pair) CAP_HIP_TRY(hipFree(p->pair));
+    p->pair = nullptr;
+    p->pair_len = 0;
+    CAP_TRY(dev_alloc(&p->pair, (size_t)len));
+    p->pair_len = len;
     return CAP_OK;
 }
 
@@ -2613,10 +2662,7 @@ int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st
 // stream.
 int read_norms(cap_plan p, unsigned long long *nb, hipStream_t st)
 {
-    if (!p->echo) {
-        CAP_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&p->echo), 64, hipHostMallocDefault));
-        std::memset(p->echo, 0, 64);  // memory of a freed plan's counts may come back
-    }
+    if (!p->echo) CAP_TRY(echo_acquire(&p->echo));
     const unsigned long long count = ++p->echoes;
     k_echo<<<1, kWave, 0, st>>>(p->norms, p->echo, count);
     CAP_HIP_TRY(hipGetLastError());
@@ -2750,22 +2796,19 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
     // allocate there
     if (p->algo == CAP_ALGO_PARTITION && p->part)
         return refined_partition(p, b, x, rhs, tol, max_iter, iters, last_rel, st);
-    CAP_TRY(ensure_refine(p, rhs, st));
     // the staged readiness array must exist before capture (no allocation
     // inside the captured steps, whose kernels bake in its address); the
     // fused sweep publishes 8-byte pairs, the correction solves 4-byte values
     const bool fused = refine_fuses(p);
+    CAP_TRY(fused ? ensure_pairs(p, rhs) : ensure_refine(p, rhs, st));
     if (p->staged) CAP_TRY(ensure_ready(p, (fused ? 8 : 4) * (size_t)p->n * rhs));
-    if (fused && !p->rblock) {
-        CAP_TRY(tune_refine_block(p, b, x, rhs, st));
-        if (p->refine_graph) CAP_HIP_TRY(hipGraphExecDestroy(p->refine_graph));
-        p->refine_graph = nullptr;
-    }
-    // The first two steps (solve from b, one correction) are one graph:
-    // captured once per (b, x, rhs), replayed on later calls; with side
-    // streams to join, two launches.
-    const bool plain = fused && join;
-    if (plain) {
+    if (fused && !p->rblock) CAP_TRY(tune_refine_block(p, b, x, rhs, st));
+    // The fused sweep is two launches: a graph of them saves nothing (101 us a
+    // call, 96 without, n = 1,000,000) and its stream, capture and
+    // instantiation, up to 0.5 ms, fall on every new (b, x).  The first two
+    // unfused steps (solve from b, one correction) are one, captured once per
+    // (b, x, rhs), replayed on later calls.
+    if (fused) {
         CAP_TRY(refine_fused(p, b, x, rhs, st, join));
     } else if (!p->refine_graph || p->graph_b != b || p->graph_x != x || p->graph_rhs != rhs) {
         if (p->refine_graph) CAP_HIP_TRY(hipGraphExecDestroy(p->refine_graph));
@@ -2774,13 +2817,8 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
         CAP_HIP_TRY(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
         hipGraph_t graph;
         CAP_HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-        int rc = CAP_OK;
-        if (fused) {
-            rc = refine_fused(p, b, x, rhs, cs);
-        } else {
-            rc = refine_step(p, b, x, rhs, true, cs);
-            if (rc == CAP_OK) rc = refine_step(p, b, x, rhs, false, cs);
-        }
+        int rc = refine_step(p, b, x, rhs, true, cs);
+        if (rc == CAP_OK) rc = refine_step(p, b, x, rhs, false, cs);
         hipError_t ec = hipStreamEndCapture(cs, &graph);
         if (rc != CAP_OK || ec != hipSuccess) {
             (void)hipStreamDestroy(cs);
@@ -2797,7 +2835,7 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
     int it = 0;
     unsigned long long nb[2];
     int rc = CAP_OK;
-    if (!plain) CAP_HIP_TRY(hipGraphLaunch(p->refine_graph, st));
+    if (!fused) CAP_HIP_TRY(hipGraphLaunch(p->refine_graph, st));
     if (join) CAP_TRY(join_parts(join, st));
     it = 2;
     while (true) {
@@ -2815,6 +2853,7 @@ int refined_impl(cap_plan p, const double *b, double *x, int rhs, double tol, in
             rc = CAP_ERR_NOT_CONVERGED;
             break;
         }
+        CAP_TRY(ensure_refine(p, rhs, st));
         CAP_TRY(refine_step(p, b, x, rhs, false, st));
         ++it;
     }

@@ -289,3 +289,21 @@ def test_spin_limit_counts_polls_without_progress(cuda, call):
         return hi
 
     assert least(chain(True)) <= 0.6 * least(chain(False))
+
+
+def test_refined_solves_of_many_plans_keep_their_norms_apart(cuda):
+    """The pinned words that the norms are read from pass from freed plans to
+    new ones, and more plans than are kept hold words at once."""
+    import torch
+    mats = [random_lower(300 + 7 * i, max_off=3, band=100, seed=60 + i) for i in range(20)]
+    for _ in range(2):
+        plans = [_plan(cuda, *m, algo="hop") for m in mats]
+        for rep in range(2):
+            for i, (plan, m) in enumerate(zip(plans, mats)):
+                b = api.uniform(70 + i + 20 * rep, len(m[0]) - 1)
+                x0, d, want = oracle.refine2(*m, b, rhs=1, rcp=True)
+                x, iters, rel = plan.solve_refined(torch.from_numpy(b).to(cuda), tol=1e-9)
+                assert iters == 2 and np.array_equal(x.cpu().numpy(), want)
+                assert rel == float(np.abs(d).max()) / float(np.abs(x0).max())
+        for plan in plans:
+            plan.close()
