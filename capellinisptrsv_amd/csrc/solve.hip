@@ -1183,6 +1183,7 @@ struct TuneKey {
 std::mutex g_tune_mu;
 struct TuneChoice {
     int algo, sync, border, bpc, lds, staged, block, tile = 0, hop = 0;
+    int width = 0;  // rows per step of the level steps
 };
 std::map<TuneKey, TuneChoice> g_tune_cache;
 
@@ -1822,14 +1823,16 @@ int level_accepts(cap_plan p, const std::vector<int> &rp, const std::vector<int>
 // keeps the values of its creation.  An autotuned plan over the caller's own
 // values copies them into the tables again on every solve (6 us at n = 2,000,
 // 8 at n = 100,000): the kernels it would run otherwise read them there, and
-// which of them wins is a matter of microseconds.
-int build_level(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, bool explicit_algo, hipStream_t st)
+// which of them wins is a matter of microseconds.  width: rows per step, when
+// a cached pick knows them.
+int build_level(cap_plan p, const std::vector<int> &rp, const std::vector<int> &ci, bool explicit_algo, hipStream_t st,
+                int width = 0)
 {
     int rhs = 0;
     if (explicit_algo) CAP_TRY(level_accepts(p, rp, ci, &rhs));
     free_level(p);
-    CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rhs : 4, p->lds_max, kStepPadMax,
-                        explicit_algo ? HUGE_VAL : kStepMaxBytes, p->rp, p->ci, p->val, st));
+    CAP_TRY(steps_build(&p->lvl, rp, ci, {make_int2(0, p->n)}, p->vt, explicit_algo ? rhs : 4, width, p->lds_max,
+                        kStepPadMax, explicit_algo ? HUGE_VAL : kStepMaxBytes, p->rp, p->ci, p->val, st));
     p->lvl_rhs = rhs;
     p->lvl_live = !explicit_algo && !p->owns_matrix;
     return CAP_OK;
@@ -1941,7 +1944,7 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
             int rc = CAP_OK;
             if (c.algo == CAP_ALGO_MIX) rc = build_mix(p, rp_host, c.border);
             else if (c.algo == CAP_ALGO_LOCAL) rc = ensure_segments(p, nullptr);
-            else if (c.algo == CAP_ALGO_LEVEL) rc = build_level(p, rp_host, ci, false, st);
+            else if (c.algo == CAP_ALGO_LEVEL) rc = build_level(p, rp_host, ci, false, st, c.width);
             else if (c.algo == CAP_ALGO_PARTITION) rc = build_partition(p, rp_host, st);
             else if (c.hop) rc = build_hop(p, rp_host, ci, st);
             // The key samples the pattern: this matrix may have a row too long
@@ -2032,7 +2035,10 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
     if (pick.algo == CAP_ALGO_MIX) CAP_TRY(build_mix(p, rp_host, pick.border));
     if (pick.algo == CAP_ALGO_LOCAL) CAP_TRY(ensure_segments(p, nullptr));
     if (pick.algo != CAP_ALGO_PARTITION) free_partition(p);
-    if (pick.algo != CAP_ALGO_LEVEL) free_level(p);
+    if (pick.algo == CAP_ALGO_LEVEL)
+        pick.width = p->lvl->block;
+    else
+        free_level(p);
     std::lock_guard<std::mutex> g(g_tune_mu);
     g_tune_cache[key] = pick;
     return CAP_OK;
@@ -3112,7 +3118,7 @@ int choose_batch_steps(cap_plan p, int k, const std::vector<int> &ro, const std:
             mats.push_back(make_int2(ro[m], ro[m + 1]));
     if (mats.empty()) return CAP_OK;
     StepTables *t = nullptr;
-    int rc = steps_build(&t, rp, ci, mats, p->vt, 4, p->lds_max, kStepPadMax, kStepMaxBytes, p->rp, p->ci, p->val, st);
+    int rc = steps_build(&t, rp, ci, mats, p->vt, 4, 0, p->lds_max, kStepPadMax, kStepMaxBytes, p->rp, p->ci, p->val, st);
     if (rc == CAP_ERR_UNSUPPORTED || rc == CAP_ERR_ALLOC) return CAP_OK;  // the plain batch stays
     if (rc != CAP_OK) return rc;
     if (!steps_take(t, k)) {

@@ -37,13 +37,14 @@ struct StepTables {
 // Schedules the rows of each matrix [first, last) of a block-diagonal CSR (host copies rp, ci with global columns; the same arrays
 // and the values on the device) and lays out the tables.  want_rhs: right-hand
 // sides a thread should solve (4, 2 or 1); fewer where the ring does not
-// fit lds_bytes (max_rhs says how many).  CAP_ERR_UNSUPPORTED when a matrix's
+// fit lds_bytes (max_rhs says how many).  want_block: rows per step (64, 128,
+// 192 or 256; 0: each matrix's best, by scheduling it for all of them).  CAP_ERR_UNSUPPORTED when a matrix's
 // dependencies reach further back than any ring, or its steps would be mostly
 // padding (more than pad_max slots per row), or the tables more than
 // max_bytes.
 int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<int> &ci,
-                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, double max_bytes,
-                const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st);
+                const std::vector<int2> &mats, int vt, int want_rhs, int want_block, int lds_bytes, int pad_max,
+                double max_bytes, const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st);
 // Copies the values into the tables again (they changed in place).
 int steps_refresh(const StepTables *t, const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st);
 // Solves k right-hand sides (interleaved, row * k + q), 1, 2 or 4 of them per

@@ -597,7 +597,7 @@ int fill_any(const StepTables *t, const int *d_rp, const int *d_ci, const void *
 }
 
 int build(StepTables *t, const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<int2> &mats,
-          int want_rhs, int lds_bytes, int pad_max, double max_bytes)
+          int want_rhs, int want_block, int lds_bytes, int pad_max, double max_bytes)
 {
     const int vb = t->vt == CAP_F64 ? 8 : 4;
     int longest = 0, reach = 0, tallest = 0;
@@ -636,6 +636,7 @@ int build(StepTables *t, const std::vector<int> &rp, const std::vector<int> &ci,
         int B = 0, steps = 0;
         double cost = 0;
         for (int cand = kWave; cand <= kStepBlock; cand += kWave) {
+            if (want_block && cand != want_block) continue;
             const int s = place_rows(rp, ci, lo, hi, cand, R, &step, &last);
             const double c = s * step_ns(t->E, K, cand / kWave);
             if (!B || c < cost) {
@@ -787,8 +788,8 @@ int launch_any(const StepTables *t, const void *b, void *x, int k, bool unfused,
 }  // namespace
 
 int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<int> &ci,
-                const std::vector<int2> &mats, int vt, int want_rhs, int lds_bytes, int pad_max, double max_bytes,
-                const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st)
+                const std::vector<int2> &mats, int vt, int want_rhs, int want_block, int lds_bytes, int pad_max,
+                double max_bytes, const int *d_rp, const int *d_ci, const void *d_val, hipStream_t st)
 {
     *out = nullptr;
     int dev = 0, cus = 0;
@@ -801,7 +802,7 @@ int steps_build(StepTables **out, const std::vector<int> &rp, const std::vector<
     t->lds = (size_t)std::max(0, lds_bytes);
     int rc;
     try {
-        rc = build(t, rp, ci, mats, want_rhs, lds_bytes, pad_max, max_bytes);
+        rc = build(t, rp, ci, mats, want_rhs, want_block, lds_bytes, pad_max, max_bytes);
     } catch (const std::bad_alloc &) {
         rc = CAP_ERR_ALLOC;
     }

@@ -102,6 +102,26 @@ def test_autotuned_steps_read_values_where_the_rule_accepts(cuda, dtype):
     plan.close()
 
 
+@pytest.mark.parametrize("width", [40, 150, 240])
+def test_cached_pick_keeps_its_rows_per_step(cuda, width):
+    """A second plan of a pattern schedules for the first one's rows per step
+    alone; a matrix taken for it by the cache's samples solves all the same."""
+    rp, ci, v = api.generate("level", n=6000, levels=6000 // width, width=width, depth=2, offdiag=9, seed=width)
+    n = len(rp) - 1
+    b = api.uniform(9, n)
+    ref = oracle.csr_forward(rp, ci, v, b, fused=True)
+    widths = []
+    for _ in range(3):
+        plan = _plan(cuda, rp, ci, v)
+        info = plan.info()
+        assert info["algo"] == "level"
+        widths.append(info["row_threads"])
+        assert np.array_equal(_solve(plan, cuda, b), ref)
+        plan.close()
+    assert len(set(widths)) == 1
+    assert _plan(cuda, rp, ci, v, algo="level").info()["row_threads"] == widths[0]
+
+
 def test_autotuned_short_chains_follow_the_callers_values(cuda):
     """The partition holds the values of plan creation: on short chains, where
     it wins by little, auto keeps a kernel that reads them."""
