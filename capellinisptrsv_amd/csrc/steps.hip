@@ -18,8 +18,9 @@ namespace cap {
 // contiguous run.  Pieces: the head {own ring slot | long << 16, start of the
 // rest (long rows), and with E = 4 the four entries' ring slots, 16 bits
 // each}; with E > 4 the E ring slots, 8 per piece; the E values; {diagonal,
-// its reciprocal}.  Unused entries name slot `ring`, which holds 0, with the
-// value 0: fma(0, 0, s) = s exactly (a sum that starts at +0 is never -0).
+// its reciprocal}.  Unused entries name slot `ring`, which holds +0, with the
+// value -0: the sum of s and their product is s for every s, also for the -0
+// that a negative product too small for a number leaves.
 // Slots a step does not need repeat the step's first row: they compute the
 // same value into the same places, so every thread runs the same
 // straight-line step and none needs a place to put a result nobody reads.
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(kBlock)
         }
         T v[E];
 #pragma unroll
-        for (int u = 0; u < E; ++u) v[u] = u < cnt ? val[e0 + u] : (T)0;
+        for (int u = 0; u < E; ++u) v[u] = u < cnt ? val[e0 + u] : -(T)0;
 #pragma unroll
         for (int h = 0; h < L::kVals; ++h) {
             uint4 w;

@@ -182,6 +182,32 @@ def test_step_division_range(cuda, dtype, bits, span):
     plain.close()
 
 
+@pytest.mark.parametrize("dtype,bits", [(np.float64, np.uint64), (np.float32, np.uint32)])
+@pytest.mark.parametrize("extra", [0, 4, 8])
+def test_unused_entries_keep_the_sign_of_a_zero_sum(cuda, extra, dtype, bits):
+    """A product that underflows to -0 leaves the sum -0, and -0 - (-0) is +0:
+    the entries a row does not have must not turn the sum into +0.  4, 8 and
+    16 entries carried (`extra` more in the last row)."""
+    n = 40
+    tiny = np.finfo(dtype).tiny
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        cols = [i - 1] if i % 2 else []
+        if i == n - 1:
+            cols = list(range(i - 1 - extra, i))
+        ci += cols + [i]
+        v += [-float(tiny)] * len(cols) + [1.0 if i % 4 else -2.0]
+        rp.append(len(ci))
+    rp, ci, v = np.array(rp, np.int32), np.array(ci, np.int32), np.array(v, dtype)
+    b = np.full(n, tiny, dtype)  # even rows: x = +-tiny, whose products with tiny underflow
+    b[1::2] = dtype(-0.0)
+    ref = oracle.csr_forward(rp, ci, v, b, fused=True)
+    assert np.signbit(ref[1::2]).any() and not np.signbit(ref[1::2]).all()
+    plan = _plan(cuda, rp, ci, v, algo="level")
+    assert np.array_equal(_solve(plan, cuda, b).view(bits), ref.view(bits))
+    plan.close()
+
+
 def _batch(seed, sizes, off, band):
     mats = [api.generate("band_rowcount", n=n, offdiag=off, band=band, seed=seed + i) if n else
             (np.zeros(1, np.int32), np.zeros(0, np.int32), np.zeros(0)) for i, n in enumerate(sizes)]
