@@ -123,6 +123,15 @@ struct RhsPick {
     int staged = -1;  // readiness: 1 staged, 0 in x itself, -1 the plan's
     int lds = -1;     // LDS window: 0 off (the 1024-thread shapes), -1 the plan's
     int tile = -1;    // row tiles: 1 on, 0 off, -1 the plan's
+    bool rows = false;  // a level plan's: the write-first kernel, not the steps
+};
+
+// The fastest plain write-first shape (value protocol, the plan's readiness)
+// of an autotuned plan whose pick solves one right-hand side otherwise, by
+// look-through tables or steps: what its several right-hand sides and its
+// fused sweeps start from.  bpc 0: none.
+struct PlainShape {
+    int bpc = 0, block = 0, lds = 0, tile = 0, staged = 0;
 };
 
 struct cap_plan_s {
@@ -157,6 +166,8 @@ struct cap_plan_s {
     // right-hand-side count on the first cap_plan_solve with that count
     bool tune_rhs = false;
     std::map<int, RhsPick> rhs_pick;
+    PlainShape plain;
+    float lvl_lead = 0;  // a level pick: the plain shape's time over the steps', one right-hand side
     int part_kr = 0;  // partition sweeps: right-hand sides per wavefront (0: the fixed rule)
     int rpl = 1;      // thread-per-row, several right-hand sides: right-hand sides per lane
     int fixed_rpl = 0;  // cap_opts.rhs_per_lane: the multi-RHS block the caller fixed (0: none)
@@ -890,6 +901,7 @@ struct RhsScope {
     {
         const auto it = k > 1 ? p->rhs_pick.find(k) : p->rhs_pick.end();
         if (it == p->rhs_pick.end()) {
+            if (k > 1 && p->plain.bpc && (!p->tune_rhs || p->reversed)) take(p->plain);
             if (k > 1 && p->fixed_rpl > 0) {  // cap_opts.rhs_per_lane
                 p->bpc = 1;
                 p->wblock = kBlockLarge;
@@ -904,6 +916,14 @@ struct RhsScope {
         if (it->second.staged >= 0) p->staged = it->second.staged != 0;
         if (it->second.lds >= 0) p->lds = it->second.lds;
         if (it->second.tile >= 0) p->tile = it->second.tile;
+    }
+    void take(const PlainShape &s)
+    {
+        p->bpc = s.bpc;
+        p->wblock = s.block;
+        p->lds = s.lds;
+        p->tile = s.tile;
+        p->staged = s.staged;
     }
     ~RhsScope()
     {
@@ -1097,6 +1117,10 @@ inline int algo_for(cap_plan p, int rhs)
 {
     if (p->algo == CAP_ALGO_LEVEL && level_allows(p, rhs) && !steps_take(p->lvl, rhs) && rhs >= 1 && rhs <= kWave)
         return CAP_ALGO_WRTFST;
+    if (p->algo == CAP_ALGO_LEVEL && rhs > 1) {
+        const auto it = p->rhs_pick.find(rhs);
+        if (it != p->rhs_pick.end() && it->second.rows) return CAP_ALGO_WRTFST;
+    }
     if (rhs > 1 && p->auto_algo &&
         (p->algo == CAP_ALGO_MIX || p->algo == CAP_ALGO_TWOPART || p->algo == CAP_ALGO_CSC ||
          (p->algo == CAP_ALGO_LEVEL && !level_takes(p, rhs))))
@@ -1184,6 +1208,8 @@ std::mutex g_tune_mu;
 struct TuneChoice {
     int algo, sync, border, bpc, lds, staged, block, tile = 0, hop = 0;
     int width = 0;  // rows per step of the level steps
+    PlainShape plain{};
+    float lead = 0;
 };
 std::map<TuneKey, TuneChoice> g_tune_cache;
 
@@ -1253,13 +1279,35 @@ int time_candidate(cap_plan p, int algo, int sync, const void *b, void *x, int r
 // lanes, poll at once), 1024-thread workgroups with 1, 2, 4 (8 in FP32)
 // right-hand sides per lane, and the pick again with readiness in x;
 // partitioned plans time 1, 2 and 4 right-hand sides per wavefront of the
-// sweeps (the ones that divide k).  Every candidate gives the same
-// bits.  The plan's own settings are timed first and another must be 2 %
-// faster to win.  Waits for the device (events).
+// sweeps (the ones that divide k); level plans, where it may be close, the
+// steps and then the thread-per-row shapes (not in a capture).  Every
+// candidate gives the same bits.  The plan's own settings (PlainShape) are
+// timed first and another must be 2 % faster to win.  Waits for the device
+// (events).
 int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
 {
     std::vector<RhsPick> cands;
-    const int algo = algo_for(p, k), sync = sync_for(p, k);
+    int algo = algo_for(p, k), sync = sync_for(p, k);
+    const bool steps = algo == CAP_ALGO_LEVEL;
+    float t_steps = 1e30f;
+    if (steps) {
+        // with k right-hand sides a step takes up to 1 + log2(k) / 5 as long
+        // (100k band: 1.03, 1.2, 1.6, 1.9 and 2.2 with 2, 4, 8, 16 and 64),
+        // the write-first kernel at least 3/4 of its time with one: only near
+        // ties are timed
+        if (p->plain.bpc == 0 || 0.75f * p->lvl_lead >= 1.0f + 0.2f * std::log2((float)k)) {
+            p->rhs_pick[k] = RhsPick{};
+            return CAP_OK;
+        }
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        CAP_HIP_TRY(hipStreamIsCapturing(st, &capturing));
+        if (capturing != hipStreamCaptureStatusNone) return CAP_OK;
+        CAP_TRY(time_candidate(p, algo, sync, b, x, k, st, t_steps, &t_steps));
+        algo = CAP_ALGO_WRTFST;
+        sync = CAP_SYNC_VALUE;
+    }
+    RhsScope own(p, 1);  // puts the plan's settings back
+    if (p->plain.bpc) own.take(p->plain);
     if (algo == CAP_ALGO_WRTFST) {
         cands.push_back({p->bpc, p->wblock, 0});
         for (int blk : {kBlock, kBlockSmall})
@@ -1297,7 +1345,7 @@ int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
         if (cands[c].tile >= 0) p->tile = cands[c].tile;
         p->part_kr = cands[c].kr;
         float t = 0;
-        rc = time_candidate(p, algo, sync, b, x, k, st, best, &t);
+        rc = time_candidate(p, algo, sync, b, x, k, st, std::min(best, t_steps), &t);
         if (rc == CAP_OK && t < (c ? 0.98f : 1.0f) * best) {
             best = t;
             pick = cands[c];
@@ -1326,9 +1374,21 @@ int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
         p->rpl = rpl0;
         p->lds = lds0;
         p->tile = tile0;
-        if (rc == CAP_OK && t < 0.98f * best) pick.staged = 0;
+        if (rc == CAP_OK && t < 0.98f * best) {
+            best = t;
+            pick.staged = 0;
+        }
     }
     if (rc != CAP_OK) return rc;
+    if (p->plain.bpc) {
+        if (pick.staged < 0) pick.staged = p->plain.staged;
+        if (pick.lds < 0) pick.lds = p->plain.lds;
+        if (pick.tile < 0) pick.tile = p->plain.tile;
+    }
+    if (steps && best >= 0.98f * t_steps)
+        pick = RhsPick{};
+    else
+        pick.rows = steps;
     p->rhs_pick[k] = pick;
     return CAP_OK;
 }
@@ -1342,6 +1402,8 @@ void apply_choice(cap_plan p, const TuneChoice &c)
     p->staged = c.staged;
     p->wblock = c.block;
     p->tile = c.tile;
+    p->plain = c.plain;
+    p->lvl_lead = c.lead;
 }
 
 // Tables of the partitioned banded solve (CAP_ALGO_PARTITION), built once:
@@ -2009,6 +2071,8 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
     float best = 1e30f;
     TuneChoice pick = cands[0];
     bool pick_set = false;
+    PlainShape plain;
+    float t_plain = 1e30f, t_steps = 0;
     int rc = CAP_OK;
     for (const TuneChoice &c : cands) {
         apply_choice(p, c);
@@ -2018,6 +2082,11 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
         float t = 0;
         if ((rc = time_candidate(p, c.algo, c.sync, b, x, 1, st, best, &t)) != CAP_OK) break;
         if (c.algo == CAP_ALGO_PARTITION) t *= part_factor;
+        if (c.algo == CAP_ALGO_LEVEL) t_steps = t;
+        if (c.algo == CAP_ALGO_WRTFST && c.sync == CAP_SYNC_VALUE && c.staged == stg && !c.hop && t < t_plain) {
+            t_plain = t;
+            plain = PlainShape{c.bpc, c.block, c.lds, c.tile, c.staged};
+        }
         // a later (less preferred) candidate must be 2% faster to win, so
         // near-ties resolve the same way from run to run
         if (t < (pick_set ? 0.98f : 1.0f) * best) {
@@ -2030,6 +2099,8 @@ int autotune(cap_plan p, const std::vector<int> &rp_host, const std::vector<int>
     (void)hipFree(x);
     p->hop = hop_tables;
     if (rc != CAP_OK) return rc;
+    if (pick.hop || pick.algo == CAP_ALGO_LEVEL) pick.plain = plain;
+    if (pick.algo == CAP_ALGO_LEVEL && t_steps > 0) pick.lead = t_plain / t_steps;
     apply_choice(p, pick);
     if (!pick.hop) free_hop(p);
     if (pick.algo == CAP_ALGO_MIX) CAP_TRY(build_mix(p, rp_host, pick.border));
@@ -2624,6 +2695,12 @@ int refine_fused(cap_plan p, const double *b, double *x, int rhs, hipStream_t st
     CAP_HIP_TRY(hipGetLastError());
     if (join) CAP_TRY(join_parts(join, st));
     if (p->n == 0) return CAP_OK;
+    RhsScope own(p, 1);
+    if (p->plain.bpc && !hop_takes(p, rhs)) {
+        const int staged = p->staged;  // where pr is
+        own.take(p->plain);
+        p->staged = staged;
+    }
     const int l = lpr_log2_for(rhs);
     // the sweep's own sizes: 128 or 256 threads, or 1024 for a batch that
     // picked it for several right-hand sides (no LDS window)

@@ -148,6 +148,81 @@ def test_autotuned_pick_is_timed_with_a_dense_right_hand_side(cuda):
     plan.close()
 
 
+def _grid(nx, ny, nz):
+    """The lower half of a 7-point stencil, natural order."""
+    i = np.arange(nx * ny * nz)
+    x, y, z = i % nx, i // nx % ny, i // (nx * ny)
+    rows = np.concatenate([i[z > 0], i[y > 0], i[x > 0]])
+    cols = np.concatenate([i[z > 0] - nx * ny, i[y > 0] - nx, i[x > 0] - 1])
+    order = np.lexsort((cols, rows))
+    rows, cols = rows[order], cols[order]
+    rp = np.r_[0, np.cumsum(np.bincount(rows, minlength=len(i)) + 1)].astype(np.int32)
+    ci = np.empty(rp[-1], np.int32)
+    ci[np.arange(len(rows)) + rows], ci[rp[1:] - 1] = cols, i
+    v = api.uniform(60, len(ci))
+    v[rp[1:] - 1] = 4.0
+    return rp, ci, v
+
+
+SEVERAL = {
+    "hop": lambda: _grid(30, 25, 20),                                                             # look-through, then rows
+    "near_tie": lambda: api.generate("level", n=30_000, levels=50, width=600, depth=2, offdiag=9, seed=61),
+    "steps": lambda: api.generate("band", n=5000, offdiag=8, band=400, seed=62),
+}
+
+
+@pytest.mark.parametrize("name", SEVERAL)
+@pytest.mark.parametrize("upper", [False, True])
+def test_several_right_hand_sides_of_hop_and_level_picks(cuda, name, upper):
+    """Where one right-hand side goes by look-through tables or steps, several
+    are timed as steps (near ties) and thread-per-row shapes: the oracle's
+    bits from each, and after them."""
+    from conftest import upper_from_lower
+    rp, ci, v = SEVERAL[name]()
+    if upper:
+        rp, ci, v = upper_from_lower(rp, ci, v)
+    n = len(rp) - 1
+    plan = _plan(cuda, rp, ci, v, upper=upper)
+    for k in (2, 3, 16, 64, 1, 16):
+        b = api.uniform(70 + k, n * k).reshape(n, k) if k > 1 else api.uniform(70, n)
+        x = _solve(plan, cuda, b).reshape(n, k)
+        for q in range(0, k, 7):
+            bq = np.ascontiguousarray(b.reshape(n, k)[:, q])
+            assert np.array_equal(x[:, q], oracle.csr_solve(rp, ci, v, bq, upper=upper, fused=True)), (k, q)
+    if not upper:
+        b = api.uniform(71, n * 4).reshape(n, 4)
+        import torch
+        xr, _, _ = plan.solve_refined(torch.from_numpy(b).to(cuda), tol=1e-12)
+        ref = oracle.csr_forward(rp, ci, v, b.reshape(-1), rhs=4, fused=True).reshape(n, 4)
+        assert np.max(np.abs(xr.cpu().numpy() - ref)) <= 1e-12 * np.max(np.abs(ref))
+    plan.close()
+
+
+def test_level_pick_captures_a_first_solve(cuda):
+    """The first solve with a number of right-hand sides may be a captured
+    one: nothing is timed then, the steps run."""
+    import torch
+    rp, ci, v = SEVERAL["near_tie"]()
+    n = len(rp) - 1
+    plan = _plan(cuda, rp, ci, v)
+    if plan.info()["algo"] != "level":
+        pytest.skip("the tuner's pick is not the steps here")
+    b = torch.from_numpy(api.uniform(72, n * 8).reshape(n, 8)).to(cuda)
+    out = torch.zeros_like(b)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        plan.solve(b, out=out, stream=torch.cuda.current_stream())
+    ref = oracle.csr_forward(rp, ci, v, b.cpu().numpy().reshape(-1), rhs=8, fused=True).reshape(n, 8)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), ref)
+        assert np.array_equal(plan.solve(b).cpu().numpy(), ref)  # timed now; the graph keeps what it holds
+    plan.close()
+
+
 @pytest.mark.parametrize("dtype,bits,span", [(np.float64, np.uint64, 620), (np.float32, np.uint32, 80)])
 def test_step_division_range(cuda, dtype, bits, span):
     """Diagonals and right-hand sides over powers of two beyond both ends of
