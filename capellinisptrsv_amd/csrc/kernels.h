@@ -1831,11 +1831,12 @@ __global__ void __launch_bounds__(kBlock)
     }
     if (t == 0) start[rows] = rp[lo + rows];
     __syncthreads();
-    for (int e = start[0] + t; e < start[rows]; e += kBlock) {
+    // unsigned: past the last entry of a matrix of nearly 2^31 the next e still is
+    for (unsigned e = (unsigned)start[0] + t, end = (unsigned)start[rows]; e < end; e += kBlock) {
         int r = 0;  // the last row that starts at or before e
 #pragma unroll
         for (int step = kBlock / 2; step > 0; step /= 2)
-            if (r + step < rows && start[r + step] <= e) r += step;
+            if (r + step < rows && (unsigned)start[r + step] <= e) r += step;
         grad_val[e] = -y[r] * x[ci[e]];
     }
 }
