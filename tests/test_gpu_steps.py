@@ -343,3 +343,61 @@ def test_loads_in_their_own_wavefronts(cuda, n, width, dtype, bits):
         ref = oracle.csr_forward(rp, ci, v, b, rhs=1, fused=True)
         assert np.array_equal(x.view(bits), ref.view(bits))
     plan.close()
+
+
+def _long_rows(n, longest, seed):
+    """Rows of 17 to `longest` entries in the 60 rows before them, and between
+    them rows of one, so that levels follow the row order."""
+    rng = np.random.default_rng(seed)
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        want = int(rng.integers(17, longest + 1)) if i % 3 == 0 else 1
+        cols = sorted(i - 1 - rng.choice(min(60, i), size=min(want, i), replace=False)) if i else []
+        ci += list(cols) + [i]
+        v += list(rng.uniform(-1, 1, len(cols))) + [1.0 + longest]
+        rp.append(len(ci))
+    return np.array(rp, np.int32), np.array(ci, np.int32), np.array(v)
+
+
+@pytest.mark.parametrize("dtype,bits", [(np.float64, np.uint64), (np.float32, np.uint32)])
+@pytest.mark.parametrize("arith", ["fused", "reference"])
+def test_rows_beyond_the_carried_entries(cuda, arith, dtype, bits):
+    """Rows of 17 to 39 entries: 16 in the step's pieces, the rest from the
+    overflow table, read behind them in the stored order."""
+    rp, ci, v = _long_rows(3000, 39, 80)
+    v = v.astype(dtype)
+    assert np.diff(rp).max() > 30
+    plan = _plan(cuda, rp, ci, v, algo="level", arith=arith)
+    b = api.uniform(81, 3000).astype(dtype)
+    ref = oracle.csr_forward(rp, ci, v, b, fused=arith == "fused")
+    for _ in range(2):
+        assert np.array_equal(_solve(plan, cuda, b).view(bits), ref.view(bits))
+    plan.close()
+
+
+@pytest.mark.parametrize("k", [6, 16])  # two and four right-hand sides per thread
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("arith", ["fused", "reference"])
+@pytest.mark.parametrize("off", [4, 8, 16, 30])
+def test_several_right_hand_sides_per_thread(cuda, off, arith, dtype, k):
+    """200 equal matrices: more workgroups of one right-hand side than the
+    compute units take at once, so a thread solves as many as divide k."""
+    import torch
+    from capellinisptrsv_amd import Batch
+    mats, n = 200, 1200
+    rp1, ci1, v1 = api.generate("level", n=n, levels=60, width=20, depth=2, offdiag=off, seed=83 + off)
+    assert off - 4 < np.diff(rp1).max() - 1 <= off
+    nnz = len(ci1)
+    rp = np.concatenate([rp1[:-1] + m * nnz for m in range(mats)] + [[mats * nnz]]).astype(np.int32)
+    ci = np.tile(ci1, mats)
+    v = (np.tile(v1, mats) * np.repeat(1.0 + 0.001 * np.arange(mats), nnz)).astype(dtype)
+    row_off = (np.arange(mats + 1) * n).astype(np.int32)
+    bt = Batch(*(torch.from_numpy(a).to(cuda) for a in (row_off, rp, ci, v)), k=k, arith=arith)
+    assert bt.step_matrices == mats
+    b = api.uniform(84 + k, mats * n * k).astype(dtype)
+    x = bt.solve(torch.from_numpy(b.reshape(mats * n, k)).to(cuda)).cpu().numpy().reshape(mats, -1)
+    for m in range(0, mats, 13):
+        ref = oracle.csr_forward(rp1, ci1, v[m * nnz:(m + 1) * nnz], b[m * n * k:(m + 1) * n * k], rhs=k,
+                                 fused=arith == "fused")
+        assert np.array_equal(x[m], ref), m
+    bt.close()
