@@ -797,17 +797,15 @@ void launch_part_fix(cap_plan p, const double *tg, int k, hipStream_t st)
         k_part_fixup<W, KQ, false><<<grid, W, 0, st>>>(ps->u, tg, wm, ps->gs, ps->t, k);
 }
 
-// Workgroups of the walks, about: one per CU.  A run of tails walks to its
-// first one and takes one product for each further one, so fewer and longer
-// runs read fewer matrices.  Whatever k: the runs set where walks start, and
-// so a right-hand side's bits.
-constexpr int kWalkGroups = 256;
-
+// One workgroup per CU, about.  A run of tails walks to its first one and
+// takes one product for each further one, so fewer and longer runs read fewer
+// matrices.  Whatever k: the runs set where walks start, and so a right-hand
+// side's bits.
 template <int W, int KQ>
 void launch_part_walk(cap_plan p, int k, hipStream_t st)
 {
     const PartState *ps = p->part;
-    const int run = (ps->Q + kWalkGroups - 1) / kWalkGroups;
+    const int run = (ps->Q + p->ncu - 1) / p->ncu;
     k_part_walk<W, KQ><<<dim3((unsigned)(((ps->Q + run - 1) / run + 7) / 8 * 8), (unsigned)(k / KQ)), kPartSplit * W, 0, st>>>(
         ps->a, ps->top, ps->bm, ps->fade, ps->t, ps->Q, run, k);
 }
@@ -1430,7 +1428,6 @@ constexpr int kPartBlocks = 1024;
 constexpr int kPartRows = 512;
 constexpr int kPartSpread = 500;
 constexpr int kPartLongest = 1280;
-constexpr int kPartCus = 256;
 // largest relative max-norm difference from the sequential solve accepted
 // when the tables are checked at plan creation (the FP64 bar is 1e-12)
 constexpr double kPartStableTol = 1e-13;
@@ -1497,9 +1494,9 @@ int build_partition(cap_plan p, const std::vector<int> &rp_host, hipStream_t st)
         const int least = std::max(W, (n + kPartBlocks - 1) / kPartBlocks);
         int m = std::max(least, std::min(std::max(kPartRows * (W / kPartW), n / kPartSpread), (n + 15) / 16));
         // whole rounds of the compute units, where a quarter more rows give them
-        const int rounds = n / m / kPartCus;
-        if (rounds > 0 && n / m % kPartCus > 0) {
-            const int even = (n + rounds * kPartCus - 1) / (rounds * kPartCus);
+        const int rounds = n / m / p->ncu;
+        if (rounds > 0 && n / m % p->ncu > 0) {
+            const int even = (n + rounds * p->ncu - 1) / (rounds * p->ncu);
             if (even <= m + m / 4) m = std::max(m, even);
         }
         int longer = 0;
