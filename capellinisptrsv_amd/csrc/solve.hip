@@ -1298,8 +1298,10 @@ int tune_rhs_block(cap_plan p, const void *b, void *x, int k, hipStream_t st)
             return CAP_OK;
         }
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        CAP_HIP_TRY(hipStreamIsCapturing(st, &capturing));
-        if (capturing != hipStreamCaptureStatusNone) return CAP_OK;
+        if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return CAP_OK;
+        }
         CAP_TRY(time_candidate(p, algo, sync, b, x, k, st, t_steps, &t_steps));
         algo = CAP_ALGO_WRTFST;
         sync = CAP_SYNC_VALUE;
