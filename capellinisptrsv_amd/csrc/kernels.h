@@ -2712,9 +2712,9 @@ __global__ void __launch_bounds__(kPartSplit * W, W >= 256 && KQ >= 2 ? 7 : 1)
     // 16 columns at a time, one to a lane: a lane's value goes to its row of
     // 16 by DPP, one LDS read per lane for 16 columns.  At W = 128 the part of
     // the next product's matrix is loaded while the current one is joined.
-    // The matrices' bytes bound it: at n = 500,000 (m = 1000, 3 products to a
-    // tail, 64 MB) 19 us; at n = 200,000 with 8 right-hand sides (m = 512, 5
-    // products) 31 us, 50 with two chunks of 4.  The scan's launches took 83
+    // The matrices' bytes bound it: at n = 500,000 (m = 1000, 97 MB) 20 us; at
+    // n = 200,000 with 8 right-hand sides (m = 512) 35 us (31 as one chunk and
+    // 50 as two of 4 while walks started later).  The scan's launches took 83
     // and 140 (1023 tails).
     constexpr bool kAhead = W == kPartW;
     constexpr int kCols = 16;

@@ -1769,11 +1769,11 @@ int build_partition_tables(cap_plan p, const PartRows &mat, int w, int m, bool m
     for (void *t : {(void *)d_rows, (void *)d_rp, (void *)d_ci, (void *)d_v, (void *)d_ops})
         if (t) (void)hipFree(t);
     if (bm && bm != ps->bm) (void)hipFree(bm);
-    // Accuracy check against the sequential solve.  The block solves and V
-    // multiply by block inverses, which the sequential solve never forms;
-    // when the blocks are not diagonally dominant their entries grow along a
-    // block (unit values in a band, as the reference's .mtx reader makes
-    // them, grow as 1.47^m) and the finish cancels.  The tables solve two
+    // Accuracy check against the sequential solve.  The records and the B_p
+    // multiply by inverses of diagonal blocks, which the sequential solve never
+    // forms; when the blocks are not diagonally dominant their entries grow
+    // along a block (unit values in a band, as the reference's .mtx reader
+    // makes them, grow as 1.47^m) and the sums cancel.  The tables solve two
     // right-hand sides -- b = L 1 (row sums in FP64) and a seeded U[-1,1] b
     // -- and each must agree with a sequential FP64 forward substitution of
     // the same system on the host to kPartStableTol relative max-norm, ten

@@ -220,10 +220,14 @@ __device__ __forceinline__ void step_load(StepStage<T, E, K> &w, Rsrc tab, unsig
 // The row data is loaded D steps ahead into registers, the row number 2D
 // steps ahead (b is gathered through it); the barriers order LDS alone, so
 // they do not wait for those loads.  The next step's ring addresses are
-// unpacked before the barrier that ends this one.  What bounds it: one wavefront's chain of dependent instructions per
-// step (LDS reads, E fused multiply-adds, the division, the ring write, the
-// barrier), with nothing else on its SIMD to hide their latency; with E = 16
-// also the compute unit's 64 bytes of loads per cycle.
+// unpacked before the barrier that ends this one.  What bounds it: one
+// wavefront's chain of dependent instructions per step (LDS reads, E fused
+// multiply-adds, the division, the ring write, the barrier) and the issue of
+// its own loads, with nothing else on its SIMD to hide their latency: 60,000
+// rows of up to 15 entries, 523 steps of 128 rows: 0.37 us a step, 59 vector,
+// 17 LDS and 14 load instructions per wavefront, a tenth of the cycles lost to
+// LDS bank conflicts, and 24.6 KB of table a step, 28 bytes a cycle, well
+// below what a compute unit loads.
 template <typename T, int E, int D, bool UNFUSED, bool LONG, int K>
 __global__ void __launch_bounds__(kStepBlock)
     k_step(const StepJob *__restrict__ jobs, int n_jobs, const uint4 *__restrict__ tab,
@@ -340,7 +344,8 @@ __global__ void __launch_bounds__(kStepBlock)
 // carries the row's offset in b and x.  Both sides meet at the one barrier
 // per step.
 // What bounds it: with one solving wavefront its chain (107 ns a step, 159
-// with k_step: 24.6 against 34.1 us for n = 2,000 in 193 steps), with more
+// with k_step: 24.6 against 34.1 us for n = 2,000 in 193 steps, both without
+// the values' copy before it), with more
 // the LDS traffic of the steps' data too: 194 / 279 / 333 ns with two, three
 // and four (k_step 221 / 303 / 355; n = 100,000 in 807 steps 156 against 178
 // us).  With 8 or 16 entries a row the data through LDS costs more than its

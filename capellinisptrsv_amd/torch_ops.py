@@ -41,7 +41,7 @@ class Plan:
     place).  Values changed in place reach the next solve, except where the
     plan holds tables of them: partition (also as auto's pick, see info()),
     algo="level", upper and unit_diagonal plans keep the values of creation,
-    the gather adjoint and solve_refined those of their first call.  algo: auto|wrtfst|twopart|mix|csc|local|partition|level|hop; sync:
+    the gather adjoint those of its first call.  algo: auto|wrtfst|twopart|mix|csc|local|partition|level|hop; sync:
     auto|value|flag.
     row_threads: 128 or 256 threads per workgroup of the thread-per-row
     kernels (0: tuned with algo auto, else 256).
@@ -291,7 +291,11 @@ def sptrsv(values: torch.Tensor, b: torch.Tensor, plan: Plan) -> torch.Tensor:
 
 
 class TriangularSolve(torch.nn.Module):
-    """Module holding the sparsity pattern and a learnable value vector."""
+    """Module holding the sparsity pattern and a learnable value vector.
+
+    The forward solve follows in-place changes of the values where its plan
+    does (see Plan: not with partition, also as auto's pick, nor level); the
+    gradients come from the values of the first backward pass."""
 
     def __init__(self, row_ptr, col_idx, values, algo="auto"):
         super().__init__()

@@ -212,7 +212,8 @@ void cap_opts_default(cap_opts *o);
  * except where a plan holds tables of them: CAP_ALGO_PARTITION (explicit or
  * AUTO's pick, cap_plan_info) and explicit CAP_ALGO_LEVEL plans, upper or
  * unit-diagonal ones, and host inputs solve with the values of plan creation;
- * the gather adjoint and refined solves keep those of their first call.
+ * the gather adjoint keeps those of its first call, and refined solves that
+ * need a third step an FP32 copy of those of the first such call.
  * cap_plan_solve is asynchronous on `stream`; b and x are device pointers of
  * n*rhs values interleaved as x[i*rhs + k] (serialref.h:57-60 layout). */
 typedef struct cap_plan_s *cap_plan;
@@ -256,10 +257,12 @@ int cap_plan_rhs_block(cap_plan plan, int k, int *blocks_per_cu,
                        int *row_threads, int *rhs_per_wave, int *rhs_per_lane,
                        int *readiness, int *row_tiles);
 /* Which algorithm / sync protocol the plan resolved to, and its mix table.
- * (An autotuned plan that resolved to mix, two-part, CSC or the level
- * steps, which solve one right-hand side, solves several with the
- * write-first kernel in the value protocol; a plan created with one of
- * those algorithms refuses k > 1 with CAP_ERR_UNSUPPORTED.) */
+ * (An autotuned plan that resolved to mix, two-part or CSC, which solve one
+ * right-hand side, solves several with the write-first kernel in the value
+ * protocol; a plan created with one of those algorithms refuses k > 1 with
+ * CAP_ERR_UNSUPPORTED.  One that resolved to the level steps solves several by
+ * steps, or by the write-first kernel where that is close and timed faster;
+ * an explicit CAP_ALGO_LEVEL plan takes 1, or 2 and 4 where its rule allows.) */
 int cap_plan_info(cap_plan plan, int *algo, int *sync, int *border,
                   int *mix_len, double *warp_occupy, double *element_occupy);
 /* No counterpart in the reference: publish -> observe waits on the longest
