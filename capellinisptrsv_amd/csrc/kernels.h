@@ -2166,9 +2166,9 @@ __global__ void __launch_bounds__(kWave)
 }
 
 // What a sweep is for: the tails a_p of history 0 (and of each the bits of the
-// largest magnitude, a NaN's above all, and of the smallest that is not 0, 0
-// for none: top[2i], top[2i + 1]), the B_p (right-hand side q's history
-// is e_q and b is 0), or x from the tails t.
+// largest magnitude, a NaN's above all, and of the smallest: top[2i],
+// top[2i + 1]), the B_p (right-hand side q's history is e_q and b is 0), or x
+// from the tails t.
 enum PartSweep { kPartTails, kPartUnit, kPartX };
 
 // One wavefront per block and KR right-hand sides (b and x interleaved, k per
@@ -2319,7 +2319,7 @@ __global__ void __launch_bounds__(kPartWaves * kWave)
     }
     if (MODE != kPartX) {  // the block's last W values: blocks of m >= W rows
         const long long out = MODE == kPartUnit ? p - 1 : p;
-        unsigned long long big[KR], low[KR];  // low: less 1, so that 0 is above all
+        unsigned long long big[KR], low[KR];
 #pragma unroll
         for (int q = 0; q < KR; ++q) {
             big[q] = 0;
@@ -2333,7 +2333,7 @@ __global__ void __launch_bounds__(kPartWaves * kWave)
                 tails[(out * k + q0 + q) * W + c] = v;
                 const unsigned long long u = as_bits(v) & ~(1ull << 63);
                 big[q] = max(big[q], u);
-                low[q] = min(low[q], u - 1);
+                low[q] = min(low[q], u);
             }
         }
         if (MODE == kPartTails) {
@@ -2346,7 +2346,7 @@ __global__ void __launch_bounds__(kPartWaves * kWave)
                 }
                 if (lane == 0) {
                     top[2 * (out * k + q0 + q)] = big[q];
-                    top[2 * (out * k + q0 + q) + 1] = low[q] + 1;
+                    top[2 * (out * k + q0 + q) + 1] = low[q];
                 }
             }
         }
@@ -2620,15 +2620,17 @@ __global__ void __launch_bounds__(W) k_part_norm(const double *__restrict__ bm, 
 // their history (four in a row by kPartDamp or more) or are few.  What block p
 // - s adds to t_p is at most norm(B_p ... B_{p-s+1}) max|a_{p-s}|; the walk to
 // t_p starts at the farthest block for which a bound of that is above
-// 2^-(57 + s/2) of the smallest magnitude in a_p that is not 0, and not below
-// the smallest double.  All that is left out then stays below 2^-55.7 of each
-// of them, a sixth of the rounding of t_p's own terms, also where the tail's
-// rows belong to systems that do not touch each other: measured against the
-// largest magnitude, one huge row of b took the digits of all the others in
-// its block's tail (4e-10 of the largest, now 4e-16).  The smallest is about
-// 9 bits below it with a dense right-hand side: 18.8 -> 19.6 us at n =
-// 500,000.  How far that is depends on the right-hand side alone, so it gets
-// the same bits in every chunk.  Blocks are looked at kPartReach back: there
+// 2^-(57 + s/2) of the smallest magnitude in a_p and not below the smallest
+// double (all the way to that where a_p holds a 0: such a row's value is its
+// history alone).  All that is left out then stays below 2^-55.7 of each of
+// a_p's values, a sixth of the rounding of t_p's own terms, also where the
+// tail's rows belong to systems that do not touch each other: measured against
+// the largest magnitude, one huge row of b took the digits of all the others
+// in its block's tail (4e-10 of the largest, now 4e-16), and without the
+// zeros a system whose right-hand side ended was 0 two blocks later.  The
+// smallest is about 9 bits below the largest with a dense right-hand side:
+// 18.8 -> 19.6 us at n = 500,000.  How far that is depends on the right-hand
+// side alone, so it gets the same bits in every chunk.  Blocks are looked at kPartReach back: there
 // the factor has passed 2^-2048, the whole range of a double.  After a block
 // with an infinity or a NaN in its tail every tail is NaN (0 times an
 // infinity is NaN, and each product has all W columns).
